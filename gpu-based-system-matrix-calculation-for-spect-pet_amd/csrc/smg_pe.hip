@@ -6,13 +6,12 @@
 // before its sub-cell loop (:1193-1362).  Here the 64 lanes of a wave share
 // detector d, so every sub-cell point is wave-uniform and:
 //   1. the wave scans the bars and holes once, 64 at a time, keeping those
-//      whose box a segment from bar d to the tile's bounding ball can meet
-//      (any other has chord 0 for every ray of the wave, so whether the
+//      whose box a segment from bar d to the tile can meet (any other has chord 0 for every ray of the wave, so whether the
 //      reference would cull it does not change the result); each survivor is
 //      then tested with the reference culling predicate per lane and stored
 //      in LDS with the 64-bit ballot of the lanes that keep it;
 //   2. for each sub-cell, the candidates are narrowed to those whose box can
-//      meet a segment from the sub-cell centre to the tile's bounding ball (a
+//      meet a segment from the sub-cell centre to the tile (a
 //      bar outside that cone has chord 0 for every lane, so dropping it is
 //      exact);
 //   3. every lane traces its own ray against the narrowed lists (wave-uniform
@@ -149,7 +148,7 @@ struct WaveSetup {
     SelfCull sc;
     float udf[3], critf;
     double tc[3], rho;
-    float tcf[3], rhof;
+    float tcf[3], te[3];  // tile centre and half extents along the world axes
     uint32_t bar_gate;  // bit m: no ray from bar d to the tile can be stopped by layer m's gate
 };
 
@@ -176,9 +175,11 @@ __device__ __forceinline__ void wave_setup(const PeLaunch& A, int d, int tile, i
     tile_ball(g, ix0, iy0, iz0, A.tile, A.cphi, A.sphi, W.tc, W.rho);
     for (int k = 0; k < 3; ++k) W.tc[k] = uniform_d(W.tc[k]);
     W.rho = uniform_d(W.rho);
-    tile_ball_f(W.tc, W.rho, W.tcf, W.rhof);
-    for (int k = 0; k < 3; ++k) W.tcf[k] = uniform_f(W.tcf[k]);
-    W.rhof = uniform_f(W.rhof);
+    tile_extents(g, ix0, iy0, iz0, A.tile, A.cphi, A.sphi, W.te);
+    for (int k = 0; k < 3; ++k) {
+        W.tcf[k] = uniform_f(float(W.tc[k]));
+        W.te[k] = uniform_f(W.te[k]);
+    }
     // plate gates that no ray from any point of bar d (inside its bounding
     // ball, the half diagonal with a rounding margin) to the tile can trigger
     const double qc[3] = {bd.cx, bd.cy, bd.cz};
@@ -189,7 +190,11 @@ __device__ __forceinline__ void wave_setup(const PeLaunch& A, int d, int tile, i
 }
 
 // Step 1: candidate bars and holes of the tile: those whose box a segment from
-// bar d to the tile can meet (bar_tile_may_hit, first on the box of each
+// bar d to the tile can meet (bar_tile_may_hit with the tile's half extents per
+// axis, which are what bounds the scan: a ball around a 4x4x4 tile is 1.7 times
+// as wide, and around an 8x8x1 tile 1.4 times along x and y and 2.5 mm instead
+// of 0 along z; with the ball the full-size PE step took 187.5 ms instead of
+// 177.4, one slice at 8x16x8 sub-cells 37.4 instead of 33.5; first on the box of each
 // group of kGroup consecutive bars or holes, then on the members of the
 // groups it keeps; any other has chord 0 for every ray of the tile, so its
 // culling decision does not matter), each with the ballot of the lanes whose
@@ -210,7 +215,7 @@ __device__ bool build_candidates(const PeLaunch& A, int d, int lane, const WaveS
         bool gpass = false;
         if (g0 + lane < n_bg) {
             const GroupBox& B = G.bar_groups[g0 + lane];
-            gpass = bar_tile_may_hit(bdf, W.tcf, W.rhof, B.c[0], B.c[1], B.c[2], 1.0f, 0.0f, B.h[0],
+            gpass = bar_tile_may_hit(bdf, W.tcf, W.te, B.c[0], B.c[1], B.c[2], 1.0f, 0.0f, B.h[0],
                                      B.h[1], B.h[2]);
         }
         uint64_t gbal = __ballot(gpass);
@@ -221,7 +226,9 @@ __device__ bool build_candidates(const PeLaunch& A, int d, int lane, const WaveS
             bool pass = false, far = false;
             if (k < g.n_det && k != d) {
                 const Bar<float>& b = G.bars_f[k];
-                pass = bar_tile_may_hit(bdf, W.tcf, W.rhof, b.cx, b.cy, b.cz, b.cb, b.sb, 0.5f * b.w,
+                float rt[3];
+                extents_in_frame(W.te, b.cb, b.sb, rt);
+                pass = bar_tile_may_hit(bdf, W.tcf, rt, b.cx, b.cy, b.cz, b.cb, b.sb, 0.5f * b.w,
                                         0.5f * b.t, 0.5f * b.h);
                 if (pass) far = fast_tile_far(G, k, W.tc, W.rho);
             }
@@ -249,7 +256,7 @@ __device__ bool build_candidates(const PeLaunch& A, int d, int lane, const WaveS
         bool gpass = false;
         if (g0 + lane < n_hg) {
             const GroupBox& B = G.hole_groups[g0 + lane];
-            gpass = bar_tile_may_hit(bdf, W.tcf, W.rhof, B.c[0], B.c[1], B.c[2], 1.0f, 0.0f, B.h[0],
+            gpass = bar_tile_may_hit(bdf, W.tcf, W.te, B.c[0], B.c[1], B.c[2], 1.0f, 0.0f, B.h[0],
                                      B.h[1], B.h[2]);
         }
         uint64_t gbal = __ballot(gpass);
@@ -260,7 +267,7 @@ __device__ bool build_candidates(const PeLaunch& A, int d, int lane, const WaveS
             bool pass = false;
             if (h < g.n_holes) {
                 const Hole<float>& o = G.holes_f[h];
-                pass = bar_tile_may_hit(bdf, W.tcf, W.rhof, o.xc, o.ymid, o.zc, 1.0f, 0.0f, o.r,
+                pass = bar_tile_may_hit(bdf, W.tcf, W.te, o.xc, o.ymid, o.zc, 1.0f, 0.0f, o.r,
                                         0.5f * tabs(o.y2 - o.y1), o.r);
             }
             uint64_t bal = __ballot(pass);
@@ -341,7 +348,9 @@ __device__ void narrow_candidates(const PeLaunch& A, const double qd[3], const W
                 cb = 1.0f; sb = 0.0f;
                 h[0] = o.r; h[1] = 0.5f * tabs(o.y2 - o.y1); h[2] = o.r;
             }
-            pass = box_meets_frustum(q, rq, W.tcf, W.rhof, c[0], c[1], c[2], cb, sb, h[0], h[1], h[2]);
+            float rt[3];
+            extents_in_frame(W.te, cb, sb, rt);
+            pass = box_meets_frustum(q, rq, W.tcf, rt, c[0], c[1], c[2], cb, sb, h[0], h[1], h[2]);
         }
         const uint64_t bb = __ballot(pass && is_bar), bh = __ballot(pass && !is_bar);
         if (pass) {

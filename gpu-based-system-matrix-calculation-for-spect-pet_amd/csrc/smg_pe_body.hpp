@@ -180,20 +180,44 @@ SMG_FN void tile_ball_f(const double tc[3], double rho, float tcf[3], float& rho
     for (int k = 0; k < 3; ++k) tcf[k] = float(tc[k]);
     rhof = float(rho) * 1.0001f;
 }
-//
-// Can a segment from a point of the box (q, rq) to a point of the ball
-// (tc, rho) meet the box of half sizes (hx, hy, hz) centred at c and turned by
-// beta about y (cos and sin in cb, sb)?  rq holds the half sizes of an
-// axis-aligned box around q in the frame of the tested box.  Such a segment is
-//   (q + e1) + s (tc + e2 - q - e1),  s in [0, 1],  |e1_i| <= rq_i,  |e2| <= rho,
-// so per axis it lies within r_i(s) = (1 - s) rq_i + s rho of the axis point
+
+// Half extents along the world axes of the box around the same voxel centres
+// (about the ball's centre), rounded up: the rotation about z turns the
+// tile's own x and y extents.
+SMG_FN void tile_extents(const GeomDesc& g, int ix0, int iy0, int iz0, const int tile[3], double cphi,
+                         double sphi, float te[3]) {
+    const int ex = tmin2(tile[0], g.nx - ix0), ey = tmin2(tile[1], g.ny - iy0),
+              ez = tmin2(tile[2], g.nz - iz0);
+    const double hx = 0.5 * (ex - 1) * tabs(g.wx), hy = 0.5 * (ey - 1) * tabs(g.wy),
+                 hz = 0.5 * (ez - 1) * tabs(g.wz);
+    te[0] = float(tabs(cphi) * hx + tabs(sphi) * hy + 1e-6) * 1.0001f;
+    te[1] = float(tabs(sphi) * hx + tabs(cphi) * hy + 1e-6) * 1.0001f;
+    te[2] = float(hz + 1e-6) * 1.0001f;
+}
+
+// Half extents, in the frame of a box turned by beta about y (cos and sin in
+// cb, sb), of an axis-aligned world box of half extents te.
+SMG_FN void extents_in_frame(const float te[3], float cb, float sb, float rt[3]) {
+    const float ac = tabs(cb), as = tabs(sb);
+    rt[0] = ac * te[0] + as * te[2];
+    rt[1] = te[1];
+    rt[2] = as * te[0] + ac * te[2];
+}
+
+// Can a segment from a point of the box (q, rq) to a point of the box (tc,
+// rt) meet the box of half sizes (hx, hy, hz) centred at c and turned by beta
+// about y (cos and sin in cb, sb)?  rq and rt hold the half sizes of
+// axis-aligned boxes around q and tc in the frame of the tested box.  Such a
+// segment is
+//   (q + e1) + s (tc + e2 - q - e1),  s in [0, 1],  |e1_i| <= rq_i,  |e2_i| <= rt_i,
+// so per axis it lies within r_i(s) = (1 - s) rq_i + s rt_i of the axis point
 // q + s (tc - q): the box grown by r_i(s) must meet the axis segment.  Per axis
 // that is two linear inequalities in s; the test intersects their intervals
 // with [0, 1].  The margin m covers the FP32 rounding of the inputs and the
 // direction components below 0.001 that the chord functions treat as zero (a
 // segment then drifts less than 0.001 off the box along that axis).  A false
 // answer means every chord of every such segment through the box is zero.
-SMG_FN bool box_meets_frustum(const float q[3], const float rq[3], const float tc[3], float rho,
+SMG_FN bool box_meets_frustum(const float q[3], const float rq[3], const float tc[3], const float rt[3],
                               float cx, float cy, float cz, float cb, float sb, float hx, float hy,
                               float hz) {
     float qx = q[0] - cx, qy = q[1] - cy, qz = q[2] - cz;
@@ -207,8 +231,8 @@ SMG_FN bool box_meets_frustum(const float q[3], const float rq[3], const float t
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         float u = b[i] - a[i];
-        float dr = rho - rq[i];
-        float m = 2e-3f + 1e-5f * (tabs(a[i]) + tabs(b[i]) + h[i] + rho + rq[i]);
+        float dr = rt[i] - rq[i];
+        float m = 2e-3f + 1e-5f * (tabs(a[i]) + tabs(b[i]) + h[i] + rt[i] + rq[i]);
         float c0 = u - dr, r0 = h[i] + m + rq[i] - a[i];   // a + s u <= h + r(s)
         float c1 = -u - dr, r1 = h[i] + m + rq[i] + a[i];  // -(a + s u) <= h + r(s)
         if (c0 > 0.0f) hi = tmin2(hi, tdiv(r0, c0));
@@ -221,17 +245,30 @@ SMG_FN bool box_meets_frustum(const float q[3], const float rq[3], const float t
     return ok && lo <= hi + 1e-5f;
 }
 
+// The same for a ball of radius rho around tc (its extent is rho in every frame).
+SMG_FN bool box_meets_frustum(const float q[3], const float rq[3], const float tc[3], float rho,
+                              float cx, float cy, float cz, float cb, float sb, float hx, float hy,
+                              float hz) {
+    const float rt[3] = {rho, rho, rho};
+    return box_meets_frustum(q, rq, tc, rt, cx, cy, cz, cb, sb, hx, hy, hz);
+}
 
-// Segments from any point of bar d to the tile ball, against a box turned by
-// beta_k (cos, sin in cbk, sbk): bar d's half sizes become the axis-aligned
-// extents of bar d seen in the frame of that box.
-SMG_FN bool bar_tile_may_hit(const Bar<float>& bd, const float tc[3], float rho, float cx,
+// Segments from any point of bar d to the tile (rt: its half extents in the
+// frame of the tested box), against a box turned by beta_k (cos, sin in cbk,
+// sbk): bar d's half sizes become the axis-aligned extents of bar d seen in
+// the frame of that box.
+SMG_FN bool bar_tile_may_hit(const Bar<float>& bd, const float tc[3], const float rt[3], float cx,
                              float cy, float cz, float cbk, float sbk, float hx, float hy, float hz) {
     const float cd = tabs(bd.cb * cbk + bd.sb * sbk), sd = tabs(bd.sb * cbk - bd.cb * sbk);
     const float hdx = 0.5f * bd.w * 1.0001f, hdy = 0.5f * bd.t * 1.0001f, hdz = 0.5f * bd.h * 1.0001f;
     const float rq[3] = {cd * hdx + sd * hdz, hdy, sd * hdx + cd * hdz};
     const float q[3] = {bd.cx, bd.cy, bd.cz};
-    return box_meets_frustum(q, rq, tc, rho, cx, cy, cz, cbk, sbk, hx, hy, hz);
+    return box_meets_frustum(q, rq, tc, rt, cx, cy, cz, cbk, sbk, hx, hy, hz);
+}
+SMG_FN bool bar_tile_may_hit(const Bar<float>& bd, const float tc[3], float rho, float cx, float cy,
+                             float cz, float cbk, float sbk, float hx, float hy, float hz) {
+    const float rt[3] = {rho, rho, rho};
+    return bar_tile_may_hit(bd, tc, rt, cx, cy, cz, cbk, sbk, hx, hy, hz);
 }
 
 // a[i] = v for a run-time i < N through unrolled selects: indexing a local
