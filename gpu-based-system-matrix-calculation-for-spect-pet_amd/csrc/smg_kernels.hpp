@@ -36,11 +36,22 @@ struct PeSpill {
     int cap_bars = 0, cap_holes = 0;
 };
 
-// Bytes of one spill slot: masks, adjoint sums and indices of every bar and
-// hole, and the face records of the first narrowed bars, in 256-byte units.
+// One spill slot: the arena (the masks of every bar and hole, then 16 KB and 2
+// bytes per bar and hole for the narrowed pairs), the selection words of at
+// least one sub-cell over every bar and hole, the redo masks of 64 sub-cells, the
+// adjoint sums and the indices; in 8-byte words, and in bytes (256-byte units).
+SMG_HD inline int pe_spill_arena_words(int n_det, int n_holes) {
+    const int n = n_det + n_holes;
+    return n + 2048 + (n + 3) / 4;
+}
+SMG_HD inline int pe_spill_sel_words(int n_det, int n_holes) {
+    const int w = (n_det + n_holes + 63) / 64;
+    return w > 64 ? w : 64;
+}
 inline int64_t pe_spill_slot_bytes(int n_det, int n_holes) {
-    const int64_t b = n_det > 0 ? n_det : 1, h = n_holes > 0 ? n_holes : 1;
-    const int64_t bytes = b * (8 + 8 + 2 + 2) + h * (8 + 2 + 2) + 32 * (7 * 4 + 1) + (b + 63) / 64 * 8;
+    const int64_t n = (int64_t)n_det + n_holes;
+    const int64_t bytes = 8 * ((int64_t)pe_spill_arena_words(n_det, n_holes) + pe_spill_sel_words(n_det, n_holes) +
+                               64 + n_det) + 2 * n;
     return (bytes + 255) / 256 * 256;
 }
 

@@ -29,27 +29,26 @@ namespace smg {
 
 namespace {
 
-// Capacity of the per-wave queue of sub-cells to redo in FP64.
-constexpr int kRedoCap = 64;
-
-// Narrowed bars of a sub-cell whose faces relative to the sub-cell point are
-// kept for fast_bar_chord (the first kFastBars).
-constexpr int kFastBars = 32;
+// Sub-cells of one block of the narrowing, at most (one lane holds each).
+constexpr int kBlockCells = 64;
+// Room for (sub-cell, candidate) records beside full candidate lists, in
+// 8-byte words.
+constexpr int kRecWords = 244;
 
 // Candidate lists of one wave, in LDS, for up to CapB bars and CapH holes.
+// arena: the lane masks of the n = nb + nh candidates of the tile (bars first,
+// then holes), then the records of the narrowed pairs: bars upward from word n,
+// holes downward from the end.  The lists are short as a rule (about 27
+// candidates on the full-size geometry), so the records of a whole block fit.
 template <int CapB, int CapH>
 struct WaveListsT {
     static constexpr int cap_bars = CapB, cap_holes = CapH;
-    uint64_t bar_mask[CapB];
-    uint64_t hole_mask[CapH];
-    uint64_t tile_far[(CapB + 63) / 64];  // bit i: candidate bar i passes fast_tile_far
-    uint16_t bar_idx[CapB];
-    uint16_t hole_idx[CapH];
-    uint16_t bar_sel[CapB];
-    uint16_t hole_sel[CapH];
-    float faces[kFastBars][7];   // narrowed bar j: faces - sub-cell point (fast_faces),
-                                 // then the bar's mu_total (a float value: exact)
-    uint8_t fast_ok[kFastBars];  // narrowed bar j qualifies for fast_bar_chord
+    static constexpr int arena_words = CapB + CapH + kRecWords;
+    static constexpr int sel_cap = 64;
+    uint64_t arena[CapB + CapH + kRecWords];
+    uint64_t sel[sel_cap];       // per sub-cell of the block: the candidates it keeps
+    uint64_t redo[kBlockCells];  // per sub-cell of the block: the lanes to redo in FP64
+    uint16_t idx[CapB + CapH];   // bar or hole number of each candidate
 };
 using WaveLists = WaveListsT<kCapBars, kCapHoles>;
 
@@ -62,43 +61,31 @@ using AdjointLists = WaveListsT<kCapBarsAdjoint, kCapHoles>;
 // slot of global memory with room for every bar and hole of the geometry (so
 // they cannot overflow), plus the adjoint's per-candidate sums.
 struct SpillLists {
-    int cap_bars, cap_holes;
-    uint64_t* bar_mask;
-    uint64_t* hole_mask;
-    uint64_t* tile_far;
+    int cap_bars, cap_holes, arena_words, sel_cap;
+    uint64_t* arena;
+    uint64_t* sel;
+    uint64_t* redo;
     double* cand_acc;
-    float (*faces)[7];
-    uint16_t* bar_idx;
-    uint16_t* hole_idx;
-    uint16_t* bar_sel;
-    uint16_t* hole_sel;
-    uint8_t* fast_ok;
+    uint16_t* idx;
 };
 
 __device__ __forceinline__ SpillLists spill_lists(const PeSpill& S, int slot) {
     unsigned char* p = S.slots + (int64_t)slot * S.slot_bytes;
+    const int n = S.cap_bars + S.cap_holes;
     SpillLists L;
     L.cap_bars = S.cap_bars;
     L.cap_holes = S.cap_holes;
-    L.bar_mask = (uint64_t*)p;
-    p += sizeof(uint64_t) * S.cap_bars;
-    L.hole_mask = (uint64_t*)p;
-    p += sizeof(uint64_t) * S.cap_holes;
-    L.tile_far = (uint64_t*)p;
-    p += sizeof(uint64_t) * ((S.cap_bars + 63) / 64);
+    L.arena_words = pe_spill_arena_words(S.cap_bars, S.cap_holes);
+    L.sel_cap = pe_spill_sel_words(S.cap_bars, S.cap_holes);
+    L.arena = (uint64_t*)p;
+    p += sizeof(uint64_t) * L.arena_words;
+    L.sel = (uint64_t*)p;
+    p += sizeof(uint64_t) * L.sel_cap;
+    L.redo = (uint64_t*)p;
+    p += sizeof(uint64_t) * kBlockCells;
     L.cand_acc = (double*)p;
     p += sizeof(double) * S.cap_bars;
-    L.faces = (float(*)[7])p;
-    p += sizeof(float) * 7 * kFastBars;
-    L.bar_idx = (uint16_t*)p;
-    p += sizeof(uint16_t) * S.cap_bars;
-    L.hole_idx = (uint16_t*)p;
-    p += sizeof(uint16_t) * S.cap_holes;
-    L.bar_sel = (uint16_t*)p;
-    p += sizeof(uint16_t) * S.cap_bars;
-    L.hole_sel = (uint16_t*)p;
-    p += sizeof(uint16_t) * S.cap_holes;
-    L.fast_ok = (uint8_t*)p;
+    L.idx = (uint16_t*)p;
     return L;
 }
 
@@ -112,30 +99,56 @@ __device__ __forceinline__ void spill_push(const PeLaunch& A, int item, int lane
     }
 }
 
-// View of the narrowed lists for one lane.
+// A 64-bit value every lane holds alike, in scalar registers; and its bit of
+// this lane, which is the wave's execution mask itself.
+__device__ __forceinline__ uint64_t uniform_u64(uint64_t x) {
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)x);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(x >> 32));
+    return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ bool lane_bit(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+// One sub-cell's narrowed candidates for the lanes of a wave, from its records
+// (the FP32 rays).
 template <class Lists>
-struct ListCands {
+struct RecCands {
     static constexpr bool kFastFaces = true;
+    static constexpr bool kHoleRecs = true;
     const Lists* L;
-    int nb, nh, lane;
-    __device__ bool fast(int j) const { return j < kFastBars && L->fast_ok[j]; }
-    __device__ const float* faces(int j) const { return L->faces[j]; }
-    // mu_total of narrowed bar j, kept beside its faces for the first kFastBars
-    __device__ bool has_mu(int j) const { return j < kFastBars; }
-    __device__ float mu(int j) const { return L->faces[j][6]; }
+    const BarRec* b;   // record j: b[j]
+    const HoleRec* h;  // record j: h[-j]
+    int nb, nh;
     __device__ int nbars() const { return nb; }
+    __device__ bool fast(int j) const { return b[j].tag & kFastBar; }
+    __device__ const float* faces(int j) const { return b[j].face; }
+    __device__ bool has_mu(int) const { return true; }
+    __device__ float mu(int j) const { return b[j].mu; }
+    __device__ int pos(int j) const { return b[j].tag & 0xffff; }
     // the index is wave-uniform: readfirstlane lets the record loads go
     // through the scalar unit
-    __device__ int bar(int j) const { return __builtin_amdgcn_readfirstlane(L->bar_idx[L->bar_sel[j]]); }
-    __device__ bool bar_on(int j) const { return (L->bar_mask[L->bar_sel[j]] >> lane) & 1ull; }
+    __device__ int bar(int j) const { return __builtin_amdgcn_readfirstlane(L->idx[pos(j)]); }
+    __device__ bool bar_on(int j) const { return lane_bit(uniform_u64(b[j].lanes)); }
     __device__ int nholes() const { return nh; }
-    __device__ int hole(int j) const { return __builtin_amdgcn_readfirstlane(L->hole_idx[L->hole_sel[j]]); }
-    __device__ bool hole_on(int j) const { return (L->hole_mask[L->hole_sel[j]] >> lane) & 1ull; }
+    __device__ const HoleRec& hole_rec(int j) const { return h[-j]; }
+    __device__ int hole(int j) const { return __builtin_amdgcn_readfirstlane(h[-j].hole); }
+    __device__ bool hole_on(int j) const { return lane_bit(uniform_u64(h[-j].lanes)); }
 };
 
-__device__ __forceinline__ int lanes_below(uint64_t m, int lane) {
-    return __popcll(m & ((1ull << lane) - 1ull));
-}
+// The same from the positions of the candidates in the list (the FP64 rays).
+template <class Lists>
+struct ListCands {
+    static constexpr bool kFastFaces = false;
+    const Lists* L;
+    const uint16_t* cur;  // bars, then holes
+    int nb, nh;
+    __device__ int nbars() const { return nb; }
+    __device__ int pos(int j) const { return cur[j]; }
+    __device__ int bar(int j) const { return __builtin_amdgcn_readfirstlane(L->idx[cur[j]]); }
+    __device__ bool bar_on(int j) const { return lane_bit(uniform_u64(L->arena[cur[j]])); }
+    __device__ int nholes() const { return nh; }
+    __device__ int hole(int j) const { return __builtin_amdgcn_readfirstlane(L->idx[cur[nb + j]]); }
+    __device__ bool hole_on(int j) const { return lane_bit(uniform_u64(L->arena[cur[nb + j]])); }
+};
 
 // Lane and tile state of one wave: voxel of the lane, tile bounding sphere
 // and the self-culling terms of bar d.
@@ -189,6 +202,38 @@ __device__ __forceinline__ void wave_setup(const PeLaunch& A, int d, int tile, i
     W.bar_gate = (uint32_t)__ballot(clear);
 }
 
+// Appends the passing lanes' candidates (numbers base + lane) to the list at
+// position n.  all: the culling test keeps the candidate for every lane (then
+// its mask is the valid lanes'); the others are tested per lane, and dropped when
+// no lane keeps them.  keep(k): this lane's culling test of candidate k.
+template <class Lists, class Keep>
+__device__ __forceinline__ void append_candidates(Lists& L, int cap, int first, int base, bool pass, bool all,
+                                                  uint64_t valid, int lane, int& n, Keep keep) {
+    uint64_t bal = __ballot(pass);
+    const uint64_t ball = __ballot(pass && all);
+    if (bal == ball) {
+        const int pos = n + __popcll(bal & ((1ull << lane) - 1ull));
+        if (pass && pos < cap) {
+            L.idx[first + pos] = (uint16_t)(base + lane);
+            L.arena[first + pos] = valid;
+        }
+        n += __popcll(bal);
+        return;
+    }
+    while (bal) {
+        const int bit = __ffsll((unsigned long long)bal) - 1;
+        bal &= bal - 1;
+        const uint64_t m = ((ball >> bit) & 1ull) ? valid : __ballot(keep(base + bit));
+        if (m) {
+            if (n < cap && lane == 0) {
+                L.idx[first + n] = (uint16_t)(base + bit);
+                L.arena[first + n] = m;
+            }
+            ++n;
+        }
+    }
+}
+
 // Step 1: candidate bars and holes of the tile: those whose box a segment from
 // bar d to the tile can meet (bar_tile_may_hit with the tile's half extents per
 // axis, which are what bounds the scan: a ball around a 4x4x4 tile is 1.7 times
@@ -197,17 +242,21 @@ __device__ __forceinline__ void wave_setup(const PeLaunch& A, int d, int tile, i
 // 177.4, one slice at 8x16x8 sub-cells 37.4 instead of 33.5; first on the box of each
 // group of kGroup consecutive bars or holes, then on the members of the
 // groups it keeps; any other has chord 0 for every ray of the tile, so its
-// culling decision does not matter), each with the ballot of the lanes whose
-// reference culling test keeps it.  Returns false on overflow.
+// culling decision does not matter), each with the lanes whose reference
+// culling test keeps it: all of them where cull_keeps_all shows so for the
+// tile (99.97% of the candidates on the full-size geometry), else by a ballot
+// of the lanes' tests.  Returns false on overflow.
 template <bool kExact, class Lists>
 __device__ bool build_candidates(const PeLaunch& A, int d, int lane, const WaveSetup& W,
                                  Lists& L, int& nb, int& nh) {
     const PeGeom& G = A.geom;
     const GeomDesc& g = G.g;
     const Bar<float>& bdf = G.bars_f[d];
+    const float cd[3] = {bdf.cx, bdf.cy, bdf.cz};
+    const float rho = float(W.rho) * 1.0001f;
+    const uint64_t valid = __ballot(W.valid);
     nb = 0;
     nh = 0;
-    for (int w = lane; w < (L.cap_bars + 63) / 64; w += 64) L.tile_far[w] = 0ull;
     // groups of kGroup bars first (one group box per lane), then the members
     // of each group that can be hit
     const int n_bg = (g.n_det + kGroup - 1) / kGroup;
@@ -222,35 +271,23 @@ __device__ bool build_candidates(const PeLaunch& A, int d, int lane, const WaveS
         while (gbal) {
             const int base = (g0 + __ffsll((unsigned long long)gbal) - 1) * kGroup;
             gbal &= gbal - 1;
-            int k = base + lane;
-            bool pass = false, far = false;
+            const int k = base + lane;
+            bool pass = false, all = false;
             if (k < g.n_det && k != d) {
                 const Bar<float>& b = G.bars_f[k];
                 float rt[3];
                 extents_in_frame(W.te, b.cb, b.sb, rt);
                 pass = bar_tile_may_hit(bdf, W.tcf, rt, b.cx, b.cy, b.cz, b.cb, b.sb, 0.5f * b.w,
                                         0.5f * b.t, 0.5f * b.h);
-                if (pass) far = fast_tile_far(G, k, W.tc, W.rho);
+                const float c[3] = {b.cx, b.cy, b.cz};
+                all = cull_keeps_all(W.tcf, rho, c, 0.5f * b.rdiag, cd, 0.5f * bdf.rdiag);
             }
-            uint64_t bal = __ballot(pass);
-            const uint64_t far_bal = __ballot(far);
-            while (bal) {
-                int bit = __ffsll((unsigned long long)bal) - 1;
-                bal &= bal - 1;
-                int kk = base + bit;
-                bool keep = W.valid && cull_bar<kExact>(G, kk, W.p, W.pf, W.sc, W.udf, W.critf);
-                uint64_t m = __ballot(keep);
-                if (m) {
-                    if (nb < L.cap_bars && lane == 0) {
-                        L.bar_idx[nb] = (uint16_t)kk;
-                        L.bar_mask[nb] = m;
-                        if ((far_bal >> bit) & 1ull) L.tile_far[nb >> 6] |= 1ull << (nb & 63);
-                    }
-                    ++nb;
-                }
-            }
+            append_candidates(L, L.cap_bars, 0, base, pass, all, valid, lane, nb, [&](int kk) {
+                return W.valid && cull_bar<kExact>(G, kk, W.p, W.pf, W.sc, W.udf, W.critf);
+            });
         }
     }
+    if (nb > L.cap_bars) return false;
     const int n_hg = (g.n_holes + kGroup - 1) / kGroup;
     for (int g0 = 0; g0 < n_hg; g0 += 64) {
         bool gpass = false;
@@ -263,50 +300,51 @@ __device__ bool build_candidates(const PeLaunch& A, int d, int lane, const WaveS
         while (gbal) {
             const int base = (g0 + __ffsll((unsigned long long)gbal) - 1) * kGroup;
             gbal &= gbal - 1;
-            int h = base + lane;
-            bool pass = false;
+            const int h = base + lane;
+            bool pass = false, all = false;
             if (h < g.n_holes) {
                 const Hole<float>& o = G.holes_f[h];
                 pass = bar_tile_may_hit(bdf, W.tcf, W.te, o.xc, o.ymid, o.zc, 1.0f, 0.0f, o.r,
                                         0.5f * tabs(o.y2 - o.y1), o.r);
+                const float c[3] = {o.xc, o.ymid, o.zc};
+                all = cull_keeps_all(W.tcf, rho, c, o.crit, cd, 0.5f * bdf.rdiag);
             }
-            uint64_t bal = __ballot(pass);
-            while (bal) {
-                int bit = __ffsll((unsigned long long)bal) - 1;
-                bal &= bal - 1;
-                int hh = base + bit;
-                bool keep = W.valid && cull_hole<kExact>(G, hh, W.p, W.pf, W.sc, W.udf, W.critf);
-                uint64_t m = __ballot(keep);
-                if (m) {
-                    if (nh < L.cap_holes && lane == 0) {
-                        L.hole_idx[nh] = (uint16_t)hh;
-                        L.hole_mask[nh] = m;
-                    }
-                    ++nh;
-                }
-            }
+            append_candidates(L, L.cap_holes, nb, base, pass, all, valid, lane, nh, [&](int hh) {
+                return W.valid && cull_hole<kExact>(G, hh, W.p, W.pf, W.sc, W.udf, W.critf);
+            });
         }
     }
-    return nb <= L.cap_bars && nh <= L.cap_holes;
+    return nh <= L.cap_holes;
 }
 
 // Sub-cell `cell` of bar d for this wave's tile (from the sub-cell table when
-// there is one), with the plate gates that no ray of the tile can trigger:
-// those cleared for the whole bar, else tested for the sub-cell point (one
-// layer per lane, then a ballot).
+// there is one: wave-uniform, so through the scalar unit), with the plate gates
+// that no ray of the tile can trigger: those cleared for the whole bar, else
+// tested for the sub-cell point (one layer per lane, then a ballot).
 __device__ __forceinline__ void tile_cell(const PeLaunch& A, const Bar<double>& bd, int d, int cell,
                                           const WaveSetup& W, int lane, CellCtx& cc) {
-    if (A.cells)
-        cc = A.cells[(int64_t)(d - A.cells_bar0) * (A.sub[0] * A.sub[1] * A.sub[2]) + cell];
-    else
+    if (A.cells) {
+        typedef const __attribute__((address_space(4))) CellCtx ScalarCell;
+        const int64_t i = (int64_t)(d - A.cells_bar0) * (A.sub[0] * A.sub[1] * A.sub[2]) + cell;
+        ScalarCell* c = (ScalarCell*)(A.cells + i);
+        for (int k = 0; k < 3; ++k) {
+            cc.q[k] = c->q[k];
+            cc.qs[k] = c->qs[k];
+            cc.lo[k] = c->lo[k];
+            cc.hi[k] = c->hi[k];
+            cc.area[k] = c->area[k];
+            cc.hc[k] = c->hc[k];
+        }
+    } else {
         make_cell_ctx_linear(bd, cell, A.sub, cc);
-    for (int k = 0; k < 3; ++k) {
-        cc.q[k] = uniform_d(cc.q[k]);
-        cc.qs[k] = uniform_d(cc.qs[k]);
-        cc.lo[k] = uniform_d(cc.lo[k]);
-        cc.hi[k] = uniform_d(cc.hi[k]);
-        cc.area[k] = uniform_d(cc.area[k]);
-        cc.hc[k] = uniform_f(cc.hc[k]);
+        for (int k = 0; k < 3; ++k) {
+            cc.q[k] = uniform_d(cc.q[k]);
+            cc.qs[k] = uniform_d(cc.qs[k]);
+            cc.lo[k] = uniform_d(cc.lo[k]);
+            cc.hi[k] = uniform_d(cc.hi[k]);
+            cc.area[k] = uniform_d(cc.area[k]);
+            cc.hc[k] = uniform_f(cc.hc[k]);
+        }
     }
     const GeomDesc& g = A.geom.g;
     const uint32_t all = (uint32_t)((1ull << g.n_layers) - 1ull);
@@ -319,62 +357,237 @@ __device__ __forceinline__ void tile_cell(const PeLaunch& A, const Bar<double>& 
     cc.gate_clear = W.bar_gate | (uint32_t)__ballot(clear);
 }
 
-// Step 2: candidates whose box a segment from the sub-cell centre qd to the
-// tile can meet (box_meets_frustum with a point source), bars and holes in
-// one pass; writes their list indices to bar_sel / hole_sel.
-template <class Lists>
-__device__ void narrow_candidates(const PeLaunch& A, const double qd[3], const WaveSetup& W,
-                                  int lane, Lists& L, int nb, int nh, int& nsb, int& nsh) {
-    const PeGeom& G = A.geom;
-    const float q[3] = {float(qd[0]), float(qd[1]), float(qd[2])};
-    const float rq[3] = {0.0f, 0.0f, 0.0f};
-    nsb = 0;
-    nsh = 0;
-    const int n = nb + nh;
-    for (int base = 0; base < n; base += 64) {
-        const int j = base + lane;
-        const bool is_bar = j < nb;
-        bool pass = false;
-        if (j < n) {
-            float c[3], cb, sb, h[3];
-            if (is_bar) {
-                const Bar<float>& bf = G.bars_f[L.bar_idx[j]];
-                c[0] = bf.cx; c[1] = bf.cy; c[2] = bf.cz;
-                cb = bf.cb; sb = bf.sb;
-                h[0] = 0.5f * bf.w; h[1] = 0.5f * bf.t; h[2] = 0.5f * bf.h;
-            } else {
-                const Hole<float>& o = G.holes_f[L.hole_idx[j - nb]];
-                c[0] = o.xc; c[1] = o.ymid; c[2] = o.zc;
-                cb = 1.0f; sb = 0.0f;
-                h[0] = o.r; h[1] = 0.5f * tabs(o.y2 - o.y1); h[2] = o.r;
-            }
-            float rt[3];
-            extents_in_frame(W.te, cb, sb, rt);
-            pass = box_meets_frustum(q, rq, W.tcf, rt, c[0], c[1], c[2], cb, sb, h[0], h[1], h[2]);
-        }
-        const uint64_t bb = __ballot(pass && is_bar), bh = __ballot(pass && !is_bar);
-        if (pass) {
-            if (is_bar) {
-                const int pos = nsb + lanes_below(bb, lane);
-                L.bar_sel[pos] = (uint16_t)j;
-                if (pos < kFastBars) {
-                    float f[6];
-                    // fast_faces: the tile part once per tile (build_candidates)
-                    const bool near_q_ok = fast_faces_q(G, L.bar_idx[j], qd, f);
-                    L.fast_ok[pos] = ((L.tile_far[j >> 6] >> (j & 63)) & 1ull) && near_q_ok ? 1 : 0;
-#pragma unroll
-                    for (int i = 0; i < 6; ++i) L.faces[pos][i] = f[i];
-                    L.faces[pos][6] = G.bars_f[L.bar_idx[j]].mut;
-                }
-            } else {
-                L.hole_sel[nsh + lanes_below(bh, lane)] = (uint16_t)(j - nb);
-            }
-        }
-        nsb += __popcll(bb);
-        nsh += __popcll(bh);
+// Centre of this lane's sub-cell `cell` of bar d.
+__device__ __forceinline__ void cell_point(const PeLaunch& A, const Bar<double>& bd, int d, int cell, double q[3]) {
+    if (A.cells) {
+        const CellCtx& c = A.cells[(int64_t)(d - A.cells_bar0) * (A.sub[0] * A.sub[1] * A.sub[2]) + cell];
+        for (int k = 0; k < 3; ++k) q[k] = c.q[k];
+    } else {
+        CellCtx c;
+        make_cell_ctx_linear(bd, cell, A.sub, c);
+        for (int k = 0; k < 3; ++k) q[k] = c.q[k];
     }
 }
 
+// Step 2: the candidates whose box a segment from a sub-cell centre to the
+// tile can meet (box_meets_frustum with a point source), for ns sub-cells at
+// once (lane s holds the number of the s-th in my_cell): bit j % 64 of
+// sel[s * words + j / 64] for candidate j.  A lane keeps one candidate's box for
+// all of them, and with at most 32 candidates a pass takes several sub-cells.
+// (One sub-cell per pass, its candidates' records gathered anew for each, was a
+// quarter of the PE kernel's instructions and most of its waits: full-size step
+// 177.4 ms, with this form 169.8 ms; 64-bar slice, one wave per SIMD, 274 -> 246 us.)
+template <class Lists>
+__device__ __forceinline__ void select_cells(const PeLaunch& A, const Bar<double>& bd, int d, int my_cell, int ns,
+                                             const WaveSetup& W, int lane, Lists& L, int nb, int n, int words) {
+    const PeGeom& G = A.geom;
+    float q0 = 0.0f, q1 = 0.0f, q2 = 0.0f;
+    if (lane < ns) {
+        double q[3];
+        cell_point(A, bd, d, my_cell, q);
+        q0 = float(q[0]);
+        q1 = float(q[1]);
+        q2 = float(q[2]);
+    }
+    const int per = n > 0 && n <= 32 ? 64 / n : 1;  // sub-cells per pass
+    const int sub = per > 1 ? lane / n : 0;         // this lane's sub-cell of the pass
+    for (int w = 0; w < words; ++w) {
+        const int j = per > 1 ? lane - sub * n : w * 64 + lane;
+        const bool act = j < n && sub < per;
+        float c[3] = {0.0f, 0.0f, 0.0f}, cb = 1.0f, sb = 0.0f, h[3] = {0.0f, 0.0f, 0.0f};
+        if (act) {
+            if (j < nb) {
+                const Bar<float>& b = G.bars_f[L.idx[j]];
+                c[0] = b.cx; c[1] = b.cy; c[2] = b.cz;
+                cb = b.cb; sb = b.sb;
+                h[0] = 0.5f * b.w; h[1] = 0.5f * b.t; h[2] = 0.5f * b.h;
+            } else {
+                const Hole<float>& o = G.holes_f[L.idx[j]];
+                c[0] = o.xc; c[1] = o.ymid; c[2] = o.zc;
+                h[0] = o.r; h[1] = 0.5f * tabs(o.y2 - o.y1); h[2] = o.r;
+            }
+        }
+        float rt[3];
+        extents_in_frame(W.te, cb, sb, rt);
+        for (int s0 = 0; s0 < ns; s0 += per) {
+            const int s = s0 + sub;
+            const float q[3] = {__shfl(q0, s & 63), __shfl(q1, s & 63), __shfl(q2, s & 63)};
+            const float rq[3] = {0.0f, 0.0f, 0.0f};
+            const bool pass = act && s < ns &&
+                              box_meets_frustum(q, rq, W.tcf, rt, c[0], c[1], c[2], cb, sb, h[0], h[1], h[2]);
+            const uint64_t bal = __ballot(pass);
+            if (per > 1) {
+                if (act && j == 0 && s < ns) L.sel[s] = (bal >> lane) & ((1ull << n) - 1ull);
+            } else if (lane == 0) {
+                L.sel[s * words + w] = bal;
+            }
+        }
+    }
+}
+
+// The candidates of word w of sub-cell s: bars in mb, holes in mh.
+template <class Lists>
+__device__ __forceinline__ void sel_word(const Lists& L, int s, int words, int w, int nb, uint64_t& mb, uint64_t& mh) {
+    const uint64_t m = uniform_u64(L.sel[s * words + w]);
+    const int lead = nb - w * 64;  // bars in this word
+    const uint64_t bars = lead >= 64 ? ~0ull : (lead <= 0 ? 0ull : (1ull << lead) - 1ull);
+    mb = m & bars;
+    mh = m & ~bars;
+}
+
+// Bars and holes kept for sub-cell s.
+template <class Lists>
+__device__ __forceinline__ void sel_count(const Lists& L, int s, int words, int nb, int& kb, int& kh) {
+    kb = 0;
+    kh = 0;
+    for (int w = 0; w < words; ++w) {
+        uint64_t mb, mh;
+        sel_word(L, s, words, w, nb, mb, mh);
+        kb += __popcll(mb);
+        kh += __popcll(mh);
+    }
+}
+
+// Sub-cells c_begin .. c_end - 1 of bar d for the tile, in blocks: narrowing
+// (step 2), the records of the pairs it keeps, then the rays.  use(cell)
+// (wave-uniform) leaves sub-cells out; f32(cell, cc, C) traces the lanes' FP32
+// rays and returns the lanes whose decisions came within tolerance of a
+// threshold; f64(cell, cc, C, mine) traces in FP64 the rays of the lanes with
+// mine set: in the FP32 kernels those of a block's flagged rays, after its FP32
+// rays (which keeps the FP64 ray's registers out of the FP32 loop), in the
+// all-FP64 kernels every ray.
+template <bool kExact, bool kUse, class Lists, class Use, class F32, class F64>
+__device__ __forceinline__ void trace_cells(const PeLaunch& A, const Bar<double>& bd, int d, int c_begin, int c_end,
+                                            const WaveSetup& W, int lane, Lists& L, int nb, int nh, Use use, F32 f32,
+                                            F64 f64) {
+    const PeGeom& G = A.geom;
+    const int n = nb + nh, words = (n + 63) / 64;
+    const int block = words > 1 ? min(kBlockCells, L.sel_cap / words) : kBlockCells;
+    const uint64_t below = (1ull << lane) - 1ull;
+    BarRec* const bars = (BarRec*)&L.arena[n];
+    HoleRec* const holes = (HoleRec*)&L.arena[L.arena_words - (int)(sizeof(HoleRec) / 8)];
+    constexpr int kBarWords = sizeof(BarRec) / 8, kHoleWords = sizeof(HoleRec) / 8;
+    const int room = L.arena_words - n;
+    int c = c_begin;
+    while (c < c_end) {  // wave-uniform
+        int ns = 0, my_cell = c + lane;
+        if constexpr (kUse) {
+            for (; c < c_end && ns < block; ++c)
+                if (use(c)) {
+                    if (lane == ns) my_cell = c;
+                    ++ns;
+                }
+        } else {
+            ns = min(block, c_end - c);
+            c += ns;
+        }
+        __syncthreads();  // the previous block's lists are no longer read
+        select_cells(A, bd, d, my_cell, ns, W, lane, L, nb, n, words);
+        __syncthreads();
+        uint64_t flagged = 0;
+        if constexpr (kExact) {
+            flagged = ns == 64 ? ~0ull : (1ull << ns) - 1ull;
+        } else {
+            int s = 0;
+            while (s < ns) {
+                // the records of as many sub-cells as fit: first their pairs
+                int e = s, nbr = 0, nhr = 0;
+                for (; e < ns; ++e) {
+                    int kb, kh;
+                    sel_count(L, e, words, nb, kb, kh);
+                    if ((nbr + kb) * kBarWords + (nhr + kh) * kHoleWords > room) break;
+                    for (int w = 0; w < words; ++w) {
+                        uint64_t mb, mh;
+                        sel_word(L, e, words, w, nb, mb, mh);
+                        const uint32_t tag = ((uint32_t)e << 16) | (uint32_t)(w * 64 + lane);
+                        if (lane_bit(mb)) bars[nbr + __popcll(mb & below)].tag = tag;
+                        if (lane_bit(mh)) holes[-(nhr + __popcll(mh & below))].tag = tag;
+                        nbr += __popcll(mb);
+                        nhr += __popcll(mh);
+                    }
+                }
+                if (e == s) {  // not even one sub-cell's: its rays go to FP64
+                    flagged |= 1ull << s;
+                    if (lane == 0) L.redo[s] = ~0ull;
+                    ++s;
+                    continue;
+                }
+                __syncthreads();
+                for (int i0 = 0; i0 < nbr; i0 += 64) {
+                    const int i = i0 + lane;
+                    const uint32_t tag = i < nbr ? bars[i].tag : 0u;
+                    const int cell = __shfl(my_cell, (int)(tag >> 16) & 63);
+                    if (i < nbr) {
+                        const int j = tag & 0xffff, k = L.idx[j];
+                        double q[3];
+                        cell_point(A, bd, d, cell, q);
+                        float f[6];
+                        const bool fast = fast_faces(G, k, q, W.tc, W.rho, f);
+                        BarRec& r = bars[i];
+#pragma unroll
+                        for (int m = 0; m < 6; ++m) r.face[m] = f[m];
+                        r.mu = G.bars_f[k].mut;
+                        r.tag = (uint32_t)j | (fast ? kFastBar : 0u);
+                        r.lanes = L.arena[j];
+                    }
+                }
+                for (int i = lane; i < nhr; i += 64) {
+                    HoleRec& r = holes[-i];
+                    const int j = r.tag & 0xffff, k = L.idx[j];
+                    const Hole<double>& o = G.holes_d[k];
+                    r.xc = o.xc;
+                    r.y1 = o.y1;
+                    r.y2 = o.y2;
+                    r.zc = o.zc;
+                    r.r = o.r;
+                    r.mu = o.mu;
+                    r.lanes = L.arena[j];
+                    r.hole = (uint32_t)k;
+                }
+                __syncthreads();
+                int ib = 0, ih = 0;
+                for (; s < e; ++s) {
+                    const int cell = __builtin_amdgcn_readlane(my_cell, s);
+                    CellCtx cc;
+                    tile_cell(A, bd, d, cell, W, lane, cc);
+                    RecCands<Lists> C{&L, bars + ib, holes - ih, 0, 0};
+                    sel_count(L, s, words, nb, C.nb, C.nh);
+                    ib += C.nb;
+                    ih += C.nh;
+                    const uint64_t m = __ballot(f32(cell, cc, C));
+                    if (m) {
+                        flagged |= 1ull << s;
+                        if (lane == 0) L.redo[s] = m;
+                    }
+                }
+                __syncthreads();
+            }
+        }
+        // FP64 rays: the candidates' positions in the place of the records
+        uint16_t* const cur = (uint16_t*)bars;
+        while (flagged) {
+            const int s = __ffsll((unsigned long long)flagged) - 1;
+            flagged &= flagged - 1;
+            const int cell = __builtin_amdgcn_readlane(my_cell, s);
+            CellCtx cc;
+            tile_cell(A, bd, d, cell, W, lane, cc);
+            ListCands<Lists> C{&L, cur, 0, 0};
+            sel_count(L, s, words, nb, C.nb, C.nh);
+            __syncthreads();
+            int ib = 0, ih = C.nb;
+            for (int w = 0; w < words; ++w) {
+                uint64_t mb, mh;
+                sel_word(L, s, words, w, nb, mb, mh);
+                if (lane_bit(mb)) cur[ib + __popcll(mb & below)] = (uint16_t)(w * 64 + lane);
+                if (lane_bit(mh)) cur[ih + __popcll(mh & below)] = (uint16_t)(w * 64 + lane);
+                ib += __popcll(mb);
+                ih += __popcll(mh);
+            }
+            __syncthreads();
+            f64(cell, cc, C, W.valid && (kExact || ((L.redo[s] >> lane) & 1ull)));
+        }
+    }
+}
 
 // Point weights of the crystal grid scatterers (kPoints; an extension with no
 // reference counterpart): the sub-cells of bar d are the grid cells, and for
@@ -466,77 +679,50 @@ __device__ __forceinline__ bool pe_forward_body(const PeLaunch& A, int item, Lis
     KahanSum<T> acc;
     unsigned fallbacks = 0;
     // Sub-cells in the reference's loop order (z outer, then x, then y;
-    // PESysMatGen.cu:1193-1197).  FP32 path: a ray whose decisions came
-    // within tolerance of a threshold is not added; its sub-cell goes to a
-    // per-wave queue with the ballot of such lanes, and the queue is redone
-    // in FP64 when full and at the end.  Keeping the FP64 ray out of the FP32
-    // loop keeps the loop's register use low.
-    __shared__ uint16_t redo_cell[kRedoCap];
-    __shared__ uint64_t redo_mask[kRedoCap];
-    int cell = c_begin;
-    while (cell < c_end) {
-        int n_redo = 0;
-        for (; cell < c_end && n_redo < kRedoCap; ++cell) {
-            CellCtx cc;
-            tile_cell(A, bd, d, cell, W, lane, cc);
-            if constexpr (kPoints) {
-                if (A.n_use_rows > 0 && !point_used(A, W, cc.q, lane)) {  // wave-uniform
+    // PESysMatGen.cu:1193-1197); FP32 rays whose decisions came within
+    // tolerance of a threshold are not added but redone in FP64.
+    auto use = [&](int cell) {
+        if constexpr (kPoints) {
+            if (A.n_use_rows > 0) {
+                double q[3];
+                cell_point(A, bd, d, cell, q);
+                if (!point_used(A, W, q, lane)) {  // wave-uniform
                     if (W.valid) pts[(int64_t)cell * g.n_vox + W.v] = 0.0f;
-                    continue;
+                    return false;
                 }
             }
-            int nsb, nsh;
-            __syncthreads();
-            narrow_candidates(A, cc.q, W, lane, L, nb, nh, nsb, nsh);
-            __syncthreads();
+        }
+        return true;
+    };
+    trace_cells<kExact, kPoints>(
+        A, bd, d, c_begin, c_end, W, lane, L, nb, nh, use,
+        [&](int cell, const CellCtx& cc, const RecCands<Lists>& C) {
             bool near = false;
             if (W.valid) {
-                ListCands<Lists> C{&L, nsb, nsh, lane};
                 if constexpr (kPoints) {
                     double aux[8];
-                    pe_cell_ray<T, kEll>(G, d, W.p, W.ps, cc, C, near, nullptr, aux);
-                    if (!near)
-                        pts[(int64_t)cell * g.n_vox + W.v] =
-                            kExact ? point_weight(bd, n_cells, aux) : point_weight_f(bd, n_cells, aux);
+                    pe_cell_ray<float, kEll>(G, d, W.p, W.ps, cc, C, near, nullptr, aux);
+                    if (!near) pts[(int64_t)cell * g.n_vox + W.v] = point_weight_f(bd, n_cells, aux);
                 } else {
-                    T val = pe_cell_ray<T, kEll>(G, d, W.p, W.ps, cc, C, near);
-                    if (!near) acc.add(val);
+                    const float val = pe_cell_ray<float, kEll>(G, d, W.p, W.ps, cc, C, near);
+                    if (!near) acc.add((T)val);
                 }
             }
-            if constexpr (!kExact) {
-                const uint64_t m = __ballot(near);
-                if (m) {
-                    if (lane == 0) {
-                        redo_cell[n_redo] = (uint16_t)cell;
-                        redo_mask[n_redo] = m;
-                    }
-                    ++n_redo;
+            return near;
+        },
+        [&](int cell, const CellCtx& cc, const ListCands<Lists>& C, bool mine) {
+            if (mine) {
+                bool n2 = false;
+                if constexpr (kPoints) {
+                    double aux[8];
+                    pe_cell_ray<double, kEll>(G, d, W.p, W.ps, cc, C, n2, nullptr, aux);
+                    pts[(int64_t)cell * g.n_vox + W.v] = point_weight(bd, n_cells, aux);
+                } else {
+                    acc.add((T)pe_cell_ray<double, kEll>(G, d, W.p, W.ps, cc, C, n2));
                 }
+                ++fallbacks;
             }
-        }
-        if constexpr (!kExact) {
-            for (int i = 0; i < n_redo; ++i) {
-                CellCtx cc;
-                tile_cell(A, bd, d, redo_cell[i], W, lane, cc);
-                int rsb, rsh;
-                __syncthreads();
-                narrow_candidates(A, cc.q, W, lane, L, nb, nh, rsb, rsh);
-                __syncthreads();
-                if ((redo_mask[i] >> lane) & 1ull) {
-                    ListCands<Lists> C{&L, rsb, rsh, lane};
-                    bool n2 = false;
-                    if constexpr (kPoints) {
-                        double aux[8];
-                        pe_cell_ray<double, kEll>(G, d, W.p, W.ps, cc, C, n2, nullptr, aux);
-                        pts[(int64_t)redo_cell[i] * g.n_vox + W.v] = point_weight(bd, n_cells, aux);
-                    } else {
-                        acc.add((T)pe_cell_ray<double, kEll>(G, d, W.p, W.ps, cc, C, n2));
-                    }
-                    ++fallbacks;
-                }
-            }
-        }
-    }
+        });
     if constexpr (!kPoints) {
         if (W.valid) out[W.v] = float(acc.value());
     }
@@ -637,60 +823,32 @@ __device__ __forceinline__ bool pe_tangent_body(const PeLaunch& A, const PeTange
     KahanSum<double> dacc;
     unsigned fallbacks = 0;
     const double* vbar = TG.v + g.n_layers;
-    __shared__ uint16_t redo_cell[kRedoCap];
-    __shared__ uint64_t redo_mask[kRedoCap];
-    int cell = 0;
-    while (cell < n_cells) {
-        int n_redo = 0;
-        for (; cell < n_cells && n_redo < kRedoCap; ++cell) {
-            CellCtx cc;
-            tile_cell(A, bd, d, cell, W, lane, cc);
-            int nsb, nsh;
-            __syncthreads();
-            narrow_candidates(A, cc.q, W, lane, L, nb, nh, nsb, nsh);
-            __syncthreads();
+    trace_cells<kExact, false>(
+        A, bd, d, 0, n_cells, W, lane, L, nb, nh, [](int) { return true; },
+        [&](int, const CellCtx& cc, const RecCands<Lists>& C) {
             bool near = false;
             if (W.valid) {
-                ListCands<Lists> C{&L, nsb, nsh, lane};
                 double dlay[kMaxLayers], aux[8], tatt = 0.0;
-                T val = pe_cell_ray<T, kExact>(G, d, W.p, W.ps, cc, C, near, dlay, aux, nullptr, 0, vbar, &tatt);
+                const float val = pe_cell_ray<float, false>(G, d, W.p, W.ps, cc, C, near, dlay, aux, nullptr, 0,
+                                                            vbar, &tatt);
                 if (!near) {
-                    acc.add(val);
+                    acc.add((T)val);
                     dacc.add(tangent_term(G, d, TG.v, (double)val, dlay, aux, tatt));
                 }
             }
-            if constexpr (!kExact) {
-                const uint64_t m = __ballot(near);
-                if (m) {
-                    if (lane == 0) {
-                        redo_cell[n_redo] = (uint16_t)cell;
-                        redo_mask[n_redo] = m;
-                    }
-                    ++n_redo;
-                }
+            return near;
+        },
+        [&](int, const CellCtx& cc, const ListCands<Lists>& C, bool mine) {
+            if (mine) {
+                bool n2 = false;
+                double dlay[kMaxLayers], aux[8], tatt = 0.0;
+                const double val = pe_cell_ray<double, kExact>(G, d, W.p, W.ps, cc, C, n2, dlay, aux, nullptr, 0,
+                                                               vbar, &tatt);
+                acc.add((T)val);
+                dacc.add(tangent_term(G, d, TG.v, val, dlay, aux, tatt));
+                ++fallbacks;
             }
-        }
-        if constexpr (!kExact) {
-            for (int i = 0; i < n_redo; ++i) {
-                CellCtx cc;
-                tile_cell(A, bd, d, redo_cell[i], W, lane, cc);
-                int rsb, rsh;
-                __syncthreads();
-                narrow_candidates(A, cc.q, W, lane, L, nb, nh, rsb, rsh);
-                __syncthreads();
-                if ((redo_mask[i] >> lane) & 1ull) {
-                    ListCands<Lists> C{&L, rsb, rsh, lane};
-                    bool n2 = false;
-                    double dlay[kMaxLayers], aux[8], tatt = 0.0;
-                    const double val = pe_cell_ray<double, kExact>(G, d, W.p, W.ps, cc, C, n2, dlay, aux,
-                                                                   nullptr, 0, vbar, &tatt);
-                    acc.add((T)val);
-                    dacc.add(tangent_term(G, d, TG.v, val, dlay, aux, tatt));
-                    ++fallbacks;
-                }
-            }
-        }
-    }
+        });
     if (W.valid) {
         TG.d_out[o] = float(dacc.value());
         if (TG.a_out) TG.a_out[o] = float(acc.value());
@@ -754,10 +912,9 @@ struct AdjAcc {
 // FP32 a lane whose ray came within tolerance of a threshold contributes
 // nothing and is reported through the return value (the caller redoes it in
 // FP64).  Every lane of the wave takes part in the wave sums.
-template <class T, bool kEll, class Lists>
-__device__ bool adjoint_cell(const PeGeom& G, int d, int lane, const WaveSetup& W,
-                             const Lists& L, const ListCands<Lists>& C, const CellCtx& cc,
-                             bool active, double wv, AdjAcc& acc, double* lay_acc,
+template <class T, bool kEll, class Cands>
+__device__ bool adjoint_cell(const PeGeom& G, int d, int lane, const WaveSetup& W, const Cands& C,
+                             const CellCtx& cc, bool active, double wv, AdjAcc& acc, double* lay_acc,
                              double* cand_acc, float* keep = nullptr) {
     const GeomDesc& g = G.g;
     const Bar<double>& bd = G.bars_d[d];
@@ -807,7 +964,7 @@ __device__ bool adjoint_cell(const PeGeom& G, int d, int lane, const WaveSetup& 
             x = -cw * l;
         }
         x = wave_sum(x);
-        if (lane == 0) cand_acc[L.bar_sel[j]] += x;
+        if (lane == 0) cand_acc[C.pos(j)] += x;
     }
     return near;
 }
@@ -821,8 +978,6 @@ __device__ __forceinline__ bool pe_backward_body(const PeLaunch& A, const PeGrad
                                                  Lists& L, double* cand_acc) {
     __shared__ double lay_acc[kMaxLayers];
     __shared__ float keep[kKeepChords * 64];  // FP32 rays' chords, [candidate][lane]
-    __shared__ uint16_t redo_cell[kRedoCap];
-    __shared__ uint64_t redo_mask[kRedoCap];
     const PeGeom& G = A.geom;
     const GeomDesc& g = G.g;
     const int lane = threadIdx.x;
@@ -840,7 +995,6 @@ __device__ __forceinline__ bool pe_backward_body(const PeLaunch& A, const PeGrad
     bool overflow = false;
     __syncthreads();
     if (bd.mut > (double)0.01f) {
-        using T = typename std::conditional<kExact, double, float>::type;
         const int n_cells = A.sub[0] * A.sub[1] * A.sub[2];
         // work items: (tile, range of sub-cells); item i is tile i / cs, range i % cs
         const int cs = S.cell_slices;
@@ -858,51 +1012,20 @@ __device__ __forceinline__ bool pe_backward_body(const PeLaunch& A, const PeGrad
             for (int j = lane; j < nb; j += 64) cand_acc[j] = 0.0;
             const double wv = W.valid ? (double)S.w[(int64_t)d * g.n_vox + W.v] : 0.0;
             __syncthreads();
-            // sub-cells in the reference's order; FP32 rays near a threshold
-            // are queued and redone in FP64 (as in the forward kernel)
-            int cell = c_begin;
-            while (cell < c_end) {
-                int n_redo = 0;
-                for (; cell < c_end && n_redo < kRedoCap; ++cell) {
-                    CellCtx cc;
-                    tile_cell(A, bd, d, cell, W, lane, cc);
-                    int nsb, nsh;
-                    __syncthreads();
-                    narrow_candidates(A, cc.q, W, lane, L, nb, nh, nsb, nsh);
-                    __syncthreads();
-                    ListCands<Lists> C{&L, nsb, nsh, lane};
-                    const bool near = adjoint_cell<T, kExact>(G, d, lane, W, L, C, cc, W.valid, wv, acc,
-                                                      lay_acc, cand_acc, kExact ? nullptr : keep + lane);
-                    if constexpr (!kExact) {
-                        const uint64_t m = __ballot(near);
-                        if (m) {
-                            if (lane == 0) {
-                                redo_cell[n_redo] = (uint16_t)cell;
-                                redo_mask[n_redo] = m;
-                            }
-                            ++n_redo;
-                        }
-                    }
-                    __syncthreads();
-                }
-                if constexpr (!kExact) {
-                    for (int i = 0; i < n_redo; ++i) {
-                        CellCtx cc;
-                        tile_cell(A, bd, d, redo_cell[i], W, lane, cc);
-                        int rsb, rsh;
-                        __syncthreads();
-                        narrow_candidates(A, cc.q, W, lane, L, nb, nh, rsb, rsh);
-                        __syncthreads();
-                        ListCands<Lists> C{&L, rsb, rsh, lane};
-                        const bool mine = (redo_mask[i] >> lane) & 1ull;
-                        adjoint_cell<double, kExact>(G, d, lane, W, L, C, cc, mine, wv, acc, lay_acc, cand_acc);
-                        fallbacks += mine;
-                    }
-                }
-            }
+            trace_cells<kExact, false>(
+                A, bd, d, c_begin, c_end, W, lane, L, nb, nh, [](int) { return true; },
+                [&](int, const CellCtx& cc, const RecCands<Lists>& C) {
+                    return adjoint_cell<float, false>(G, d, lane, W, C, cc, W.valid, wv, acc, lay_acc, cand_acc,
+                                                      keep + lane);
+                },
+                [&](int, const CellCtx& cc, const ListCands<Lists>& C, bool mine) {
+                    adjoint_cell<double, kExact>(G, d, lane, W, C, cc, mine, wv, acc, lay_acc, cand_acc);
+                    fallbacks += mine;
+                });
+            __syncthreads();
             // fold this tile's candidate partials into the dense row (one
             // entry per candidate, each bar at most once per tile)
-            for (int j = lane; j < nb; j += 64) out_row[L.bar_idx[j]] += cand_acc[j];
+            for (int j = lane; j < nb; j += 64) out_row[L.idx[j]] += cand_acc[j];
             __syncthreads();
         }
     }
@@ -993,7 +1116,7 @@ __global__ __launch_bounds__(256) void pe_grad_reduce(PeGradScratch S, int n_det
 // the candidates overflow L; adds the lane's FP64 re-computations to fallbacks.
 template <bool kExact, bool kEll, class Lists>
 __device__ bool pe_element(const PeLaunch& A, int d, int lane, const WaveSetup& W, Lists& L,
-                           uint16_t* redo_cell, uint64_t* redo_mask, unsigned& fallbacks, double& a) {
+                           unsigned& fallbacks, double& a) {
     const PeGeom& G = A.geom;
     const Bar<double>& bd = G.bars_d[d];
     a = 0.0;
@@ -1004,51 +1127,23 @@ __device__ bool pe_element(const PeLaunch& A, int d, int lane, const WaveSetup& 
     __syncthreads();
     using T = typename std::conditional<kExact, double, float>::type;
     KahanSum<T> acc;
-    const int n_cells = A.sub[0] * A.sub[1] * A.sub[2];
-    int cell = 0;
-    while (cell < n_cells) {
-        int n_redo = 0;
-        for (; cell < n_cells && n_redo < kRedoCap; ++cell) {
-            CellCtx cc;
-            tile_cell(A, bd, d, cell, W, lane, cc);
-            int nsb, nsh;
-            __syncthreads();
-            narrow_candidates(A, cc.q, W, lane, L, nb, nh, nsb, nsh);
-            __syncthreads();
+    trace_cells<kExact, false>(
+        A, bd, d, 0, A.sub[0] * A.sub[1] * A.sub[2], W, lane, L, nb, nh, [](int) { return true; },
+        [&](int, const CellCtx& cc, const RecCands<Lists>& C) {
             bool near = false;
             if (W.valid) {
-                ListCands<Lists> C{&L, nsb, nsh, lane};
-                T val = pe_cell_ray<T, kEll>(G, d, W.p, W.ps, cc, C, near);
-                if (!near) acc.add(val);
+                const float val = pe_cell_ray<float, kEll>(G, d, W.p, W.ps, cc, C, near);
+                if (!near) acc.add((T)val);
             }
-            if constexpr (!kExact) {
-                const uint64_t m = __ballot(near);
-                if (m) {
-                    if (lane == 0) {
-                        redo_cell[n_redo] = (uint16_t)cell;
-                        redo_mask[n_redo] = m;
-                    }
-                    ++n_redo;
-                }
+            return near;
+        },
+        [&](int, const CellCtx& cc, const ListCands<Lists>& C, bool mine) {
+            if (mine) {
+                bool n2 = false;
+                acc.add((T)pe_cell_ray<double, kEll>(G, d, W.p, W.ps, cc, C, n2));
+                ++fallbacks;
             }
-        }
-        if constexpr (!kExact) {
-            for (int i = 0; i < n_redo; ++i) {
-                CellCtx cc;
-                tile_cell(A, bd, d, redo_cell[i], W, lane, cc);
-                int rsb, rsh;
-                __syncthreads();
-                narrow_candidates(A, cc.q, W, lane, L, nb, nh, rsb, rsh);
-                __syncthreads();
-                if ((redo_mask[i] >> lane) & 1ull) {
-                    ListCands<Lists> C{&L, rsb, rsh, lane};
-                    bool n2 = false;
-                    acc.add((T)pe_cell_ray<double, kEll>(G, d, W.p, W.ps, cc, C, n2));
-                    ++fallbacks;
-                }
-            }
-        }
-    }
+        });
     // the element as the matrix kernel stores it (FP32), so that projecting
     // equals multiplying by the stored matrix
     a = (double)float(acc.value());
@@ -1067,8 +1162,6 @@ __device__ __forceinline__ void add_fallbacks(const PeLaunch& A, int lane, unsig
 template <bool kExact, bool kEll, class Lists>
 __device__ __forceinline__ bool pe_project_body(const PeLaunch& A, const float* x, double* partial, int item,
                                                 Lists& L) {
-    __shared__ uint16_t redo_cell[kRedoCap];
-    __shared__ uint64_t redo_mask[kRedoCap];
     const int lane = threadIdx.x;
     const int n_tiles = A.tiles[0] * A.tiles[1] * A.tiles[2];
     const int d = item / n_tiles;
@@ -1077,7 +1170,7 @@ __device__ __forceinline__ bool pe_project_body(const PeLaunch& A, const float* 
     wave_setup(A, d, tile, lane, W);
     unsigned fallbacks = 0;
     double a;
-    if (!pe_element<kExact, kEll>(A, d, lane, W, L, redo_cell, redo_mask, fallbacks, a)) return false;
+    if (!pe_element<kExact, kEll>(A, d, lane, W, L, fallbacks, a)) return false;
     const double s = wave_sum(W.valid ? a * (double)x[W.v] : 0.0);
     if (lane == 0) partial[item] = s;
     if constexpr (!kExact) add_fallbacks(A, lane, fallbacks);
@@ -1097,8 +1190,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pe
 template <bool kExact, bool kEll, class Lists>
 __device__ __forceinline__ bool pe_backproject_body(const PeLaunch& A, const float* y, int group,
                                                     double* partial, int item, Lists& L) {
-    __shared__ uint16_t redo_cell[kRedoCap];
-    __shared__ uint64_t redo_mask[kRedoCap];
     const GeomDesc& g = A.geom.g;
     const int lane = threadIdx.x;
     const int n_tiles = A.tiles[0] * A.tiles[1] * A.tiles[2];
@@ -1113,7 +1204,7 @@ __device__ __forceinline__ bool pe_backproject_body(const PeLaunch& A, const flo
         WaveSetup W;
         wave_setup(A, d, tile, lane, W);
         double a;
-        if (!pe_element<kExact, kEll>(A, d, lane, W, L, redo_cell, redo_mask, fallbacks, a)) return false;
+        if (!pe_element<kExact, kEll>(A, d, lane, W, L, fallbacks, a)) return false;
         acc += a * (double)yd;
     }
     // the lane's voxel (it does not depend on the bar)

@@ -156,6 +156,36 @@ SMG_FN bool cull_hole(const PeGeom& G, int h, const double p[3], const float pf[
     return cull_test<double>(p[0], p[1], p[2], o.xc, o.ymid, o.zc, o.crit, 0.0, sc.ud, sc.crit, near);
 }
 
+// True when the culling test keeps the sphere (centre c, numerator num of its
+// criterion: rdiag / 2 of a bar, crit of a hole) for every voxel of the ball
+// (tc, rho), seen with bar d (centre cd, rdiag / 2 in num_d).  Seen from a point
+// of the ball a centre at distance L from tc is turned by at most
+// rho / (L - rho) (chord of the angle asin(rho / L)) and is at most L + rho away,
+// so the angular distance and the limit of every voxel are within those bounds
+// of the ball centre's; the margin 1e-4 is above the FP32 rounding (~1e-6).
+SMG_FN bool cull_keeps_all(const float tc[3], float rho, const float c[3], float num, const float cd[3],
+                           float num_d) {
+    float e[3], f[3], le = 0.0f, lf = 0.0f;
+    for (int k = 0; k < 3; ++k) {
+        e[k] = c[k] - tc[k];
+        f[k] = cd[k] - tc[k];
+        le += e[k] * e[k];
+        lf += f[k] * f[k];
+    }
+    le = tsqrt(le);
+    lf = tsqrt(lf);
+    if (!(le > 2.0f * rho + 0.01f) || !(lf > 2.0f * rho + 0.01f)) return false;
+    const float re = trcp(le), rf = trcp(lf);
+    float s = 0.0f;
+    for (int k = 0; k < 3; ++k) {
+        const float d = e[k] * re - f[k] * rf;
+        s += d * d;
+    }
+    const float turn = tdiv(rho, le - rho) + tdiv(rho, lf - rho);
+    const float lim = tdiv(num, le + rho) + tdiv(num_d, lf + rho);
+    return tsqrt(s) + turn <= lim - 1e-4f;
+}
+
 // ---- candidate narrowing for a tile of voxels ------------------------------------------
 
 // Bounding ball of the voxel centres of the tile with first voxel (ix0, iy0,
@@ -204,6 +234,16 @@ SMG_FN void extents_in_frame(const float te[3], float cb, float sb, float rt[3])
     rt[2] = as * te[0] + ac * te[2];
 }
 
+// Intersects the interval [lo, hi] of s with c s <= r, without branches: c = 0
+// is taken as -1e-30, which leaves the interval alone when r >= 0 and empties it
+// when r < 0.
+SMG_FN void frustum_cut(float c, float r, float& lo, float& hi) {
+    const float cs = c == 0.0f ? -1e-30f : c;
+    const float t = tdiv(r, cs);
+    hi = cs > 0.0f ? tmin2(hi, t) : hi;
+    lo = cs < 0.0f ? tmax2(lo, t) : lo;
+}
+
 // Can a segment from a point of the box (q, rq) to a point of the box (tc,
 // rt) meet the box of half sizes (hx, hy, hz) centred at c and turned by beta
 // about y (cos and sin in cb, sb)?  rq and rt hold the half sizes of
@@ -227,7 +267,6 @@ SMG_FN bool box_meets_frustum(const float q[3], const float rq[3], const float t
     float b[3] = {tx * cb + tz * sb, ty, tz * cb - tx * sb};
     float h[3] = {hx, hy, hz};
     float lo = 0.0f, hi = 1.0f;
-    bool ok = true;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         float u = b[i] - a[i];
@@ -235,14 +274,10 @@ SMG_FN bool box_meets_frustum(const float q[3], const float rq[3], const float t
         float m = 2e-3f + 1e-5f * (tabs(a[i]) + tabs(b[i]) + h[i] + rt[i] + rq[i]);
         float c0 = u - dr, r0 = h[i] + m + rq[i] - a[i];   // a + s u <= h + r(s)
         float c1 = -u - dr, r1 = h[i] + m + rq[i] + a[i];  // -(a + s u) <= h + r(s)
-        if (c0 > 0.0f) hi = tmin2(hi, tdiv(r0, c0));
-        else if (c0 < 0.0f) lo = tmax2(lo, tdiv(r0, c0));
-        else ok &= r0 >= 0.0f;
-        if (c1 > 0.0f) hi = tmin2(hi, tdiv(r1, c1));
-        else if (c1 < 0.0f) lo = tmax2(lo, tdiv(r1, c1));
-        else ok &= r1 >= 0.0f;
+        frustum_cut(c0, r0, lo, hi);
+        frustum_cut(c1, r1, lo, hi);
     }
-    return ok && lo <= hi + 1e-5f;
+    return lo <= hi + 1e-5f;
 }
 
 // The same for a ball of radius rho around tc (its extent is rho in every frame).
@@ -417,6 +452,25 @@ SMG_FN bool plate_gate_clear_ball(const Layer<double>& L, const double qc[3], do
     return true;
 }
 
+// Records of one (sub-cell, candidate) pair that the narrowing keeps, shared by
+// the lanes of a wave: a bar's faces relative to the sub-cell point
+// (fast_faces), its mu_total (a float value, so exact), the position in the
+// candidate list with kFastBar set when it qualifies for fast_bar_chord, and the
+// lanes whose culling test keeps it; a hole's axis, y span, radius and mu, its
+// hole number and lanes.
+constexpr uint32_t kFastBar = 0x80000000u;
+struct BarRec {
+    float face[6];
+    float mu;
+    uint32_t tag;
+    uint64_t lanes;
+};
+struct HoleRec {
+    double xc, y1, y2, zc, r, mu;
+    uint64_t lanes;
+    uint32_t tag, hole;
+};
+
 // Sub-cell number `cell` in the reference's loop order: z outermost, then x,
 // then y (PESysMatGen.cu:1193-1197).
 SMG_FN void make_cell_ctx_linear(const Bar<double>& bd, int cell, const int sub[3], CellCtx& cc) {
@@ -562,6 +616,17 @@ SMG_FN void ray_dir(const double p[3], const double q[3], double D[3], double& d
     segdir_init<T>(sw, T(D[0]), T(D[1]), T(D[2]), tol_d, near);
 }
 
+// Whether a candidate list carries hole records (hole_rec(j)), as the GPU's
+// lists do; a list without them is traced through the hole table.
+template <class C, class = void>
+struct HasHoleRecs {
+    static constexpr bool value = false;
+};
+template <class C>
+struct HasHoleRecs<C, typename std::enable_if<C::kHoleRecs>::type> {
+    static constexpr bool value = true;
+};
+
 // Chords a caller may keep from pe_cell_ray (the adjoint's second use).
 constexpr int kKeepChords = 8;
 
@@ -666,6 +731,13 @@ SMG_FN T pe_cell_ray(const PeGeom& G, int d, const double p[3], const double ps[
         for (int j = 0; j < C.nholes(); ++j) {
             int h = C.hole(j);
             if (h < first || h >= last || !C.hole_on(j)) continue;
+            if constexpr (HasHoleRecs<Cands>::value && !kEll) {
+                const HoleRec& r = C.hole_rec(j);
+                const double l = cyl_chord<kF32>(p, cr, dd, r.xc, r.y1, r.y2, r.zc, r.r);
+                sum += l;
+                att += r.mu * l;
+                continue;
+            }
             const Hole<double>& o = G.holes_d[h];
             double l;
             if constexpr (kEll)

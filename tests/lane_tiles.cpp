@@ -113,4 +113,75 @@ int tile_extent_check(const float* coll, const float* det, const float* img, con
     return 0;
 }
 
+// n_waves seeded (bar, tile) pairs: a bar or hole that cull_keeps_all keeps for
+// the whole tile must pass the reference culling test (FP64) of every voxel of
+// the tile.  stats[0] candidates kept for all, [1] of them failing some voxel's
+// test, [2] candidates every voxel's test keeps.
+int cull_all_check(const float* coll, const float* det, const float* img, const float* phys, int rot, int tx,
+                   int ty, int tz, int n_waves, unsigned seed, double* stats) {
+    HostGeom hg;
+    std::string why;
+    if (parse_geometry(coll, det, img, phys, hg, why) != 0) return -1;
+    const GeomDesc& g = hg.g;
+    PeGeom G{};
+    G.g = g;
+    G.bars_f = hg.bars_f.data();
+    G.bars_d = hg.bars_d.data();
+    G.holes_f = hg.holes_f.data();
+    G.holes_d = hg.holes_d.data();
+    const int tile[3] = {tx, ty, tz};
+    const int nt[3] = {(g.nx + tx - 1) / tx, (g.ny + ty - 1) / ty, (g.nz + tz - 1) / tz};
+    const double phi = (double)rot * g.dphi, cphi = std::cos(phi), sphi = std::sin(phi);
+    uint64_t st = seed * 2654435761ull + 1;
+    auto next = [&]() {
+        st ^= st << 13;
+        st ^= st >> 7;
+        st ^= st << 17;
+        return st;
+    };
+    for (int i = 0; i < 3; ++i) stats[i] = 0.0;
+    for (int w = 0; w < n_waves; ++w) {
+        const int d = (int)(next() % g.n_det);
+        const int t = (int)(next() % ((uint64_t)nt[0] * nt[1] * nt[2]));
+        const int ix0 = (t % nt[0]) * tx, iy0 = ((t / nt[0]) % nt[1]) * ty, iz0 = (t / (nt[0] * nt[1])) * tz;
+        const Bar<float>& bdf = hg.bars_f[d];
+        double tc[3], rho;
+        tile_ball(g, ix0, iy0, iz0, tile, cphi, sphi, tc, rho);
+        float tcf[3], rhof;
+        tile_ball_f(tc, rho, tcf, rhof);
+        const float cd[3] = {bdf.cx, bdf.cy, bdf.cz};
+        for (int k = 0; k < g.n_det + g.n_holes; ++k) {
+            if (k == d) continue;
+            const bool is_bar = k < g.n_det;
+            float c[3], num;
+            if (is_bar) {
+                const Bar<float>& b = hg.bars_f[k];
+                c[0] = b.cx; c[1] = b.cy; c[2] = b.cz;
+                num = 0.5f * b.rdiag;
+            } else {
+                const Hole<float>& o = hg.holes_f[k - g.n_det];
+                c[0] = o.xc; c[1] = o.ymid; c[2] = o.zc;
+                num = o.crit;
+            }
+            const bool all = cull_keeps_all(tcf, rhof, c, num, cd, 0.5f * bdf.rdiag);
+            bool every = true;
+            for (int l = 0; l < tx * ty * tz; ++l) {
+                const int ix = ix0 + l % tx, iy = iy0 + (l / tx) % ty, iz = iz0 + l / (tx * ty);
+                if (ix >= g.nx || iy >= g.ny || iz >= g.nz) continue;
+                double p[3];
+                voxel_position(g, ix, iy, iz, cphi, sphi, p);
+                const float pf[3] = {float(p[0]), float(p[1]), float(p[2])}, udf[3] = {0, 0, 0};
+                SelfCull sc;
+                self_cull(hg.bars_d[d], p, sc);
+                every &= is_bar ? cull_bar<true>(G, k, p, pf, sc, udf, 0.0f)
+                                : cull_hole<true>(G, k - g.n_det, p, pf, sc, udf, 0.0f);
+            }
+            stats[0] += all;
+            stats[1] += all && !every;
+            stats[2] += every;
+        }
+    }
+    return 0;
+}
+
 }  // extern "C"

@@ -22,7 +22,29 @@ def tiles_lib():
     dp = np.ctypeslib.ndpointer(np.float64, flags="C")
     L.tile_extent_check.restype = C.c_int
     L.tile_extent_check.argtypes = [fp, fp, fp, fp, fp] + [C.c_int] * 9 + [C.c_uint, dp]
+    L.cull_all_check.restype = C.c_int
+    L.cull_all_check.argtypes = [fp, fp, fp, fp] + [C.c_int] * 5 + [C.c_uint, dp]
     return L
+
+
+@pytest.mark.parametrize("case,rot,tile", [("small", 0, (8, 8, 1)), ("volume", 3, (4, 4, 4)), ("full", 0, (4, 4, 4)),
+                                           ("turned", 1, (8, 4, 2)), ("close", 0, (8, 8, 1))])
+def test_cull_keeps_all_is_conservative(tiles_lib, params_mod, case, rot, tile):
+    """A candidate kept for a whole tile at once passes the reference culling test
+    of each of its voxels; "close": voxels of 6 mm next to the plate, where the
+    tile is large against its distance."""
+    if case == "full":
+        p = params_mod.config(2)
+    elif case == "turned":
+        p = small_geometry(params_mod, beta=0.4, nx=9, ny=9, nz=2, dphi=0.3, n_rot=3)
+    else:
+        p = params_mod.config(1)
+        dims, w = {"small": ((19, 13, 1), 1.0), "volume": ((10, 9, 7), 1.1), "close": ((9, 9, 1), 6.0)}[case]
+        params_mod.set_image(p, *dims, w, w, w, 12, 0.31)
+    st = np.zeros(3)
+    assert tiles_lib.cull_all_check(p.coll, p.det, p.img, p.phys, rot, *tile, 20, 11, st) == 0
+    print(f"{case}: {int(st[0])} of {int(st[2])} fully kept candidates found at once")
+    assert st[0] > 0 and st[1] == 0
 
 
 @pytest.mark.parametrize("case,rot,tile,sub,waves", [
