@@ -108,6 +108,10 @@ __device__ __forceinline__ uint64_t uniform_u64(uint64_t x) {
 }
 __device__ __forceinline__ bool lane_bit(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
+// Set bits of m, as a signed number: the hole records are indexed downward
+// (__popcll is unsigned, and a negated unsigned index wraps at 2^32).
+__device__ __forceinline__ int bit_count(uint64_t m) { return (int)__popcll(m); }
+
 // One sub-cell's narrowed candidates for the lanes of a wave, from its records
 // (the FP32 rays).
 template <class Lists>
@@ -212,12 +216,12 @@ __device__ __forceinline__ void append_candidates(Lists& L, int cap, int first, 
     uint64_t bal = __ballot(pass);
     const uint64_t ball = __ballot(pass && all);
     if (bal == ball) {
-        const int pos = n + __popcll(bal & ((1ull << lane) - 1ull));
+        const int pos = n + bit_count(bal & ((1ull << lane) - 1ull));
         if (pass && pos < cap) {
             L.idx[first + pos] = (uint16_t)(base + lane);
             L.arena[first + pos] = valid;
         }
-        n += __popcll(bal);
+        n += bit_count(bal);
         return;
     }
     while (bal) {
@@ -443,8 +447,8 @@ __device__ __forceinline__ void sel_count(const Lists& L, int s, int words, int 
     for (int w = 0; w < words; ++w) {
         uint64_t mb, mh;
         sel_word(L, s, words, w, nb, mb, mh);
-        kb += __popcll(mb);
-        kh += __popcll(mh);
+        kb += bit_count(mb);
+        kh += bit_count(mh);
     }
 }
 
@@ -500,10 +504,10 @@ __device__ __forceinline__ void trace_cells(const PeLaunch& A, const Bar<double>
                         uint64_t mb, mh;
                         sel_word(L, e, words, w, nb, mb, mh);
                         const uint32_t tag = ((uint32_t)e << 16) | (uint32_t)(w * 64 + lane);
-                        if (lane_bit(mb)) bars[nbr + __popcll(mb & below)].tag = tag;
-                        if (lane_bit(mh)) holes[-(nhr + __popcll(mh & below))].tag = tag;
-                        nbr += __popcll(mb);
-                        nhr += __popcll(mh);
+                        if (lane_bit(mb)) bars[nbr + bit_count(mb & below)].tag = tag;
+                        if (lane_bit(mh)) holes[-(nhr + bit_count(mh & below))].tag = tag;
+                        nbr += bit_count(mb);
+                        nhr += bit_count(mh);
                     }
                 }
                 if (e == s) {  // not even one sub-cell's: its rays go to FP64
@@ -578,10 +582,10 @@ __device__ __forceinline__ void trace_cells(const PeLaunch& A, const Bar<double>
             for (int w = 0; w < words; ++w) {
                 uint64_t mb, mh;
                 sel_word(L, s, words, w, nb, mb, mh);
-                if (lane_bit(mb)) cur[ib + __popcll(mb & below)] = (uint16_t)(w * 64 + lane);
-                if (lane_bit(mh)) cur[ih + __popcll(mh & below)] = (uint16_t)(w * 64 + lane);
-                ib += __popcll(mb);
-                ih += __popcll(mh);
+                if (lane_bit(mb)) cur[ib + bit_count(mb & below)] = (uint16_t)(w * 64 + lane);
+                if (lane_bit(mh)) cur[ih + bit_count(mh & below)] = (uint16_t)(w * 64 + lane);
+                ib += bit_count(mb);
+                ih += bit_count(mh);
             }
             __syncthreads();
             f64(cell, cc, C, W.valid && (kExact || ((L.redo[s] >> lane) & 1ull)));
