@@ -6,14 +6,14 @@
 // before its sub-cell loop (:1193-1362).  Here the 64 lanes of a wave share
 // detector d, so every sub-cell point is wave-uniform and:
 //   1. the wave scans the bars and holes once, 64 at a time, keeping those
-//      whose box a segment from bar d to the tile can meet (any other has chord 0 for every ray of the wave, so whether the
-//      reference would cull it does not change the result); each survivor is
-//      then tested with the reference culling predicate per lane and stored
-//      in LDS with the 64-bit ballot of the lanes that keep it;
-//   2. for each sub-cell, the candidates are narrowed to those whose box can
-//      meet a segment from the sub-cell centre to the tile (a
-//      bar outside that cone has chord 0 for every lane, so dropping it is
-//      exact);
+//      whose box a segment from bar d to the tile can meet (any other has
+//      chord 0 for every ray of the wave, so whether the reference would cull
+//      it does not change the result), with the lanes whose reference culling
+//      predicate keeps them, in LDS;
+//   2. for a block of sub-cells at once, the candidates are narrowed to those
+//      whose box can meet a segment from the sub-cell centre to the tile (a bar
+//      outside that cone has chord 0 for every lane, so dropping it is exact),
+//      and the records of the kept (sub-cell, candidate) pairs are formed in LDS;
 //   3. every lane traces its own ray against the narrowed lists (wave-uniform
 //      loops, per-lane masks) and accumulates the sub-cell terms with a
 //      two-sum compensated sum;
@@ -126,7 +126,7 @@ struct RecCands {
     __device__ bool fast(int j) const { return b[j].tag & kFastBar; }
     __device__ const float* faces(int j) const { return b[j].face; }
     __device__ bool has_mu(int) const { return true; }
-    __device__ float mu(int j) const { return b[j].mu; }
+    __device__ double mu(int j) const { return b[j].mu; }
     __device__ int pos(int j) const { return b[j].tag & 0xffff; }
     // the index is wave-uniform: readfirstlane lets the record loads go
     // through the scalar unit
@@ -204,6 +204,8 @@ __device__ __forceinline__ void wave_setup(const PeLaunch& A, int d, int tile, i
     const bool clear = lane < g.n_layers &&
                        plate_gate_clear_ball(G.layers_d[lane < g.n_layers ? lane : 0], qc, rb, W.tc, W.rho);
     W.bar_gate = (uint32_t)__ballot(clear);
+    if (bd.sb == 0.0 && bd.cb == 1.0) W.bar_gate |= kUnturned;
+    W.bar_gate = __builtin_amdgcn_readfirstlane(W.bar_gate);
 }
 
 // Appends the passing lanes' candidates (numbers base + lane) to the list at
@@ -353,7 +355,7 @@ __device__ __forceinline__ void tile_cell(const PeLaunch& A, const Bar<double>& 
     const GeomDesc& g = A.geom.g;
     const uint32_t all = (uint32_t)((1ull << g.n_layers) - 1ull);
     if ((W.bar_gate & all) == all) {  // wave-uniform
-        cc.gate_clear = W.bar_gate;
+        cc.gate_clear = W.bar_gate;  // with its kUnturned bit
         return;
     }
     const bool clear = lane < g.n_layers && !((W.bar_gate >> lane) & 1u) &&
@@ -380,7 +382,7 @@ __device__ __forceinline__ void cell_point(const PeLaunch& A, const Bar<double>&
 // all of them, and with at most 32 candidates a pass takes several sub-cells.
 // (One sub-cell per pass, its candidates' records gathered anew for each, was a
 // quarter of the PE kernel's instructions and most of its waits: full-size step
-// 177.4 ms, with this form 169.8 ms; 64-bar slice, one wave per SIMD, 274 -> 246 us.)
+// 177.4 ms, with this form 169.8; 64-bar slice, one wave per SIMD, 274 -> 246 us.)
 template <class Lists>
 __device__ __forceinline__ void select_cells(const PeLaunch& A, const Bar<double>& bd, int d, int my_cell, int ns,
                                              const WaveSetup& W, int lane, Lists& L, int nb, int n, int words) {
@@ -530,23 +532,25 @@ __device__ __forceinline__ void trace_cells(const PeLaunch& A, const Bar<double>
                         BarRec& r = bars[i];
 #pragma unroll
                         for (int m = 0; m < 6; ++m) r.face[m] = f[m];
-                        r.mu = G.bars_f[k].mut;
+                        r.mu = G.bars_d[k].mut;
                         r.tag = (uint32_t)j | (fast ? kFastBar : 0u);
                         r.lanes = L.arena[j];
                     }
                 }
-                for (int i = lane; i < nhr; i += 64) {
-                    HoleRec& r = holes[-i];
-                    const int j = r.tag & 0xffff, k = L.idx[j];
-                    const Hole<double>& o = G.holes_d[k];
-                    r.xc = o.xc;
-                    r.y1 = o.y1;
-                    r.y2 = o.y2;
-                    r.zc = o.zc;
-                    r.r = o.r;
-                    r.mu = o.mu;
-                    r.lanes = L.arena[j];
-                    r.hole = (uint32_t)k;
+                for (int i0 = 0; i0 < nhr; i0 += 64) {
+                    const int i = i0 + lane;
+                    const uint32_t tag = i < nhr ? holes[-i].tag : 0u;
+                    const int cell = __shfl(my_cell, (int)(tag >> 16) & 63);
+                    if (i < nhr) {
+                        const int j = tag & 0xffff, k = L.idx[j];
+                        const Hole<double>& o = G.holes_d[k];
+                        double q[3];
+                        cell_point(A, bd, d, cell, q);
+                        HoleRec& r = holes[-i];
+                        hole_rec(o, q, r);
+                        r.lanes = fabs(o.y1 - o.y2) < kCylDy ? 0ull : L.arena[j];
+                        r.hole = (uint32_t)k;
+                    }
                 }
                 __syncthreads();
                 int ib = 0, ih = 0;

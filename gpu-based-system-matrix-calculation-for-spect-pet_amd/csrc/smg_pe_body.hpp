@@ -324,11 +324,16 @@ SMG_FN T exp_neg(double x) {
     if constexpr (std::is_same<T, double>::value) {
         return exp(-x);
     } else {
-        double y = x * 1.4426950408889634;  // log2(e)
-        if (y > 200.0) return 0.0f;
-        double n = floor(y);
-        float f = (float)(y - n);
-        return ldexpf(exp2f(-f), -(int)n);
+        const double y = x * 1.4426950408889634;  // log2(e)
+        const int n = (int)y;  // towards 0; a tiny negative x leaves n = 0
+        const float f = (float)(y - (double)n);
+        // f in (-1, 1): the hardware exp2 needs no denormal handling, and a large
+        // n underflows to 0 in ldexp
+#if defined(__HIP_DEVICE_COMPILE__)
+        return ldexpf(__builtin_amdgcn_exp2f(-f), -n);
+#else
+        return ldexpf(exp2f(-f), -n);
+#endif
     }
 }
 
@@ -453,23 +458,33 @@ SMG_FN bool plate_gate_clear_ball(const Layer<double>& L, const double qc[3], do
 }
 
 // Records of one (sub-cell, candidate) pair that the narrowing keeps, shared by
-// the lanes of a wave: a bar's faces relative to the sub-cell point
-// (fast_faces), its mu_total (a float value, so exact), the position in the
-// candidate list with kFastBar set when it qualifies for fast_bar_chord, and the
-// lanes whose culling test keeps it; a hole's axis, y span, radius and mu, its
-// hole number and lanes.
+// the lanes of a wave.  Bar: its faces relative to the sub-cell point
+// (fast_faces), its mu_total, the position in the candidate list with kFastBar
+// set when it qualifies for fast_bar_chord, and the lanes whose culling test
+// keeps it.  Hole: axis and end planes relative to the sub-cell point, squared
+// radius, mu, hole number and lanes (none for a hole shorter than 0.001, whose
+// chord is 0).
 constexpr uint32_t kFastBar = 0x80000000u;
 struct BarRec {
-    float face[6];
-    float mu;
-    uint32_t tag;
+    double mu;
     uint64_t lanes;
+    float face[6];
+    uint32_t tag, pad;
 };
 struct HoleRec {
-    double xc, y1, y2, zc, r, mu;
+    double x, y1, y2, z, r2, mu;
     uint64_t lanes;
     uint32_t tag, hole;
 };
+
+SMG_FN void hole_rec(const Hole<double>& o, const double q[3], HoleRec& r) {
+    r.x = o.xc - q[0];
+    r.y1 = o.y1 - q[1];
+    r.y2 = o.y2 - q[1];
+    r.z = o.zc - q[2];
+    r.r2 = o.r * o.r;
+    r.mu = o.mu;
+}
 
 // Sub-cell number `cell` in the reference's loop order: z outermost, then x,
 // then y (PESysMatGen.cu:1193-1197).
@@ -516,11 +531,15 @@ SMG_FN T other_bar_chord(const PeGeom& G, int k, const double p[3], const double
                            tol_d, near);
         return seg_box_local(sr, of, lim_lo, lim_hi, lo, hi, near);
     } else {
-        double a[3], b[3];
-        to_frame(bk, p, a);
-        to_frame(bk, q, b);
         double lo[3] = {-0.5 * bk.w, -0.5 * bk.t, -0.5 * bk.h};
         double hi[3] = {0.5 * bk.w, 0.5 * bk.t, 0.5 * bk.h};
+        double a[3], b[3];
+        if (bk.sb == 0.0 && bk.cb == 1.0) {
+            for (int i = 0; i < 3; ++i) a[i] = p[i] - (i == 0 ? bk.cx : i == 1 ? bk.cy : bk.cz);
+            return seg_box<double>(sw, a, lo, hi, near);
+        }
+        to_frame(bk, p, a);
+        to_frame(bk, q, b);
         SegDir<double> sr;
         segdir_init<double>(sr, b[0] - a[0], b[1] - a[1], b[2] - a[2], 0.0, near);
         return seg_box<double>(sr, a, lo, hi, near);
@@ -592,13 +611,11 @@ SMG_FN bool fast_faces(const PeGeom& G, int k, const double q[3], const double t
 // (length_box_ray, PESysMatGen.cu:236-312, for a segment with no direction
 // component below eps).
 SMG_FN float fast_bar_chord(const SegDir<float>& s, const float n[6], bool& near) {
-    float t_in = -INFINITY, t_out = INFINITY, e = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const float a = -n[k] * s.inv[k], b = -n[3 + k] * s.inv[k];
-        t_in = tmax2(t_in, tmin2(a, b));
-        t_out = tmin2(t_out, tmax2(a, b));
-    }
+    const float a0 = -n[0] * s.inv[0], b0 = -n[3] * s.inv[0];
+    const float a1 = -n[1] * s.inv[1], b1 = -n[4] * s.inv[1];
+    const float a2 = -n[2] * s.inv[2], b2 = -n[5] * s.inv[2];
+    const float t_in = tmax2(tmax2(tmin2(a0, b0), tmin2(a1, b1)), tmin2(a2, b2));
+    const float t_out = tmin2(tmin2(tmax2(a0, b0), tmax2(a1, b1)), tmax2(a2, b2));
     const float chord = t_out - t_in;
     if (!(chord > 0.0f) || !(t_in > 0.0f) || !(t_in < s.len)) return 0.0f;
     const float tol = 4.0f * kUnit<float> * (tabs(t_in) + tabs(t_out)) + 1e-9f;
@@ -630,126 +647,156 @@ struct HasHoleRecs<C, typename std::enable_if<C::kHoleRecs>::type> {
 // Chords a caller may keep from pe_cell_ray (the adjoint's second use).
 constexpr int kKeepChords = 8;
 
-// kEll: the elliptical-hole chord is compiled in (the all-FP64 kernels, which
-// the library runs whenever a hole is elliptical); otherwise every hole is
-// traced as the parameter file's circle, which keeps the ellipse's code, and
-// its registers, out of the FP32 kernels.
-// tan_bar (optional): a direction over the bars' mu_total; *tan_att then
-// receives sum_k tan_bar[k] l_k over the other bars on the ray (the tangent of
-// their attenuation).
-template <class T, bool kEll, class Cands>
-SMG_FN T pe_cell_ray(const PeGeom& G, int d, const double p[3], const double ps[3],
-                     const CellCtx& cc, const Cands& C, bool& near, double* dl_layer = nullptr,
-                     double* aux = nullptr, float* keep = nullptr, int keep_stride = 0,
-                     const double* tan_bar = nullptr, double* tan_att = nullptr) {
+// Set in CellCtx::gate_clear, beside the layers' bits, by a caller that knows
+// bar d is unturned (beta = 0): the ray's direction in its frame is then the
+// world direction.
+constexpr uint32_t kUnturned = 0x80000000u;
+
+// Chord through the hole of record h for the ray that ends at the sub-cell
+// point (cyl_chord with every position relative to that point and the ray
+// parameter t - len): kx, kz the unit direction, rdy = 1 / D_y, sxk, szk = D_x,
+// D_z / D_y, inv_ky = len / D_y.
+SMG_FN double cyl_chord_rec(const HoleRec& h, const double D[3], double inv_dd, double len, double sxk,
+                            double szk, double inv_ky) {
+    const double xl = sxk * h.y1 - h.x, zl = szk * h.y1 - h.z;
+    const double xr = sxk * h.y2 - h.x, zr = szk * h.y2 - h.z;
+    const double t_lo = h.y1 * inv_ky, t_hi = h.y2 * inv_ky, t0 = kCylT - len;
+    const bool in_l = xl * xl + zl * zl <= h.r2, in_r = xr * xr + zr * zr <= h.r2;
+    double ta = t_lo, tb = t_hi;
+    if (!(in_l && in_r)) {
+        const double kx = D[0] * inv_dd, kz = D[2] * inv_dd;
+        const double qa = kx * kx + kz * kz, cr = kz * h.x - kx * h.z;
+        const double disc = qa * h.r2 - cr * cr;
+        if (disc <= kCylDisc) return 0.0;
+        const double sq = disc * rsq_fast(disc), qb = kx * h.x + kz * h.z, inv_qa = rcp_fast(qa);
+        const double t1 = (qb - sq) * inv_qa, t2 = (qb + sq) * inv_qa;
+        if (!in_l && !in_r && !(t1 >= t_lo && t2 <= t_hi)) return 0.0;
+        ta = in_l ? t_lo : t1;
+        tb = in_r ? t_hi : t2;
+    }
+    if (ta <= t0 || tb <= t0 || ta >= 0.0 || tb >= 0.0) return 0.0;
+    return fabs(tb - ta);
+}
+
+// Quantities of one ray that the adjoint, the tangent and the point weights need.
+SMG_FN void ray_aux(double aux[8], double eff, double om, double l1, double l2, double la, double ea, double dsq) {
+    aux[0] = eff * om;  // Omega e^-att
+    aux[1] = l1 - l2;   // own-bar path
+    aux[2] = la;        // absorption chord
+    aux[3] = ea;
+    aux[4] = l2;        // the sub-cell's own chord
+    aux[5] = eff;       // e^-att
+    aux[6] = dsq;       // |q - p|^2
+}
+
+// One FP32 ray (FP64: directions, lengths, plate and hole paths, attenuation
+// sums).  What the reference's branches for direction components below eps
+// change is either nothing here (the own bar, see below) or flagged: a lane with
+// such a component and another bar on its list, or nearly parallel to the
+// plates.  The kernels are bound by this function's vector instructions: one
+// FP64 reciprocal square root gives the length, the solid angle and the unit
+// direction, an unturned bar's own chords take the world direction data, and
+// holes are met in coordinates relative to the sub-cell point (with direction
+// data per frame, per-axis eps flags and absolute hole coordinates the full-size
+// PE step took 169.8 ms instead of 131.3, a slice at 8x16x8 sub-cells 30.1
+// instead of 22.7).
+template <bool kEll, class Cands>
+SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const double ps[3], const CellCtx& cc,
+                             const Cands& C, bool& near, double* dl_layer, double* aux, float* keep,
+                             int keep_stride, const double* tan_bar, double* tan_att) {
     const GeomDesc& g = G.g;
     const Bar<double>& bd = G.bars_d[d];
-    constexpr bool kF32 = std::is_same<T, float>::value;
-    double D[3] = {cc.q[0] - p[0], cc.q[1] - p[1], cc.q[2] - p[2]};
-    double dsq = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
-    // FP64 path: |D| and cos(alpha) as the reference forms them; the FP32
-    // path takes |D| and 1/|D| from a refined hardware reciprocal square root
-    // below, where the hole and bar chords need them
-    double dd = 0.0, inv_dd = 0.0, cosang = 0.0;
-    if constexpr (!kF32) {
-        dd = sqrt(dsq);
-        inv_dd = 1.0 / dd;
-        cosang = D[1] / dd;
+    const bool unturned = cc.gate_clear & kUnturned;  // wave-uniform
+    const double D[3] = {cc.q[0] - p[0], cc.q[1] - p[1], cc.q[2] - p[2]};
+    const double dsq = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
+    const double inv_dd = rsq_fast(dsq), dd = dsq * inv_dd;
+    SegDir<float> sw;
+    sw.ns = 0;
+    sw.len = float(dd);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        sw.D[k] = float(D[k]);
+        sw.inv[k] = sw.len * trcp(sw.D[k]);
+        sw.small[k] = 0;
+    }
+    sw.tol_d = 12.0f * kUnit<float> * sw.len;  // rounding of a component of D
+    const float dmin = tmin2(tmin2(tabs(sw.D[0]), tabs(sw.D[1])), tabs(sw.D[2]));
+    const bool thin = dmin < kSlabEps<float> + sw.tol_d;
+    const bool flat = tabs(sw.D[1]) < kSlabEps<float> + sw.tol_d;
+    near |= flat;
+    const double dy = flat ? 1.0 : D[1];
+
+    // direction in the frame of bar d
+    float Db[3] = {sw.D[0], sw.D[1], sw.D[2]}, ib[3] = {tabs(sw.inv[0]), tabs(sw.inv[1]), tabs(sw.inv[2])};
+    if (!unturned) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            Db[k] = float(cc.qs[k] - ps[k]);
+            ib[k] = tabs(sw.len * trcp(Db[k]));
+        }
     }
 
-    // solid angle: largest of the three projected cell faces (PESysMatGen.cu:1223-1231)
-    T om;
-    if constexpr (std::is_same<T, double>::value) {
-        const double cb = bd.cb, sb = bd.sb, four_pi = 4.0 * 3.14159265358979323846;
-        double omx = cc.area[0] / (four_pi * dsq) * tabs(D[0] * cb - D[2] * sb) / dd;
-        double omz = cc.area[2] / (four_pi * dsq) * tabs(D[0] * sb + D[2] * cb) / dd;
-        double omy = cc.area[1] / (four_pi * dsq) * tabs(D[1]) / dd;
-        om = tmax2(tmax2(omx, omy), omz);
-    } else {
-        // one reciprocal of 4 pi |D|^3 for the three faces
-        const float cb = float(bd.cb), sb = float(bd.sb);
-        const float Dx = float(D[0]), Dy = float(D[1]), Dz = float(D[2]);
-        const float dsqf = float(dsq);
-        const float r = trcp(float(4.0 * 3.14159265358979323846) * dsqf * tsqrt(dsqf));
-        float omx = float(cc.area[0]) * tabs(Dx * cb - Dz * sb);
-        float omz = float(cc.area[2]) * tabs(Dx * sb + Dz * cb);
-        float omy = float(cc.area[1]) * tabs(Dy);
-        om = tmax2(tmax2(omx, omy), omz) * r;
-    }
+    // solid angle: largest of the three projected cell faces over 4 pi |D|^3
+    // (PESysMatGen.cu:1223-1231)
+    const float om = tmax2(tmax2(float(cc.area[0]) * tabs(Db[0]), float(cc.area[1]) * tabs(Db[1])),
+                           float(cc.area[2]) * tabs(Db[2])) *
+                     (float(inv_dd * inv_dd * inv_dd) * float(1.0 / (4.0 * 3.14159265358979323846)));
 
     double att = 0.0;
-    // world-frame direction data, shared by the plates and unrotated bars
-    SegDir<T> sw;
-    T tol_d = T(4) * kUnit<T> * (tabs(T(D[0])) + tabs(T(D[1])) + tabs(T(D[2])));
-    segdir_init<T>(sw, T(D[0]), T(D[1]), T(D[2]), tol_d, near);
-    const T pw[3] = {T(p[0]), T(p[1]), T(p[2])};
-
     // plate gate: a ray that does not cross a plate is blocked (PESysMatGen.cu:1240-1254)
-    for (int m = 0; m < g.n_layers; ++m) {
-        if ((cc.gate_clear >> m) & 1u) continue;
-        T lo[3], hi[3];
-        if constexpr (std::is_same<T, float>::value) {
+    const uint32_t all = (uint32_t)((1ull << g.n_layers) - 1ull);
+    if ((cc.gate_clear & all) != all) {  // wave-uniform
+        SegDir<float> sg;
+        const float tol_d = 4.0f * kUnit<float> * (tabs(sw.D[0]) + tabs(sw.D[1]) + tabs(sw.D[2]));
+        segdir_init<float>(sg, sw.D[0], sw.D[1], sw.D[2], tol_d, near);
+        const float pw[3] = {float(p[0]), float(p[1]), float(p[2])};
+        for (int m = 0; m < g.n_layers; ++m) {
+            if ((cc.gate_clear >> m) & 1u) continue;
             const Layer<float>& L = G.layers_f[m];
-            for (int k = 0; k < 3; ++k) {
-                lo[k] = L.lo[k];
-                hi[k] = L.hi[k];
-            }
-        } else {
-            const Layer<double>& L = G.layers_d[m];
-            for (int k = 0; k < 3; ++k) {
-                lo[k] = L.lo[k];
-                hi[k] = L.hi[k];
-            }
+            const float l = seg_box<float>(sg, pw, L.lo, L.hi, near);
+            if (g_lt(l, 0.1f, 1e-4f, near)) att += 100000.0;
         }
-        T l = seg_box<T>(sw, pw, lo, hi, near);
-        if (g_lt(l, T(0.1f), T(1e-4), near)) att += 100000.0;
     }
 
-    // holes and plate material, FP64 (PESysMatGen.cu:1257-1286).  The FP32
-    // path forms T / cos(alpha) as T |D| / D_y and the hole-ray set-up from
-    // the same two reciprocals, only when the sub-cell has hole candidates.
-    CylRay cr;
-    double inv_cos;
-    if constexpr (std::is_same<T, double>::value) {
-        cyl_ray(D, dd, cr);
-        inv_cos = 0.0;
-    } else {
-        inv_dd = rsq_fast(dsq);
-        dd = dsq * inv_dd;
-        inv_cos = tabs(D[1]) > 1e-300 ? dd * rcp_fast(D[1]) : dd / D[1];
-        if (C.nholes() > 0) cyl_ray_from(D, inv_dd, inv_cos, cr);
-    }
+    // holes and plate material, FP64 (PESysMatGen.cu:1257-1286); T / cos(alpha)
+    // is T |D| / D_y
+    const double rdy = rcp_fast(dy), inv_ky = dd * rdy;
+    const double sxk = D[0] * rdy, szk = D[2] * rdy;
     for (int m = 0; m < g.n_layers; ++m) {
         const Layer<double>& L = G.layers_d[m];
-        int first = g.ranges[m].first, last = first + g.ranges[m].count;
-        double in_coll;
-        if constexpr (std::is_same<T, double>::value)
-            in_coll = L.thick / cosang;
-        else
-            in_coll = L.thick * inv_cos;
+        const int first = g.ranges[m].first, last = first + g.ranges[m].count;
+        const double in_coll = L.thick * inv_ky;
         double sum = 0.0;
         for (int j = 0; j < C.nholes(); ++j) {
-            int h = C.hole(j);
+            const int h = C.hole(j);
             if (h < first || h >= last || !C.hole_on(j)) continue;
-            if constexpr (HasHoleRecs<Cands>::value && !kEll) {
+            double l, mu;
+            if constexpr (kEll) {
+                const Hole<double>& o = G.holes_d[h];
+                mu = o.mu;
+                if (o.erx > 0.0) {
+                    l = ell_chord(o, p[0], p[1], p[2], D[0] * inv_dd, D[2] * inv_dd, inv_ky, dd);
+                } else {
+                    HoleRec r;
+                    hole_rec(o, cc.q, r);
+                    l = fabs(o.y1 - o.y2) < kCylDy ? 0.0 : cyl_chord_rec(r, D, inv_dd, dd, sxk, szk, inv_ky);
+                }
+            } else if constexpr (HasHoleRecs<Cands>::value) {
                 const HoleRec& r = C.hole_rec(j);
-                const double l = cyl_chord<kF32>(p, cr, dd, r.xc, r.y1, r.y2, r.zc, r.r);
-                sum += l;
-                att += r.mu * l;
-                continue;
+                mu = r.mu;
+                l = cyl_chord_rec(r, D, inv_dd, dd, sxk, szk, inv_ky);
+            } else {
+                const Hole<double>& o = G.holes_d[h];
+                HoleRec r;
+                hole_rec(o, cc.q, r);
+                mu = o.mu;
+                l = fabs(o.y1 - o.y2) < kCylDy ? 0.0 : cyl_chord_rec(r, D, inv_dd, dd, sxk, szk, inv_ky);
             }
-            const Hole<double>& o = G.holes_d[h];
-            double l;
-            if constexpr (kEll)
-                l = o.erx > 0.0 ? ell_chord(o, p[0], p[1], p[2], cr.kx, cr.kz, cr.inv_ky, dd)
-                                : cyl_chord(p, cr, dd, o.xc, o.y1, o.y2, o.zc, o.r);
-            else
-                l = cyl_chord<kF32>(p, cr, dd, o.xc, o.y1, o.y2, o.zc, o.r);
             sum += l;
-            att += o.mu * l;
+            att += mu * l;
         }
-        double rest = in_coll - sum;
-        bool counted = rest >= (double)0.00001f;
+        const double rest = in_coll - sum;
+        const bool counted = rest >= (double)0.00001f;
         if (counted) att += L.mu * rest;
         if (dl_layer) store_at<kMaxLayers>(dl_layer, m, counted ? rest : 0.0);
     }
@@ -762,102 +809,186 @@ SMG_FN T pe_cell_ray(const PeGeom& G, int d, const double p[3], const double ps[
             if (keep && j < kKeepChords) keep[j * keep_stride] = 0.0f;
             continue;
         }
-        T l;
+        near |= thin;
+        float l;
         double mu_k;
-        if constexpr (Cands::kFastFaces && std::is_same<T, float>::value) {
-            // the first narrowed bars carry their mu_total in the lists: a
-            // fast chord then reads no bar record
-            if (C.has_mu(j)) {
+        bool fast = false;
+        if constexpr (Cands::kFastFaces) fast = C.fast(j);
+        if (fast) {
+            if constexpr (Cands::kFastFaces) {
                 mu_k = double(C.mu(j));
-                if (sw.ns == 0 && C.fast(j))
-                    l = fast_bar_chord(sw, C.faces(j), near);
-                else
-                    l = other_bar_chord<T>(G, C.bar(j), p, D, dd, inv_dd, cc.q, sw, tol_d, near);
-            } else {
-                const int k = C.bar(j);
-                mu_k = G.bars_d[k].mut;
-                l = other_bar_chord<T>(G, k, p, D, dd, inv_dd, cc.q, sw, tol_d, near);
+                l = fast_bar_chord(sw, C.faces(j), near);
             }
         } else {
             const int k = C.bar(j);
             mu_k = G.bars_d[k].mut;
-            l = other_bar_chord<T>(G, k, p, D, dd, inv_dd, cc.q, sw, tol_d, near);
+            l = other_bar_chord<float>(G, k, p, D, dd, inv_dd, cc.q, sw, sw.tol_d, near);
         }
-        if (keep && j < kKeepChords) keep[j * keep_stride] = float(l);
+        if (keep && j < kKeepChords) keep[j * keep_stride] = l;
         att += double(l) * mu_k;
         if (tan_bar) *tan_att += double(l) * tan_bar[C.bar(j)];
     }
 
     // own bar from its surface to the sub-cell (PESysMatGen.cu:1329-1346), and the
-    // absorption chord along the ray extended 1000 mm (PESysMatGen.cu:1350-1357)
-    double Ds[3] = {cc.qs[0] - ps[0], cc.qs[1] - ps[1], cc.qs[2] - ps[2]};
-    T l1, l2, la;
-    if constexpr (std::is_same<T, float>::value) {
-        // The sub-cell centre q lies inside bar d and is the centre of its
-        // sub-cell, and the voxel lies outside bar d.  Then the reference's
-        // chords (PESysMatGen.cu:1329-1357) reduce to distances from q:
-        //   l1 = len - t_entry(bar)  = min_k dist_k(q to the bar face on the voxel's side) / |u_k|
-        //   l2 = len - t_entry(cell) = min_k hc_k / |u_k|
-        //   la = t_exit - t_entry of the extended ray through the cell = 2 l2
-        // with u the unit direction over the axes whose component is not below
-        // eps (the reference's one- and two-small-component branches,
-        // PESysMatGen.cu:333-434, drop those axes; the premises put the start
-        // strictly inside their faces, as the branches require); no
-        // difference of two ray parameters is formed.  Rays outside the
-        // premises (all components below eps, |D_y| near 0.001, the voxel
-        // within 0.01 of bar d along the ray, sub-cells below 0.01) are
-        // flagged for the FP64 path, which keeps the reference's general form.
-        const Bar<float>& bf = G.bars_f[d];
-        SegDir<float> ss;
-        float tds = 4.0f * kUnit<float> * (tabs(float(Ds[0])) + tabs(float(Ds[1])) + tabs(float(Ds[2])));
-        segdir_init<float>(ss, float(Ds[0]), float(Ds[1]), float(Ds[2]), tds, near);
-        near |= ss.ns == 3;
-        const float hb[3] = {0.5f * bf.w, 0.5f * bf.t, 0.5f * bf.h};
-        float d1 = INFINITY, d2 = INFINITY;
+    // absorption chord along the ray extended 1000 mm (PESysMatGen.cu:1350-1357).
+    // The sub-cell centre q lies inside bar d and is the centre of its
+    // sub-cell, and the voxel lies outside bar d.  Then the reference's
+    // chords (PESysMatGen.cu:1329-1357) reduce to distances from q:
+    //   l1 = len - t_entry(bar)  = min_k dist_k(q to the bar face on the voxel's side) / |u_k|
+    //   l2 = len - t_entry(cell) = min_k hc_k / |u_k|
+    //   la = t_exit - t_entry of the extended ray through the cell = 2 l2
+    // with u the unit direction; no difference of two ray parameters is formed.
+    // The reference's one- and two-small-component branches
+    // (PESysMatGen.cu:333-434) drop an axis whose component is below eps and
+    // its share (below 1e-9) of the length: such an axis has 1 / |u_k| above
+    // 1000 len, so it never gives the minimum here.  Rays outside the premises
+    // (|D_y| near 0.001, the voxel within 0.01 of bar d along the ray,
+    // sub-cells below 0.01) are flagged for the FP64 path, which keeps the
+    // reference's general form.
+    const Bar<float>& bf = G.bars_f[d];
+    const float hb[3] = {0.5f * bf.w, 0.5f * bf.t, 0.5f * bf.h};
+    float d1 = INFINITY, d2 = INFINITY;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            if (ss.small[k]) continue;
-            const float ia = tabs(ss.inv[k]);  // 1 / |u_k|
-            const float qk = float(cc.qs[k]);
-            const float face = ss.D[k] > 0.0f ? qk + hb[k] : hb[k] - qk;
-            d1 = tmin2(d1, face * ia);
-            d2 = tmin2(d2, cc.hc[k] * ia);
+    for (int k = 0; k < 3; ++k) {
+        const float qk = float(cc.qs[k]);
+        const float face = Db[k] > 0.0f ? qk + hb[k] : hb[k] - qk;
+        d1 = tmin2(d1, face * ib[k]);
+        d2 = tmin2(d2, cc.hc[k] * ib[k]);
+    }
+    near |= (sw.len - d1 < 0.01f) | (d2 < 0.01f);
+    const float la = 2.0f * d2;
+    att += (double(d1) - double(d2)) * bd.mut;
+    const float eff = exp_neg<float>(att);
+    const float ea = exp_neg<float>(double(la) * bd.mut);
+    const float absf = (1.0f - ea) * float(bd.pe_frac);
+    if (aux) ray_aux(aux, eff, om, d1, d2, la, ea, dsq);
+    return eff * om * absf;
+}
+
+// One FP64 ray, the reference's form.  The direction data (|D|, the components
+// below eps, len / D_k) serve every box in the world's orientation: the unturned
+// bars, and bar d when it is one; a turned bar gets its own.  Bound by the FP64
+// divisions and roots (about 11 instructions each): sharing them took a turned
+// 286-bar panel from 2.02 to 1.75 ms.
+template <bool kEll, class Cands>
+SMG_FN double pe_cell_ray_f64(const PeGeom& G, int d, const double p[3], const double ps[3], const CellCtx& cc,
+                              const Cands& C, double* dl_layer, double* aux, const double* tan_bar,
+                              double* tan_att) {
+    const GeomDesc& g = G.g;
+    const Bar<double>& bd = G.bars_d[d];
+    bool near = false;
+    const double D[3] = {cc.q[0] - p[0], cc.q[1] - p[1], cc.q[2] - p[2]};
+    const double dsq = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
+    const double dd = sqrt(dsq), inv_dd = 1.0 / dd;
+
+    // solid angle: largest of the three projected cell faces (PESysMatGen.cu:1223-1231)
+    const double cb = bd.cb, sb = bd.sb;
+    const double om = tmax2(tmax2(cc.area[0] * tabs(D[0] * cb - D[2] * sb), cc.area[1] * tabs(D[1])),
+                            cc.area[2] * tabs(D[0] * sb + D[2] * cb)) *
+                      (inv_dd * inv_dd * inv_dd * (1.0 / (4.0 * 3.14159265358979323846)));
+
+    double att = 0.0;
+    SegDir<double> sw;
+    segdir_init<double>(sw, D[0], D[1], D[2], 0.0, near);
+
+    // plate gate: a ray that does not cross a plate is blocked (PESysMatGen.cu:1240-1254)
+    for (int m = 0; m < g.n_layers; ++m) {
+        if ((cc.gate_clear >> m) & 1u) continue;
+        const Layer<double>& L = G.layers_d[m];
+        const double l = seg_box<double>(sw, p, L.lo, L.hi, near);
+        if (l < (double)0.1f) att += 100000.0;
+    }
+
+    // holes and plate material (PESysMatGen.cu:1257-1286)
+    CylRay cr;
+    cr.kx = D[0] * inv_dd;
+    cr.ky = D[1] * inv_dd;
+    cr.kz = D[2] * inv_dd;
+    cr.inv_ky = dd / D[1];
+    cr.sxk = cr.kx * cr.inv_ky;
+    cr.szk = cr.kz * cr.inv_ky;
+    cr.qa = cr.kx * cr.kx + cr.kz * cr.kz;
+    cr.inv_qa = C.nholes() > 0 ? 1.0 / cr.qa : 0.0;
+    for (int m = 0; m < g.n_layers; ++m) {
+        const Layer<double>& L = G.layers_d[m];
+        const int first = g.ranges[m].first, last = first + g.ranges[m].count;
+        const double in_coll = L.thick * cr.inv_ky;
+        double sum = 0.0;
+        for (int j = 0; j < C.nholes(); ++j) {
+            const int h = C.hole(j);
+            if (h < first || h >= last || !C.hole_on(j)) continue;
+            const Hole<double>& o = G.holes_d[h];
+            double l;
+            if constexpr (kEll)
+                l = o.erx > 0.0 ? ell_chord(o, p[0], p[1], p[2], cr.kx, cr.kz, cr.inv_ky, dd)
+                                : cyl_chord(p, cr, dd, o.xc, o.y1, o.y2, o.zc, o.r);
+            else
+                l = cyl_chord(p, cr, dd, o.xc, o.y1, o.y2, o.zc, o.r);
+            sum += l;
+            att += o.mu * l;
         }
-        const bool flat = g_lt(tabs(ss.D[1]), float(kInsideDy), ss.tol_d, near);
-        near |= (ss.len - d1 < 0.01f) | (d2 < 0.01f);
-        l1 = flat ? 0.0f : d1;
-        l2 = flat ? 0.0f : d2;
-        la = 2.0f * d2;
+        const double rest = in_coll - sum;
+        const bool counted = rest >= (double)0.00001f;
+        if (counted) att += L.mu * rest;
+        if (dl_layer) store_at<kMaxLayers>(dl_layer, m, counted ? rest : 0.0);
+    }
+
+    // other bars on the way (PESysMatGen.cu:1290-1325)
+    for (int j = 0; j < C.nbars(); ++j) {
+        if (!C.bar_on(j)) continue;
+        const int k = C.bar(j);
+        const double l = other_bar_chord<double>(G, k, p, D, dd, inv_dd, cc.q, sw, 0.0, near);
+        att += l * G.bars_d[k].mut;
+        if (tan_bar) *tan_att += l * tan_bar[k];
+    }
+
+    // own bar from its surface to the sub-cell (PESysMatGen.cu:1329-1346), and the
+    // absorption chord along the ray extended 1000 mm (PESysMatGen.cu:1350-1357):
+    // the extension leaves len / D_k, and so the slab parameters, as they are
+    SegDir<double> ss = sw;
+    if (!(bd.sb == 0.0 && bd.cb == 1.0))
+        segdir_init<double>(ss, cc.qs[0] - ps[0], cc.qs[1] - ps[1], cc.qs[2] - ps[2], 0.0, near);
+    const double blo[3] = {-bd.w / 2.0, -bd.t / 2.0, -bd.h / 2.0};
+    const double bhi[3] = {bd.w / 2.0, bd.t / 2.0, bd.h / 2.0};
+    const double l1 = seg_box_inside<double>(ss, ps, blo, bhi, near);
+    const double l2 = seg_box_inside<double>(ss, ps, cc.lo, cc.hi, near);
+    double la;
+    if (ss.ns == 0) {
+        double tmin, tmax, e0, e1;
+        slab(ss, ps, cc.lo, cc.hi, tmin, tmax, e0, e1);
+        const double eps = kSlabEps<double>, end = ss.len + 1000.0;
+        const bool hit = tmax - tmin >= eps && tmin < end && tmax < end && tmin > eps && tmax > eps;
+        la = hit ? tmax - tmin : 0.0;
     } else {
-        double ext[3], De[3];
-        for (int k = 0; k < 3; ++k) {
-            ext[k] = cc.qs[k] + 1000.0 * (cc.qs[k] - ps[k]) / dd;
-            De[k] = ext[k] - ps[k];
-        }
-        double blo[3] = {-bd.w / 2.0, -bd.t / 2.0, -bd.h / 2.0};
-        double bhi[3] = {bd.w / 2.0, bd.t / 2.0, bd.h / 2.0};
-        SegDir<double> ss, se;
-        segdir_init<double>(ss, Ds[0], Ds[1], Ds[2], 0.0, near);
-        l1 = seg_box_inside<double>(ss, ps, blo, bhi, near);
-        l2 = seg_box_inside<double>(ss, ps, cc.lo, cc.hi, near);
+        double De[3];
+        for (int k = 0; k < 3; ++k) De[k] = (cc.qs[k] + 1000.0 * (cc.qs[k] - ps[k]) / dd) - ps[k];
+        SegDir<double> se;
         segdir_init<double>(se, De[0], De[1], De[2], 0.0, near);
         la = seg_box<double>(se, ps, cc.lo, cc.hi, near);
     }
-    att += (double(l1) - double(l2)) * bd.mut;
-    T eff = exp_neg<T>(att);
-    T mut = T(bd.mut), mupe = T(bd.mupe);
-    T ea = exp_neg<T>(double(la) * bd.mut);
-    T absf = (T(1) - ea) * T(bd.pe_frac);
-    if (aux) {  // quantities the adjoint needs
-        aux[0] = double(eff) * double(om);  // Omega e^-att
-        aux[1] = double(l1) - double(l2);   // own-bar path
-        aux[2] = double(la);                // absorption chord
-        aux[3] = double(ea);
-        aux[4] = double(l2);                // the sub-cell's own chord
-        aux[5] = double(eff);               // e^-att
-        aux[6] = dsq;                       // |q - p|^2
-    }
+    att += (l1 - l2) * bd.mut;
+    const double eff = exp_neg<double>(att), ea = exp_neg<double>(la * bd.mut);
+    const double absf = (1.0 - ea) * bd.pe_frac;
+    if (aux) ray_aux(aux, eff, om, l1, l2, la, ea, dsq);
     return eff * om * absf;
+}
+
+// kEll: the elliptical-hole chord is compiled in (the all-FP64 kernels, which
+// the library runs whenever a hole is elliptical); otherwise every hole is
+// traced as the parameter file's circle, which keeps the ellipse's code, and
+// its registers, out of the FP32 kernels.
+// tan_bar (optional): a direction over the bars' mu_total; *tan_att then
+// receives sum_k tan_bar[k] l_k over the other bars on the ray (the tangent of
+// their attenuation).
+template <class T, bool kEll, class Cands>
+SMG_FN T pe_cell_ray(const PeGeom& G, int d, const double p[3], const double ps[3],
+                     const CellCtx& cc, const Cands& C, bool& near, double* dl_layer = nullptr,
+                     double* aux = nullptr, float* keep = nullptr, int keep_stride = 0,
+                     const double* tan_bar = nullptr, double* tan_att = nullptr) {
+    if constexpr (std::is_same<T, float>::value)
+        return pe_cell_ray_f32<kEll>(G, d, p, ps, cc, C, near, dl_layer, aux, keep, keep_stride, tan_bar, tan_att);
+    else
+        return pe_cell_ray_f64<kEll>(G, d, p, ps, cc, C, dl_layer, aux, tan_bar, tan_att);
 }
 
 }  // namespace smg
