@@ -95,7 +95,7 @@ struct smg_ctx {
     DevBuf<Sphere<double>> hsph_d;
     DevBuf<ScatterPt<double>> pts_bar;   // bar centres (crystal scatter)
     DevBuf<ScatterPt<double>> pts_hole;  // layer-0 hole centres (collimator scatter)
-    DevBuf<PairTerm> pair;
+    DevBuf<PairRec> pair;
     DevBuf<double> sc_partial;   // per-slice scatter sums
     DevBuf<double> sc_row_cut;   // energy-window cut per output row of a scatter launch
     DevBuf<double> proj;         // projection partial sums

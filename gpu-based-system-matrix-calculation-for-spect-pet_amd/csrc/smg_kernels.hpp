@@ -148,7 +148,7 @@ struct ScatterLaunch {
     int variant;                     // collimator: 0 combined (r = 0.1), 1 standalone (r = 0.2)
     const float* pe;                 // crystal: PE block [N][V]
     const uint32_t* bitmap;          // crystal or collimator bitmap
-    PairTerm* pair;                  // [N][n_pts][cells]
+    PairRec* pair;                   // [N][n_pts][cells]
     float* dst;                      // [N][V]
     unsigned long long* counters;    // [0] FP64 fallback terms
     double cphi, sphi;

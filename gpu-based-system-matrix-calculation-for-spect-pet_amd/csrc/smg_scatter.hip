@@ -99,8 +99,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
     // the bar holding the scatter point (crystal scatter)
     const int sbar = A.kind == 3 ? A.pt_bar0 + s / A.pts_per_bar : s;
     PairTerm out{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    PairRec& rec = A.pair[tid];
     if ((A.kind == 0 || A.kind == 3) && sbar == d) {
-        A.pair[tid] = out;
+        rec.t = out;
         return;
     }
     const Bar<double>& bd = G.bars_d[d];
@@ -110,7 +111,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
     const ScatterPt<double>& sp = A.pts_d[s];
     double qs[3] = {sp.x, sp.y, sp.z};
     if (below_window_all(A, A.row_cut[r], qs, cc.q)) {  // never read: every voxel's term is below
-        A.pair[tid] = out;                    // the window (scatter_kernel tests first)
+        rec.t = out;                          // the window (scatter_kernel tests first)
         return;
     }
     bool near = false;
@@ -201,7 +202,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
     SegDir<double> se;
     segdir_init<double>(se, De[0], De[1], De[2], 0.0, near);
     out.la = seg_box<double>(se, qss, cc.lo, cc.hi, near);
-    A.pair[tid] = out;
+    rec.t = out;
+    for (int k = 0; k < 8; ++k) rec.ic[k] = inv_corner(cc.lo, cc.hi, qss, k);
 }
 
 // Waves per element row: the scatter points split into `slices` ranges, each
@@ -426,7 +428,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void sc
                     sk.qs[1] = sp.y;
                     sk.qs[2] = sp.z;
                     to_frame(bd, sk.qs, sk.qss);
-                    sk.pt = A.pair[((int64_t)r * A.n_pts + si) * ncell + cell];
+                    const PairRec& rec = A.pair[((int64_t)r * A.n_pts + si) * ncell + cell];
+                    sk.pt = rec.t;
+                    sk.ic = rec.ic;
                     const T wgt = weight(si, v0 + o, po);
                     T val = T(0);
                     if (wgt != T(0)) {
