@@ -98,8 +98,10 @@ struct smg_ctx {
     DevBuf<PairRec> pair;
     DevBuf<double> sc_partial;   // per-slice scatter sums
     DevBuf<double> sc_row_cut;   // energy-window cut per output row of a scatter launch
+    DevBuf<WinRow> sc_win_rows;  // and the rows' window tables (FP32 launches)
+    DevBuf<float> sc_win_tab;
     DevBuf<double> proj;         // projection partial sums
-    DevBuf<double> kn_tab;       // KN prefix table of kn_tab_e0
+    DevBuf<double> kn_tab;       // KN prefix polynomials of kn_tab_e0
     double kn_tab_e0 = -1.0;
     DevBuf<CellCtx> cell_tab;    // PE sub-cell table of every bar
     DevBuf<CellCtx> cell_tab_pts;  // sub-cell table of one chunk of crystal grid points
@@ -329,12 +331,12 @@ smg_status load_bitmap(smg_ctx* c, bool collimator, const uint32_t* words, int64
     return SMG_OK;
 }
 
-// KN prefix table for the FP32 scatter term at the launch's E0 (built on the
+// KN prefix polynomials of the scatter term at the launch's E0 (built on the
 // context's stream when E0 changes).
 hipError_t kn_table(smg_ctx* c, ScatterLaunch& A) {
     if (c->kn_tab_e0 != A.e0) {
         c->kn_tab_e0 = -1.0;
-        hipError_t e = c->kn_tab.reserve((size_t)(kKnPhase + 1) * kKnSteps);
+        hipError_t e = c->kn_tab.reserve((size_t)kKnPolySize);
         if (e != hipSuccess) return e;
         e = launch_kn_table(A.e0, c->kn_tab.ptr, c->stream);
         if (e != hipSuccess) return e;
@@ -344,14 +346,45 @@ hipError_t kn_table(smg_ctx* c, ScatterLaunch& A) {
     return hipSuccess;
 }
 
-// Energy-window cut of each output row of a scatter launch (A.row_cut), on
-// the context's stream ahead of the pair terms and scatter kernels.
-hipError_t scatter_row_cuts(smg_ctx* c, ScatterLaunch& A) {
+// Energy-window cut of each output row of a scatter launch (A.row_cut) and, for
+// FP32 launches, the rows' window tables (A.win_rows, A.win_tab) with as many
+// intervals as the sharpest row needs, on the context's stream ahead of the pair
+// terms and scatter kernels.  rows_h: the launch's rows on the host, or all bars.
+hipError_t scatter_row_cuts(smg_ctx* c, ScatterLaunch& A, bool exact, const int* rows_h) {
     const size_t rows = (size_t)(A.rows ? A.n_rows : A.geom.g.n_det);
     hipError_t e = c->sc_row_cut.reserve(rows > 0 ? rows : 1);
     if (e != hipSuccess) return e;
     A.row_cut = c->sc_row_cut.ptr;
-    return launch_row_cuts(A, c->sc_row_cut.ptr, c->stream);
+    A.win_n = 0;
+    if (!exact && rows > 0) {
+        // a row's table depends on its resolution only; the sharpest row (and,
+        // with windows relative to the resolution, the widest) sets the intervals
+        double lo = INFINITY, hi = 0.0;
+        for (size_t r = 0; r < rows; ++r) {
+            const double res = c->hg.bars_d[rows_h ? rows_h[r] : (int)r].res;
+            lo = std::min(lo, res);
+            hi = std::max(hi, res);
+        }
+        int n[2];
+        for (int i = 0; i < 2; ++i) {
+            const double res = i ? hi : lo;
+            ScatterPhys ph;
+            ph.e0 = A.e0;
+            ph.lo = A.same_window ? A.win_lo : (1 - res / 2.0) * A.e0;
+            ph.hi = A.same_window ? A.win_hi : (1 + res / 2.0) * A.e0;
+            ph.res = res;
+            n[i] = win_intervals(ph, window_reject_cos(ph, 0.0));
+        }
+        A.win_n = n[0] > 0 && n[1] > 0 ? std::max(n[0], n[1]) : 0;
+    }
+    if (A.win_n > 0) {
+        e = c->sc_win_rows.reserve(rows);
+        if (e == hipSuccess) e = c->sc_win_tab.reserve(rows * (size_t)A.win_n * 4);
+        if (e != hipSuccess) return e;
+        A.win_rows = c->sc_win_rows.ptr;
+        A.win_tab = c->sc_win_tab.ptr;
+    }
+    return launch_row_cuts(A, c->sc_row_cut.ptr, c->sc_win_rows.ptr, c->sc_win_tab.ptr, c->stream);
 }
 
 // Partial-sum buffer of a scatter launch whose scatter points are split over
@@ -461,7 +494,7 @@ smg_status scatter_launch(smg_ctx* c, bool collimator, int rotation, int variant
     A.n_rows = 0;
     A.pts_per_bar = 1;
     A.pt_bar0 = 0;
-    SMG_HIP(c, scatter_row_cuts(c, A));
+    SMG_HIP(c, scatter_row_cuts(c, A, prec == SMG_PREC_FP64, nullptr));
     SMG_HIP(c, launch_pair_terms(A, c->stream));
     SMG_HIP(c, scatter_partials(c, A));
     SMG_HIP(c, launch_scatter(A, prec == SMG_PREC_FP64, c->stream));
@@ -603,6 +636,8 @@ smg_status smg_destroy(smg_ctx* c) {
     c->pair.release();
     c->sc_partial.release();
     c->sc_row_cut.release();
+    c->sc_win_rows.release();
+    c->sc_win_tab.release();
     c->proj.release();
     c->kn_tab.release();
     c->cell_tab.release();
@@ -1159,12 +1194,12 @@ smg_status smg_scatter_collimator_grid(smg_ctx* c, int rotation, double pitch_mm
     if (pts.empty()) {
         SMG_HIP(c, hipMemsetAsync(out, 0, n_el * sizeof(float), c->stream));
     }
+    SMG_HIP(c, scatter_row_cuts(c, A, prec == SMG_PREC_FP64, nullptr));
     for (int64_t s0 = 0; s0 < (int64_t)pts.size(); s0 += chunk) {
         A.pts_d = c->pts_grid.ptr + s0;
         A.n_pts = (int)std::min<int64_t>(chunk, (int64_t)pts.size() - s0);
         A.accumulate = s0 > 0;
         SMG_HIP(c, launch_first_leg(A, c->w1.ptr, c->stream));
-        SMG_HIP(c, scatter_row_cuts(c, A));
         SMG_HIP(c, launch_pair_terms(A, c->stream));
         SMG_HIP(c, scatter_partials(c, A));
         SMG_HIP(c, launch_scatter(A, prec == SMG_PREC_FP64, c->stream));
@@ -1303,6 +1338,7 @@ smg_status smg_scatter_crystal_grid(smg_ctx* c, int rotation, int gx, int gy, in
             P.n_use_rows = nr;
         }
     }
+    SMG_HIP(c, scatter_row_cuts(c, A, prec == SMG_PREC_FP64, rows));
     std::vector<ScatterPt<double>> pts((size_t)nbc * npb);
     const int sub[3] = {gx, gy, gz};
     for (int b0 = 0; b0 < g.n_det; b0 += (int)nbc) {
@@ -1327,7 +1363,6 @@ smg_status smg_scatter_crystal_grid(smg_ctx* c, int rotation, int gx, int gy, in
         A.n_pts = nb * npb;
         A.pt_bar0 = b0;
         A.accumulate = b0 > 0;
-        SMG_HIP(c, scatter_row_cuts(c, A));
         SMG_HIP(c, launch_pair_terms(A, c->stream));
         SMG_HIP(c, scatter_partials(c, A));
         SMG_HIP(c, launch_scatter(A, prec == SMG_PREC_FP64, c->stream));

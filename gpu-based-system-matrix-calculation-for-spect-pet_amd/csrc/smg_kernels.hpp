@@ -138,6 +138,11 @@ struct BitmapLaunch {
 
 hipError_t launch_bitmap(const BitmapLaunch& a, bool collimator, hipStream_t stream);
 
+// Domain of a row's window table and the row's 2-sigma cuts (win_domain).
+struct WinRow {
+    double x0, scale, omc_lo, omc_hi;
+};
+
 struct ScatterLaunch {
     PeGeom geom;
     const ScatterPt<double>* pts_d;  // scatter points
@@ -166,12 +171,16 @@ struct ScatterLaunch {
     int pts_per_bar, pt_bar0;        // kind 3: point s lies in bar pt_bar0 + s / pts_per_bar
     double* partial;                 // [slices][rows][V] per-slice sums when the scatter points
                                      // are split over several waves per element
-    const double* kn_table;          // KN prefix table of e0 (FP32 path), or nullptr
+    const double* kn_table;          // KN prefix polynomials of e0 (launch_kn_table)
     const double* row_cut;           // [rows] energy-window cut of each output row
                                      // (window_reject_cos, no margin; launch_row_cuts)
+    int win_n;                       // FP32 launches: intervals of the rows' window tables, or 0:
+                                     // the term evaluates the window probability itself
+    const WinRow* win_rows;          // [rows], and
+    const float* win_tab;            // [rows][win_n][4] (launch_row_cuts)
 };
 
-// KN prefix table of e0 ((kKnPhase + 1) x kKnSteps doubles) into tab.
+// KN prefix polynomials of e0 (kKnPolySize doubles) into tab.
 hipError_t launch_kn_table(double e0, double* tab, hipStream_t stream);
 
 // Grid scatterers: first-leg weights w1[s][v] = w_s / (4 pi L^2) exp(-att) of
@@ -180,7 +189,8 @@ hipError_t launch_first_leg(const ScatterLaunch& a, float* w1, hipStream_t strea
 
 // The energy-window cut of each output row into cut[rows], read by the pair
 // terms and scatter kernels of the same launch (a.row_cut).
-hipError_t launch_row_cuts(const ScatterLaunch& a, double* cut, hipStream_t stream);
+// With a.win_n > 0 also the rows' window tables (win[rows], tab[rows][win_n][4]).
+hipError_t launch_row_cuts(const ScatterLaunch& a, double* cut, WinRow* win, float* tab, hipStream_t stream);
 hipError_t launch_pair_terms(const ScatterLaunch& a, hipStream_t stream);
 // out[i] = a[i] + b[i], i < n (the PE + scatter block).
 hipError_t launch_add_blocks(const float* a, const float* b, float* out, size_t n, hipStream_t stream);

@@ -29,9 +29,8 @@ namespace smg {
 
 namespace {
 
-// The energy-window cut of bar d's row (window_reject_cos with no margin).
-__device__ double row_window_cos(const ScatterLaunch& A, const Bar<double>& bd) {
-    ScatterPhys ph;
+// The energy window of bar d's row.
+__device__ __forceinline__ void row_phys(const ScatterLaunch& A, const Bar<double>& bd, ScatterPhys& ph) {
     ph.e0 = A.e0;
     if (A.same_window) {
         ph.lo = A.win_lo;
@@ -41,17 +40,37 @@ __device__ double row_window_cos(const ScatterLaunch& A, const Bar<double>& bd) 
         ph.hi = (1 + bd.res / 2.0) * A.e0;
     }
     ph.res = bd.res;
-    return window_reject_cos(ph, 0.0);
 }
 
-// One thread per output row: its energy-window cut, once per launch instead
-// of once per pair-term thread and per scatter wave (an 80-step FP64
-// bisection).
-__global__ __launch_bounds__(64) void row_cut_kernel(ScatterLaunch A, double* cut) {
+// One thread per output row: its energy-window cut (window_reject_cos with no
+// margin), and the domain of its window table, once per launch instead of once
+// per pair-term thread and per scatter wave (80-step FP64 bisections).
+__global__ __launch_bounds__(64) void row_cut_kernel(ScatterLaunch A, double* cut, WinRow* win) {
     const int r = (int)(blockIdx.x * 64 + threadIdx.x);
     const int n_rows = A.rows ? A.n_rows : A.geom.g.n_det;
     if (r >= n_rows) return;
-    cut[r] = row_window_cos(A, A.geom.bars_d[A.rows ? A.rows[r] : r]);
+    ScatterPhys ph;
+    row_phys(A, A.geom.bars_d[A.rows ? A.rows[r] : r], ph);
+    cut[r] = window_reject_cos(ph, 0.0);
+    if (A.win_n > 0) {
+        win_domain(ph, cut[r], A.win_n);
+        win[r] = WinRow{ph.win_x0, ph.win_scale, ph.omc_lo, ph.omc_hi};
+    }
+}
+
+// One thread per interval of a row's window table.
+__global__ __launch_bounds__(256) void win_table_kernel(ScatterLaunch A, const WinRow* win, float* tab) {
+    const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int n_rows = A.rows ? A.n_rows : A.geom.g.n_det;
+    if (tid >= (int64_t)n_rows * A.win_n) return;
+    const int r = (int)(tid / A.win_n), i = (int)(tid % A.win_n);
+    ScatterPhys ph;
+    row_phys(A, A.geom.bars_d[A.rows ? A.rows[r] : r], ph);
+    ph.win_x0 = win[r].x0;
+    ph.win_scale = win[r].scale;
+    float c[4];
+    win_interval(ph, i, c);
+    *(float4*)(tab + 4 * tid) = make_float4(c[0], c[1], c[2], c[3]);
 }
 
 // True when the terms of scatter point qs and sub-cell centre q lie below the
@@ -265,7 +284,8 @@ struct ScatterLists {
 // inline FP64 fallback holds; measured 14% faster (FP32) and 5% (FP64) than the
 // 2 waves the unconstrained allocation gives.  LDS: 11.3 KB (FP32) / 10.2 KB
 // (FP64) per wave, 12 waves per CU.
-template <bool kExact>
+// kWin: the FP32 term with the row's window table (scatter_term's kTab).
+template <bool kExact, bool kWin>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void scatter_kernel(
     ScatterLaunch A, SliceShape sh) {
     using T = typename std::conditional<kExact, double, float>::type;
@@ -304,19 +324,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void sc
     to_frame(bd, p, ps);
 
     ScatterPhys ph;
-    ph.e0 = A.e0;
-    if (A.same_window) {
-        ph.lo = A.win_lo;
-        ph.hi = A.win_hi;
-    } else {  // per-bar window E0 (1 -+ res/2) (scatter.cu:1154-1163)
-        ph.lo = (1 - bd.res / 2.0) * A.e0;
-        ph.hi = (1 + bd.res / 2.0) * A.e0;
-    }
+    row_phys(A, bd, ph);
     ph.norm = A.kn_norm;
+    ph.inv_norm = uniform_d(1.0 / A.kn_norm);
     ph.tab = A.tables;
     ph.tabf = A.tables_f;
-    ph.knt = A.kn_table;
-    ph.res = bd.res;
+    ph.knp = A.kn_table;
+    if constexpr (kWin) {
+        const WinRow& w = A.win_rows[r];
+        ph.win = A.win_tab + (int64_t)r * A.win_n * 4;
+        ph.win_n = A.win_n;
+        ph.win_x0 = uniform_d(w.x0);
+        ph.win_scale = uniform_d(w.scale);
+        ph.omc_lo = uniform_d(w.omc_lo);
+        ph.omc_hi = uniform_d(w.omc_hi);
+    }
     ph.mupe = bd.mupe;
     ph.muc = bd.muc;
     {
@@ -435,11 +457,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void sc
                     T val = T(0);
                     if (wgt != T(0)) {
                         bool near = false;
-                        val = scatter_term<T>(ph, po, pso, sk, wgt, near);
+                        val = scatter_term<T, kExact || kWin>(ph, po, pso, sk, wgt, near);
                         if constexpr (!kExact) {
                             if (near) {
                                 bool n2 = false;
-                                val = T(scatter_term<double>(ph, po, pso, sk, double(wgt), n2));
+                                val = T(scatter_term<double, true>(ph, po, pso, sk, double(wgt), n2));
                                 ++fallbacks;
                             }
                         }
@@ -470,11 +492,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void sc
     }
 }
 
-// One thread per row of the KN prefix table.
-__global__ __launch_bounds__(64) void kn_table_kernel(double alpha, double* tab) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j > kKnPhase) return;
-    kn_prefix_row(alpha, j, tab + (size_t)j * kKnSteps);
+// The KN prefix polynomials of alpha, one block: thread k forms node k of every
+// phase, one thread per phase sums them in order, thread k expands its
+// polynomial.
+__global__ __launch_bounds__(kKnSteps) void kn_table_kernel(double alpha, double* tab) {
+    __shared__ double node[kKnDeg + 1][kKnSteps];
+    const int k = threadIdx.x;
+    for (int m = 0; m <= kKnDeg; ++m) node[m][k] = kn_node(alpha, kn_phase(m), k);
+    __syncthreads();
+    if (k <= kKnDeg) {
+        KahanSum<double> s;
+        for (int i = 0; i < kKnSteps; ++i) {
+            s.add(node[k][i]);
+            node[k][i] = s.value();
+        }
+    }
+    __syncthreads();
+    double v[kKnDeg + 1], c[kKnDeg + 1];
+    for (int m = 0; m <= kKnDeg; ++m) v[m] = node[m][k];
+    kn_poly_coeffs(v, c);
+    for (int j = 0; j < kKnStride; ++j) tab[(size_t)k * kKnStride + j] = j <= kKnDeg ? c[j] : 0.0;
 }
 
 // Sum of the slices' partial sums of one element, in slice order (a fixed
@@ -526,14 +563,18 @@ hipError_t launch_first_leg(const ScatterLaunch& A, float* w1, hipStream_t strea
 }
 
 hipError_t launch_kn_table(double e0, double* tab, hipStream_t stream) {
-    hipLaunchKernelGGL(kn_table_kernel, dim3((kKnPhase + 1 + 63) / 64), dim3(64), 0, stream, e0 / 511.0, tab);
+    hipLaunchKernelGGL(kn_table_kernel, dim3(1), dim3(kKnSteps), 0, stream, e0 / 511.0, tab);
     return hipGetLastError();
 }
 
-hipError_t launch_row_cuts(const ScatterLaunch& A, double* cut, hipStream_t stream) {
+hipError_t launch_row_cuts(const ScatterLaunch& A, double* cut, WinRow* win, float* tab, hipStream_t stream) {
     const int64_t rows = A.rows ? A.n_rows : A.geom.g.n_det;
     if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL(row_cut_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0, stream, A, cut);
+    if (A.win_n > 0 && (!win || !tab)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(row_cut_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0, stream, A, cut, win);
+    if (A.win_n > 0)
+        hipLaunchKernelGGL(win_table_kernel, dim3((unsigned)((rows * A.win_n + 255) / 256)), dim3(256), 0, stream, A,
+                           win, tab);
     return hipGetLastError();
 }
 
@@ -557,9 +598,11 @@ hipError_t launch_scatter(const ScatterLaunch& A, bool exact, hipStream_t stream
     if (blocks <= 0) return hipSuccess;
     if (sh.slices > 1 && !A.partial) return hipErrorInvalidValue;
     if (exact)
-        hipLaunchKernelGGL(scatter_kernel<true>, dim3((unsigned)blocks), dim3(64), 0, stream, A, sh);
+        hipLaunchKernelGGL((scatter_kernel<true, false>), dim3((unsigned)blocks), dim3(64), 0, stream, A, sh);
+    else if (A.win_n > 0)
+        hipLaunchKernelGGL((scatter_kernel<false, true>), dim3((unsigned)blocks), dim3(64), 0, stream, A, sh);
     else
-        hipLaunchKernelGGL(scatter_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, stream, A, sh);
+        hipLaunchKernelGGL((scatter_kernel<false, false>), dim3((unsigned)blocks), dim3(64), 0, stream, A, sh);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || sh.slices == 1) return e;
     const int64_t n = sh.rows * A.geom.g.n_vox;

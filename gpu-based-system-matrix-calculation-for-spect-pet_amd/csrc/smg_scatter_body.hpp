@@ -265,6 +265,14 @@ struct ScatterPhys {
     const double* knt = nullptr;    // KN prefix table (FP32 path), or the node loop
     double c_rej = -2.0;            // cos(theta) below this is outside the window for
                                     // sure (window_reject_cos with the path's margin)
+    // the kernels' tables (scatter_term with kTab set)
+    const double* knp = nullptr;    // KN prefix polynomials (kn_poly_sum)
+    double inv_norm = 0.0;          // 1 / norm
+    const float* win = nullptr;     // window probability of the row (win_table_value), FP32
+    double win_x0 = 0.0, win_scale = 0.0;  // its first 1 - cos(theta) and intervals per unit of it
+    int win_n = 0;                  // its intervals
+    double omc_lo = 3.0, omc_hi = -1.0;    // terms with 1 - cos(theta) >= omc_lo lie below the
+                                    // window, those <= omc_hi above it
 };
 
 // Thresholds with their reference values.
@@ -402,6 +410,181 @@ SMG_FN double kn_sum_table(const double* tab, float lo, float hi, bool& near) {
     return a0 + w * (a1 - a0);
 }
 
+// KN rectangle sums from prefix polynomials.  P(phi, k) above is smooth in phi
+// for every k: over phi = t step, 0 <= t < 1, it is held as a polynomial of degree
+// kKnDeg through its values at the Chebyshev points of [0, 1], kKnStride doubles
+// per k.  The truncation is below FP64 rounding (the step is 0.01 rad), so a sum
+// is good to ~1e-15 absolute; 20 KB stay in a compute unit's first-level cache,
+// where the 658 KB table of phases (kn_prefix_row) was read from the second level.
+constexpr int kKnDeg = 6;
+constexpr int kKnStride = 8;
+constexpr int kKnPolySize = kKnSteps * kKnStride;
+
+// Chebyshev point m of kKnDeg + 1 on [0, 1].
+SMG_FN double kn_phase(int m) {
+    return 0.5 * (1.0 - cos(3.14159265358979323846 * (2 * m + 1) / (2.0 * (kKnDeg + 1))));
+}
+// Node k of phase t (in steps): KN sin times the step.
+SMG_FN double kn_node(double alpha, double t, int k) {
+    const double th = (t + (double)k) * kKnStep;
+    return kn_of_cos<double>(cos(th), alpha) * sin(th) * kKnStep;
+}
+// Power coefficients of the polynomial with the values v at the points kn_phase
+// (Newton's divided differences, expanded).
+SMG_FN void kn_poly_coeffs(const double v[kKnDeg + 1], double c[kKnDeg + 1]) {
+    double d[kKnDeg + 1], x[kKnDeg + 1];
+    for (int i = 0; i <= kKnDeg; ++i) {
+        d[i] = v[i];
+        x[i] = kn_phase(i);
+        c[i] = 0.0;
+    }
+    for (int j = 1; j <= kKnDeg; ++j)
+        for (int i = kKnDeg; i >= j; --i) d[i] = (d[i] - d[i - 1]) / (x[i] - x[i - j]);
+    for (int i = kKnDeg; i >= 0; --i) {  // c <- c (t - x_i) + d_i
+        for (int j = kKnDeg; j >= 1; --j) c[j] = c[j - 1] - x[i] * c[j];
+        c[0] = d[i] - x[i] * c[0];
+    }
+}
+SMG_FN double kn_poly_value(const double* tab, int k, double t) {
+    const double* c = tab + (size_t)(k < 0 ? 0 : (k >= kKnSteps ? kKnSteps - 1 : k)) * kKnStride;
+    double p = c[kKnDeg];
+#pragma unroll
+    for (int j = kKnDeg - 1; j >= 0; --j) p = p * t + c[j];
+    return p;
+}
+// Sum of n + 1 nodes from lo.
+SMG_FN double kn_poly_sum(const double* tab, double lo, int n) {
+    const double u = lo * (1.0 / kKnStep);
+    const int k0 = (int)floor(u);
+    const double t = u - (double)k0;
+    const double a = kn_poly_value(tab, k0 + n, t);
+    return k0 > 0 ? a - kn_poly_value(tab, k0 - 1, t) : a;
+}
+
+// Energy-window probability of a term with scattered energy ratio g = E'/E0
+// (scatter.cu:1025-1033), FP64; erfc keeps the difference accurate when both
+// ends lie on one side.
+SMG_FN double window_prob(double e0, double lo, double hi, double res, double g) {
+    const double ep = e0 * g, s2 = res * sqrt(g) / kFwhm * ep * sqrt(2.0);
+    const double z1 = (lo - ep) / s2, z2 = (hi - ep) / s2;
+    if (z1 >= 0.0) return 0.5 * (erfc(z1) - erfc(z2));
+    if (z2 <= 0.0) return 0.5 * (erfc(-z2) - erfc(-z1));
+    return 0.5 * (erf(z2) - erf(z1));
+}
+
+// The upper 2-sigma cut of a term (scatter.cu:1263-1269) rejects it when
+// e0 g (1 - r sqrt(g)) >= hi, r = 2 res / FWHM; for r < 2/3 the left side grows
+// with g on [0, 1], so the test is 1 - cos(theta) <= omc_hi for one value per
+// row, found by bisection; -1 when nothing is rejected.
+SMG_FN double window_reject_omc_hi(const ScatterPhys& ph) {
+    const double alpha = ph.e0 / 511.0, r = ph.res * (2.0 / kFwhm);
+    if (ph.e0 * (1.0 - r) < ph.hi) return -1.0;
+    double g0 = 0.0, g1 = 1.0;  // below hi at g0, at or above it at g1
+    for (int it = 0; it < 80; ++it) {
+        const double gm = 0.5 * (g0 + g1);
+        if (ph.e0 * gm * (1.0 - r * sqrt(gm)) >= ph.hi) g1 = gm;
+        else g0 = gm;
+    }
+    return (1.0 / g1 - 1.0) / alpha;
+}
+
+// The window probability of a row as cubics over equal intervals of x =
+// 1 - cos(theta), for the x the 2-sigma cuts leave: interval i holds 4 floats,
+// value = ((c3 t + c2) t + c1) t + c0, t in [0, 1).  The probability is a Gaussian
+// integral with its ends at z1, z2 standard deviations (times sqrt 2) from E':
+// with z moving by at most kWinStep per interval the cubic through the interval's
+// 4 Chebyshev points is within 2e-8 of it, relative.
+constexpr double kWinStep = 0.04;
+constexpr int kWinMin = 128, kWinMax = 1024;  // intervals
+
+SMG_FN void win_cubic(const double v[4], float c[4]) {
+    // Chebyshev points of [0, 1]
+    const double x[4] = {0.5 * (1.0 - 0.92387953251128675613), 0.5 * (1.0 - 0.38268343236508977173),
+                         0.5 * (1.0 + 0.38268343236508977173), 0.5 * (1.0 + 0.92387953251128675613)};
+    double d[4] = {v[0], v[1], v[2], v[3]}, p[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int j = 1; j < 4; ++j)
+        for (int i = 3; i >= j; --i) d[i] = (d[i] - d[i - 1]) / (x[i] - x[i - j]);
+    for (int i = 3; i >= 0; --i) {
+        for (int j = 3; j >= 1; --j) p[j] = p[j - 1] - x[i] * p[j];
+        p[0] = d[i] - x[i] * p[0];
+    }
+    for (int i = 0; i < 4; ++i) c[i] = float(p[i]);
+}
+SMG_FN double win_point(int m) {
+    return 0.5 * (1.0 + (m < 2 ? -1.0 : 1.0) * (m == 0 || m == 3 ? 0.92387953251128675613 : 0.38268343236508977173));
+}
+// Interval i of the table of a row with n intervals.
+SMG_FN void win_interval(const ScatterPhys& ph, int i, float c[4]) {
+    const double alpha = ph.e0 / 511.0;
+    double v[4];
+    for (int m = 0; m < 4; ++m) {
+        const double x = ph.win_x0 + ((double)i + win_point(m)) / ph.win_scale;
+        v[m] = window_prob(ph.e0, ph.lo, ph.hi, ph.res, 1.0 / (1.0 + alpha * x));
+    }
+    win_cubic(v, c);
+}
+// The table's domain from the row's cuts: cut is window_reject_cos(ph, 0).
+SMG_FN void win_domain(ScatterPhys& ph, double cut, int n) {
+    ph.omc_lo = cut < -1.5 ? 3.0 : (cut > 1.5 ? -1.0 : 1.0 - cut);
+    ph.omc_hi = window_reject_omc_hi(ph);
+    const double a = tmax2(ph.omc_hi, 0.0), b = tmin2(ph.omc_lo, 2.0);
+    ph.win_n = n;
+    ph.win_x0 = a;
+    ph.win_scale = b > a ? (double)n / (b - a) : 1.0;
+}
+SMG_FN float win_table_value(const ScatterPhys& ph, double omc) {
+    const double x = (omc - ph.win_x0) * ph.win_scale;
+    int i = (int)x;
+    i = i < 0 ? 0 : (i >= ph.win_n ? ph.win_n - 1 : i);
+    const float t = float(x - (double)i);
+    const float* c = ph.win + 4 * i;
+    return ((c[3] * t + c[2]) * t + c[1]) * t + c[0];
+}
+// Intervals a row needs for kWinStep (host: the launch takes the largest over its
+// rows), or 0 when kWinMax do not do (a resolution below ~1%) or the upper cut is
+// not monotonic (a resolution above 78%): the FP32 term then evaluates the
+// probability directly.
+inline int win_intervals(const ScatterPhys& ph, double cut) {
+    if (!(ph.res * (2.0 / kFwhm) < 0.66) || !(ph.res > 0.0) || !(ph.e0 > 0.0)) return 0;
+    ScatterPhys q = ph;
+    win_domain(q, cut, 1);
+    const double alpha = q.e0 / 511.0, a = q.win_x0, b = a + 1.0 / q.win_scale;
+    if (!(b > a)) return kWinMin;
+    // |dz/dx| <= (|dE'/dx| / sigma + |lo or hi - E'| |dsigma/dx| / sigma^2) / sqrt 2,
+    // largest at the interval's ends in g; bounded with the smallest sigma, and an
+    // end of the window more than 7.5 sigma off (|z| > 5.3) is as good as infinite
+    const double g0 = 1.0 / (1.0 + alpha * b), g1 = 1.0 / (1.0 + alpha * a);
+    const double sig = q.res / kFwhm * q.e0 * g0 * sqrt(g0);
+    const double far = tmin2(tmax2(tmax2(tabs(q.lo - q.e0 * g0), tabs(q.hi - q.e0 * g0)),
+                                   tmax2(tabs(q.lo - q.e0 * g1), tabs(q.hi - q.e0 * g1))),
+                             7.5 * q.res / kFwhm * q.e0 * g1 * sqrt(g1));
+    const double dz = (q.e0 * alpha * g1 * g1 / sig + far * 1.5 * alpha * g1 / sig) / 1.4142135623730951;
+    const double need = dz * (b - a) / kWinStep;
+    for (int n = kWinMin; n <= kWinMax; n *= 2)
+        if (need <= n) return n;
+    return 0;
+}
+
+// atan2(s, c) for s >= 0, in [0, pi]: the smaller over the larger of s and |c|
+// through a minimax polynomial of atan(a) / a in a^2 on [0, 1] (relative error
+// 1.5e-8, fitted by Remez exchange), so a small angle keeps its relative precision.
+SMG_FN float angle_f(float s, float c) {
+    const float ac = tabs(c), hi = tmax2(s, ac), lo = tmin2(s, ac);
+    const float a = hi > 0.0f ? lo * trcp(hi) : 0.0f, z = a * a;
+    float p = 2.849889686e-03f;
+    p = p * z - 1.606862992e-02f;
+    p = p * z + 4.269152135e-02f;
+    p = p * z - 7.504294813e-02f;
+    p = p * z + 1.064093411e-01f;
+    p = p * z - 1.420364380e-01f;
+    p = p * z + 1.999261975e-01f;
+    p = p * z - 3.333307207e-01f;
+    p = p * z + 1.0f;
+    float r = a * p;
+    r = s > ac ? 1.57079632679489662f - r : r;
+    return c < 0.0f ? 3.14159265358979324f - r : r;
+}
+
 // Angle between u and w (vectors src -> a and a -> det), used for the polar
 // range.  FP64 follows the reference, acos of the clamped cosine
 // (scatter.cu:996-1013); FP32 uses atan2(|u x w|, u.w), which keeps its
@@ -463,8 +646,9 @@ SMG_FN bool below_window(const ScatterPhys& ph, const double p[3], const Scatter
 
 // One (voxel, scatter point, sub-cell) term.  wgt is the weight of the
 // scatter point for this voxel.  Returns 0 for terms outside the 2-sigma
-// energy window (scatter.cu:1263-1269).
-template <class T>
+// energy window (scatter.cu:1263-1269).  kTab: with the kernels' tables (the KN
+// prefix polynomials; in FP32 also the row's window probability).
+template <class T, bool kTab = false>
 SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[3],
                       const ScatterCell& sc, T wgt, bool& near) {
     // Cone angle at the scatter point (scatter.cu:1254), scattered energy
@@ -510,18 +694,21 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
             omc = 1.0 - c;  // the reference's cos and sin of acos(c)
             st = sqrt((1.0 - c) * (1.0 + c));
         } else {
-            double cx = a[1] * b[2] - a[2] * b[1], cy = a[2] * b[0] - a[0] * b[2],
-                   cz = a[0] * b[1] - a[1] * b[0];
-            double inv = 1.0 / sqrt(na2 * nb2);
-            double c = dot * inv;
-            double s2 = (cx * cx + cy * cy + cz * cz) * inv * inv;
-            st = sqrt(s2);
-            omc = c < 0.5 ? 1.0 - c : s2 / (1.0 + c);
+            // 1 - c and 1 - c^2 in FP64 keep nine digits at 0.001 rad
+            const double c = tmax2(tmin2(dot * rsq_fast(na2 * nb2), 1.0), -1.0);
+            omc = 1.0 - c;
+            const double s2 = omc * (1.0 + c);
+            st = s2 > 1e-300 ? s2 * rsq_fast(s2) : 0.0;
         }
     }
     // E' = E0 g with g = 1 / (1 + alpha (1 - cos)); the FP32 path forms the
     // window from g and one reciprocal, the FP64 path as the reference does
-    double ep, resp, z1, z2;
+    double ep = 0.0, resp, z1 = 0.0, z2 = 0.0;
+    T pe_win;
+    if constexpr (kTab && std::is_same<T, float>::value) {
+        if (omc >= ph.omc_lo || omc <= ph.omc_hi) return T(0);  // scatter.cu:1263-1269
+        pe_win = win_table_value(ph, omc);
+    } else {
     if constexpr (std::is_same<T, double>::value) {
         ep = ph.e0 / (1.0 + alpha * omc);
         resp = ph.res * sqrt(ep / ph.e0);
@@ -534,16 +721,15 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
     } else {
         // sigma sqrt(2) = resp E' sqrt(2) / FWHM
         constexpr double k2 = 2.0 / kFwhm, ks2 = 1.4142135623730950488 / kFwhm;
-        const double g = 1.0 / (1.0 + alpha * omc);
+        const double g = rcp_fast(1.0 + alpha * omc);
         ep = ph.e0 * g;
-        resp = ph.res * sqrt(g);
+        resp = ph.res * g * rsq_fast(g);
         if (ep * (1 + resp * k2) <= ph.lo || ep * (1 - resp * k2) >= ph.hi)
             return T(0);  // 2-sigma energy-window early out (scatter.cu:1263-1269)
-        const double inv_s2 = 1.0 / (resp * ks2 * ep);  // 1 / (sigma sqrt 2)
+        const double inv_s2 = resp > 0.0 ? rcp_fast(resp * ks2 * ep) : INFINITY;  // 1 / (sigma sqrt 2)
         z1 = (ph.lo - ep) * inv_s2;
         z2 = (ph.hi - ep) * inv_s2;
     }
-    T pe_win;
     if constexpr (std::is_same<T, double>::value) {
         pe_win = 0.5 * (erf(z2) - erf(z1));
     } else {  // erfc keeps the difference accurate when both z lie on one side
@@ -555,6 +741,7 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
         else
             pe_win = 0.5f * (erff(f2) - erff(f1));
     }
+    }
 
     // azimuthal range from the sub-cell's bounding sphere (scatter.cu:1275-1287);
     // asin is ill-conditioned next to 1, where 1 - r is formed in FP64
@@ -563,19 +750,12 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
         const double L = sc.pt.len, rdet = ph.rcell;
         if (L * st * 2.0 <= rdet) {
             phi = T(kTwoPi);
-        } else {
-            double r;
-            if constexpr (std::is_same<T, double>::value)
-                r = rdet / 2.0 / L / st;
-            else
-                r = rdet / (2.0 * L * st);
-            if constexpr (std::is_same<T, double>::value) {
-                phi = 4.0 * asin(r <= 1.0 ? r : 1.0);
-            } else if (r < 0.75) {
-                phi = 4.0f * asinf(float(r));
-            } else {  // asin(r) = pi/2 - 2 asin(sqrt((1 - r)/2))
-                phi = float(kTwoPi) - 8.0f * asinf(float(sqrt((1.0 - r) * 0.5)));
-            }
+        } else if constexpr (std::is_same<T, double>::value) {
+            const double r = rdet / 2.0 / L / st;
+            phi = 4.0 * asin(r <= 1.0 ? r : 1.0);
+        } else {  // asin(r) as the angle of (r, sqrt((1 - r)(1 + r)))
+            const double r = rdet * rcp_fast(2.0 * L * st);
+            phi = 4.0f * angle_f(float(r), tsqrt(float(tmax2((1.0 - r) * (1.0 + r), 0.0))));
         }
     }
     const T alpha_t = T(alpha);
@@ -612,8 +792,8 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
             tmin = acos(cmax);
             tmax = acos(cmin);
         } else {
-            tmin = atan2f(tsqrt(float((1.0 - cmax) * (1.0 + cmax))), float(cmax));
-            tmax = atan2f(tsqrt(float((1.0 - cmin) * (1.0 + cmin))), float(cmin));
+            tmin = angle_f(tsqrt(float((1.0 - cmax) * (1.0 + cmax))), float(cmax));
+            tmax = angle_f(tsqrt(float((1.0 - cmin) * (1.0 + cmin))), float(cmin));
         }
     }
     // the line voxel -> scatter point, extended 1000 mm, through the sub-cell.
@@ -637,11 +817,13 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
         double D[3];
         for (int k = 0; k < 3; ++k) D[k] = sc.qss[k] - ps[k];
         dis2 = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
-        double dis = sqrt(dis2);
+        double dis = 0.0;
         if constexpr (std::is_same<T, float>::value) {
+            const double idis = rsq_fast(dis2);
+            dis = dis2 * idis;
             // De = D (1 + 1000 / |D|), so |De| - |D| = 1000 up to rounding,
             // which the FP32 end parameter does not see
-            const double f = 1.0 + 1000.0 / dis;
+            const double f = 1.0 + 1000.0 * idis;
             const float De[3] = {float(D[0] * f), float(D[1] * f), float(D[2] * f)};
             SegDir<float> se;
             float tde = 4.0f * kUnit<float> * (tabs(De[0]) + tabs(De[1]) + tabs(De[2]));
@@ -653,6 +835,7 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
             lthru = seg_box_local<true>(se, of, float(double(kSlabEps<float>) - dis), 1000.0f, lo, hi,
                                         near, af);
         } else {
+            dis = sqrt(dis2);
             double De[3];
             for (int k = 0; k < 3; ++k) De[k] = (sc.qss[k] + 1000.0 * D[k] / dis) - ps[k];
             SegDir<double> se;
@@ -662,7 +845,18 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
     }
     if (g_gt(lthru, T(0.001f), T(1e-5), near)) tmin = T(0);
     T K;
-    if constexpr (std::is_same<T, double>::value)
+    if constexpr (kTab) {
+        int n;  // as the node loops form it, with the FP32 loop's flag
+        if constexpr (std::is_same<T, float>::value) {
+            const float x = (tmax - tmin) / float(kKnStep);
+            n = (int)x;
+            const float fr = x - float(n);
+            near |= (fr < 2e-4f && n > 0) | (fr > 1.0f - 2e-4f);
+        } else {
+            n = (int)((tmax - tmin) / kKnStep);
+        }
+        K = T(kn_poly_sum(ph.knp, double(tmin), n) * ph.inv_norm);
+    } else if constexpr (std::is_same<T, double>::value)
         K = kn_sum<T>(tmin, tmax, alpha_t, near) / T(ph.norm);
     else if (ph.knt)
         K = float(kn_sum_table(ph.knt, tmin, tmax, near) / ph.norm);
