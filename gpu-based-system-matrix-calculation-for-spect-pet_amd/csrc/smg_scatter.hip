@@ -268,23 +268,66 @@ SliceShape slice_shape(const ScatterLaunch& A) {
 // k, whatever its voxel), and each lane then adds its own terms in point
 // order: the same sums, in the same order, as the per-point loop.
 constexpr int kScatterBatchPts = 128;  // points with a passing lane per batch
+constexpr int kTestPts = 4;            // points tested per step
 template <bool kExact>
 struct ScatterLists {
-    static constexpr int kCap = kExact ? 512 : 1024;  // pairs per batch
+    static constexpr int kCap = kExact ? 512 : 704;  // pairs per batch
+    static constexpr int kRedo = kExact ? 1 : 128;   // FP32 terms waiting for FP64
     using T = typename std::conditional<kExact, double, float>::type;
     uint64_t mask[kScatterBatchPts];  // lanes whose term passes, per batch point
     int pre[kScatterBatchPts];        // pairs listed before the point
     int pt[kScatterBatchPts];         // the point's index
     uint16_t pair[kCap];              // (batch point << 6) | lane
     T val[kCap];                      // the pairs' terms
-    double vp[3][64], vps[3][64];     // the lanes' voxels: world, frame of bar d
+    double vp[3][64];                 // the lanes' voxels
+    float4 ptest[64];                 // 64 points: the FP32 window test's vector and limit
+    int redo_pt[kRedo];               // the waiting terms' points, and (sub-cell << 6) | lane
+    uint32_t redo_at[kRedo];
 };
 
-// 3 waves per SIMD: the register cap (168) spills a few values that the
-// inline FP64 fallback holds; measured 14% faster (FP32) and 5% (FP64) than the
-// 2 waves the unconstrained allocation gives.  LDS: 11.3 KB (FP32) / 10.2 KB
-// (FP64) per wave, 12 waves per CU.
+// Ball around the wave's voxels: the middle of their extent and the largest
+// distance from it.
+__device__ __forceinline__ void wave_ball(const double p[3], bool valid, double C[3], double& R) {
+    double d2 = 0.0;
+    for (int k = 0; k < 3; ++k) {
+        double lo = valid ? p[k] : 1e300, hi = valid ? p[k] : -1e300;
+        for (int off = 32; off > 0; off >>= 1) {
+            lo = tmin2(lo, __shfl_xor(lo, off));
+            hi = tmax2(hi, __shfl_xor(hi, off));
+        }
+        C[k] = uniform_d(0.5 * (lo + hi));
+        d2 += (p[k] - C[k]) * (p[k] - C[k]);
+    }
+    if (!valid) d2 = 0.0;
+    for (int off = 32; off > 0; off >>= 1) d2 = tmax2(d2, __shfl_xor(d2, off));
+    R = uniform_d(sqrt(d2) * (1.0 + 1e-9) + 1e-9);
+}
+
+// True when the terms of scatter point qs (b = q - qs, nb2 = |b|^2) lie below
+// the energy window for every voxel of the ball (C, R): below_window_all for a
+// wave's voxels, with cos(alpha - beta), sin(beta) = R / L, from products.
+__device__ __forceinline__ bool below_window_ball(double c_lo, const double qs[3], const double b[3], double nb2,
+                                                  const double C[3], double R) {
+    if (c_lo <= -1.5) return false;  // nothing is rejected
+    const double u[3] = {qs[0] - C[0], qs[1] - C[1], qs[2] - C[2]};
+    const double L2 = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
+    if (!(L2 > R * R * (1.0 + 1e-6) + 1e-9) || !(nb2 > 1e-12)) return false;
+    const double iL = rsq_fast(L2);
+    const double ca = tmax2(tmin2((u[0] * b[0] + u[1] * b[1] + u[2] * b[2]) * iL * rsq_fast(nb2), 1.0), -1.0);
+    const double sb = R * iL, cb = sqrt(tmax2(1.0 - sb * sb, 0.0));
+    if (ca >= cb) return false;  // the ball reaches the forward direction
+    return ca * cb + sqrt(tmax2(1.0 - ca * ca, 0.0)) * sb < c_lo - 1.1e-4;
+}
+
 // kWin: the FP32 term with the row's window table (scatter_term's kTab).
+// Bound by the latency of the terms' FP64 chains and gathers: 168 VGPRs, 3 waves
+// per SIMD; a cap of 128 for 4 waves spills as much as the wave gains (1 mm
+// collimator grid 237.6 ms against 239.0, crystal grid 20.9 against 19.2).
+// Dropping whole points by the wave's ball before the lanes' tests took crystal
+// scatter, where 99% of the terms fail, from 28.8 to 25.5 ms; letting FP32 terms
+// near a threshold wait for an FP64 loop outside the FP32 one took the grid from
+// 262.8 to 246.4 ms (with the inline FP64 term its registers are live across the
+// FP32 term).  LDS 9.9 KB per wave.
 template <bool kExact, bool kWin>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void scatter_kernel(
     ScatterLaunch A, SliceShape sh) {
@@ -319,9 +362,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void sc
     const int64_t vv = valid ? v : 0;
     const int nxy = g.nx * g.ny;
     const int iz = (int)(vv / nxy), rem = (int)(vv % nxy);
-    double p[3], ps[3];
+    double p[3];
     voxel_position(g, rem % g.nx, rem / g.nx, iz, A.cphi, A.sphi, p);
-    to_frame(bd, p, ps);
 
     ScatterPhys ph;
     row_phys(A, bd, ph);
@@ -369,10 +411,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void sc
         skip_hi = skip_lo + A.pts_per_bar;
     }
     const int64_t v0 = v - lane;  // first voxel of the wave
-    for (int k = 0; k < 3; ++k) {
-        S.vp[k][lane] = p[k];
-        S.vps[k][lane] = ps[k];
-    }
+    for (int k = 0; k < 3; ++k) S.vp[k][lane] = p[k];
+    double C[3], R;
+    wave_ball(p, valid, C, R);
+    const double c_lo = uniform_d(A.row_cut[r]);
+    const float c_rej = float(ph.c_rej);
     // weight of scatter point s for voxel vo at po
     auto weight = [&](int s, int64_t vo, const double po[3]) -> T {
         if (A.kind == 0) return T(A.pe[(int64_t)s * g.n_vox + vo]) * wscale;
@@ -394,89 +437,198 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void sc
     const uint64_t below = (1ull << lane) - 1ull;  // the lanes under this one
     KahanSum<T> acc;
     unsigned fallbacks = 0;
-    for (int cell = 0; cell < ncell; ++cell) {
+    auto set_cell = [&](int cell, ScatterCell& o) {
         const int a = cell % A.sub[0], b = (cell / A.sub[0]) % A.sub[1], c = cell / (A.sub[0] * A.sub[1]);
         CellCtx cc;
         make_cell_ctx(bd, a, b, c, A.sub[0], A.sub[1], A.sub[2], cc);
-        ScatterCell sc;
-        for (int k = 0; k < 3; ++k) {  // the same for every lane
-            sc.q[k] = uniform_d(cc.q[k]);
-            sc.lo[k] = uniform_d(cc.lo[k]);
-            sc.hi[k] = uniform_d(cc.hi[k]);
+        for (int k = 0; k < 3; ++k) {
+            o.q[k] = cc.q[k];
+            o.lo[k] = cc.lo[k];
+            o.hi[k] = cc.hi[k];
         }
-        int s = s_begin;
-        while (s < s_end) {  // wave-uniform
-            // 1. the batch: points in order until kScatterBatchPts of them have
-            // a passing lane or the list could overflow with the next point
-            int n = 0, nb = 0;
-            while (s < s_end && nb < kScatterBatchPts && n <= Lists::kCap - 64) {
-                const int si = s++;
-                if (si >= skip_lo && si < skip_hi) continue;  // wave-uniform
-                const ScatterPt<double>& sp = A.pts_d[si];
-                sc.qs[0] = sp.x;
-                sc.qs[1] = sp.y;
-                sc.qs[2] = sp.z;
-                const bool pass = valid && !below_window<T>(ph, p, sc);
-                const uint64_t m = __ballot(pass);
-                if (m) {  // wave-uniform
-                    if (pass) S.pair[n + __popcll(m & below)] = (uint16_t)((nb << 6) | lane);
-                    if (lane == 0) {
-                        S.mask[nb] = m;
-                        S.pre[nb] = n;
-                        S.pt[nb] = si;
-                    }
-                    n += __popcll(m);
-                    ++nb;
+    };
+    // scatter point si and the voxel of lane o into sk (its sub-cell set
+    // before), po and pso; the point's weight for the voxel
+    auto set_pair = [&](int si, int o, int cell, ScatterCell& sk, double po[3], double pso[3]) -> T {
+        for (int q = 0; q < 3; ++q) po[q] = S.vp[q][o];
+        to_frame(bd, po, pso);
+        const ScatterPt<double>& sp = A.pts_d[si];
+        sk.qs[0] = sp.x;
+        sk.qs[1] = sp.y;
+        sk.qs[2] = sp.z;
+        to_frame(bd, sk.qs, sk.qss);
+        const PairRec& rec = A.pair[((int64_t)r * A.n_pts + si) * ncell + cell];
+        sk.pt = rec.t;
+        sk.ic = rec.ic;
+        return weight(si, v0 + o, po);
+    };
+    ScatterCell sc;          // the current sub-cell
+    int cell = -1;
+    int s = s_end;           // next point of the range
+    int s_blk = s_end;       // first point of the 64 that `live` describes
+    uint64_t live = 0;       // of those, the ones still to be tested
+    int n = 0, nb = 0;       // the batch: its pairs and its points with a passing lane
+    int base = 0;            // its next 64 pairs
+    bool more = s_begin < s_end;
+    while (more) {  // wave-uniform
+        int n_redo = 0;
+        while (kExact || n_redo <= Lists::kRedo - 64) {
+            if (base >= n) {
+                // 3. the finished batch: each lane's terms in point order (a
+                // term of weight 0 adds an exact 0)
+                __syncthreads();
+                for (int j = 0; j < nb; ++j) {
+                    const uint64_t m = S.mask[j];
+                    if ((m >> lane) & 1ull) acc.add(S.val[S.pre[j] + __popcll(m & below)]);
                 }
-            }
-            __syncthreads();
-            // 2. the listed terms, 64 at a time
-            for (int base = 0; base < n; base += 64) {
-                const int k = base + lane;
-                if (k < n) {
-                    const int e = S.pair[k];
-                    const int j = e >> 6, o = e & 63;
-                    const int si = S.pt[j];
-                    const double po[3] = {S.vp[0][o], S.vp[1][o], S.vp[2][o]};
-                    const double pso[3] = {S.vps[0][o], S.vps[1][o], S.vps[2][o]};
-                    ScatterCell sk;
-                    for (int q = 0; q < 3; ++q) {
-                        sk.q[q] = sc.q[q];
-                        sk.lo[q] = sc.lo[q];
-                        sk.hi[q] = sc.hi[q];
+                __syncthreads();  // the lists are refilled
+                n = nb = base = 0;
+                if (!live && s >= s_end) {
+                    if (++cell >= ncell) {
+                        more = false;
+                        break;
                     }
-                    const ScatterPt<double>& sp = A.pts_d[si];
-                    sk.qs[0] = sp.x;
-                    sk.qs[1] = sp.y;
-                    sk.qs[2] = sp.z;
-                    to_frame(bd, sk.qs, sk.qss);
-                    const PairRec& rec = A.pair[((int64_t)r * A.n_pts + si) * ncell + cell];
-                    sk.pt = rec.t;
-                    sk.ic = rec.ic;
-                    const T wgt = weight(si, v0 + o, po);
-                    T val = T(0);
-                    if (wgt != T(0)) {
-                        bool near = false;
-                        val = scatter_term<T, kExact || kWin>(ph, po, pso, sk, wgt, near);
-                        if constexpr (!kExact) {
-                            if (near) {
-                                bool n2 = false;
-                                val = T(scatter_term<double, true>(ph, po, pso, sk, double(wgt), n2));
-                                ++fallbacks;
+                    s = s_begin;
+                    set_cell(cell, sc);
+                    for (int k = 0; k < 3; ++k) {  // the same for every lane
+                        sc.q[k] = uniform_d(sc.q[k]);
+                        sc.lo[k] = uniform_d(sc.lo[k]);
+                        sc.hi[k] = uniform_d(sc.hi[k]);
+                    }
+                }
+                // 1. the next batch: points in order until kScatterBatchPts of
+                // them have a passing lane or the list could overflow with the
+                // next ones.  Points go through 64 at a time, lane l looking at
+                // point s_blk + l: those below the window for every voxel of the
+                // wave are dropped, and the others leave b = q - qs and the
+                // limit of the lanes' test.
+                while (nb <= kScatterBatchPts - kTestPts && n <= Lists::kCap - 64 * kTestPts) {
+                    if (!live) {
+                        if (s >= s_end) break;
+                        s_blk = s;
+                        s = min(s + 64, s_end);
+                        const int si = s_blk + lane;
+                        bool keep = si < s && !(si >= skip_lo && si < skip_hi);
+                        if (keep) {
+                            const ScatterPt<double>& sp = A.pts_d[si];
+                            const double qs[3] = {sp.x, sp.y, sp.z};
+                            const double bq[3] = {sc.q[0] - qs[0], sc.q[1] - qs[1], sc.q[2] - qs[2]};
+                            const double nb2 = bq[0] * bq[0] + bq[1] * bq[1] + bq[2] * bq[2];
+                            keep = !below_window_ball(c_lo, qs, bq, nb2, C, R);
+                            // a.b < c |a| |b| as signed squares: a.b |a.b| < (c |c| |b|^2) |a|^2
+                            S.ptest[lane] = make_float4(float(bq[0]), float(bq[1]), float(bq[2]),
+                                                        c_rej * tabs(c_rej) * float(nb2));
+                        }
+                        live = __ballot(keep);
+                        __syncthreads();
+                        continue;
+                    }
+                    // kTestPts points at a time, their data fetched together
+                    int pi[kTestPts];
+                    double qx[kTestPts], qy[kTestPts], qz[kTestPts];
+                    float4 t[kTestPts];
+                    bool on[kTestPts];
+#pragma unroll
+                    for (int u = 0; u < kTestPts; ++u) {
+                        on[u] = live != 0;
+                        pi[u] = on[u] ? __ffsll((unsigned long long)live) - 1 : (u ? pi[u - 1] : 0);
+                        if (on[u]) live &= live - 1;
+                        const ScatterPt<double>& sp = A.pts_d[s_blk + pi[u]];
+                        qx[u] = sp.x;
+                        qy[u] = sp.y;
+                        qz[u] = sp.z;
+                        if constexpr (!kExact) t[u] = S.ptest[pi[u]];
+                    }
+#pragma unroll
+                    for (int u = 0; u < kTestPts; ++u) {
+                        bool pass;
+                        if constexpr (kExact) {
+                            sc.qs[0] = qx[u];
+                            sc.qs[1] = qy[u];
+                            sc.qs[2] = qz[u];
+                            pass = valid && on[u] && !below_window<T>(ph, p, sc);
+                        } else {
+                            const float ax = float(qx[u] - p[0]), ay = float(qy[u] - p[1]), az = float(qz[u] - p[2]);
+                            const float ab = ax * t[u].x + ay * t[u].y + az * t[u].z;
+                            pass = valid && on[u] && !(ab * tabs(ab) < t[u].w * (ax * ax + ay * ay + az * az));
+                        }
+                        const uint64_t m = __ballot(pass);
+                        if (m) {  // wave-uniform
+                            if (pass) S.pair[n + __popcll(m & below)] = (uint16_t)((nb << 6) | lane);
+                            if (lane == 0) {
+                                S.mask[nb] = m;
+                                S.pre[nb] = n;
+                                S.pt[nb] = s_blk + pi[u];
                             }
+                            n += __popcll(m);
+                            ++nb;
                         }
                     }
-                    S.val[k] = val;
+                }
+                __syncthreads();
+                continue;
+            }
+            // 2. the batch's next 64 terms
+            const int k = base + lane;
+            base += 64;
+            bool near = false;
+            int at = 0, si = 0;
+            if (k < n) {
+                const int e = S.pair[k];
+                at = e & 63;
+                si = S.pt[e >> 6];
+                ScatterCell sk;
+                double po[3], pso[3];
+                for (int q = 0; q < 3; ++q) {
+                    sk.q[q] = sc.q[q];
+                    sk.lo[q] = sc.lo[q];
+                    sk.hi[q] = sc.hi[q];
+                }
+                const T wgt = set_pair(si, at, cell, sk, po, pso);
+                T val = T(0);
+                if (wgt != T(0)) val = scatter_term<T, kExact || kWin>(ph, po, pso, sk, wgt, near);
+                S.val[k] = (!kExact && near) ? T(0) : val;
+            }
+            if constexpr (!kExact) {
+                // an FP32 term near a threshold waits for FP64
+                const uint64_t m = __ballot(near);
+                if (m) {  // wave-uniform
+                    if (near) {
+                        const int i = n_redo + __popcll(m & below);
+                        S.redo_pt[i] = si;
+                        S.redo_at[i] = ((uint32_t)cell << 6) | (uint32_t)at;
+                    }
+                    n_redo += __popcll(m);
+                }
+            }
+        }
+        if constexpr (!kExact) {
+            // the waiting terms, outside the loop above so that their FP64
+            // registers are not live in it; each goes to its voxel's lane, in
+            // list order
+            __syncthreads();
+            for (int i0 = 0; i0 < n_redo; i0 += 64) {
+                const int i = i0 + lane;
+                double val = 0.0;
+                int at = 0;
+                if (i < n_redo) {
+                    const int c = (int)(S.redo_at[i] >> 6);
+                    at = (int)(S.redo_at[i] & 63u);
+                    ScatterCell sk;
+                    double po[3], pso[3];
+                    set_cell(c, sk);
+                    const T wgt = set_pair(S.redo_pt[i], at, c, sk, po, pso);
+                    bool n2 = false;
+                    val = scatter_term<double, true>(ph, po, pso, sk, double(wgt), n2);
+                    ++fallbacks;
+                }
+                const int cnt = min(64, n_redo - i0);
+                for (int e = 0; e < cnt; ++e) {
+                    const double x = __shfl(val, e);
+                    if (lane == __shfl(at, e)) acc.add(T(x));
                 }
             }
             __syncthreads();
-            // 3. each lane's terms in point order (a term of weight 0 adds
-            // an exact 0)
-            for (int j = 0; j < nb; ++j) {
-                const uint64_t m = S.mask[j];
-                if ((m >> lane) & 1ull) acc.add(S.val[S.pre[j] + __popcll(m & below)]);
-            }
-            __syncthreads();  // the lists are refilled by the next batch
         }
     }
     if (valid) {

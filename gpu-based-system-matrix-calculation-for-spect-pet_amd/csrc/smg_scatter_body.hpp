@@ -220,7 +220,21 @@ SMG_FN int mu_seg_f(const MuTablesF& t, float L) {
 }
 
 SMG_FN float mu_ratio_f(const MuTablesF& t, int which, int j, float L) {
-    return expf(t.c[which][j] - t.s[which][j] * L);
+    const float x = t.c[which][j] - t.s[which][j] * L;
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_exp2f(x * 1.44269504088896341f);  // |x| is a few units: no denormals
+#else
+    return expf(x);
+#endif
+}
+
+// ln(x) for x >= 1 not far above it (E0/E').
+SMG_FN float log_f(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_logf(x) * 0.693147180559945309f;  // log2, normal argument
+#else
+    return logf(x);
+#endif
 }
 
 // Host: the FP32 form of t for photopeak e0 (alpha = e0 / 511).
@@ -667,11 +681,14 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
         // FP32 pre-test of the lower window cut (most terms of a scatter
         // matrix fall below the window): cos theta < c_rej  <=>
         // a.b < c_rej |a| |b|; a term near the cut goes on to the FP64 test
-        const float ax = float(a[0]), ay = float(a[1]), az = float(a[2]);
-        const float bx = float(b[0]), by = float(b[1]), bz = float(b[2]);
-        const float ab = ax * bx + ay * by + az * bz;
-        const float nn = (ax * ax + ay * ay + az * az) * (bx * bx + by * by + bz * bz);
-        if (ab < float(ph.c_rej) * tsqrt(nn)) return T(0);
+        // (kTab: the caller has made it)
+        if constexpr (!kTab) {
+            const float ax = float(a[0]), ay = float(a[1]), az = float(a[2]);
+            const float bx = float(b[0]), by = float(b[1]), bz = float(b[2]);
+            const float ab = ax * bx + ay * by + az * bz;
+            const float nn = (ax * ax + ay * ay + az * az) * (bx * bx + by * by + bz * bz);
+            if (ab < float(ph.c_rej) * tsqrt(nn)) return T(0);
+        }
         // mu(E) tables without an FP32 form (more segments in range than it
         // holds): the whole term goes to the FP64 path, which keeps FP64
         // logarithms and exponentials out of the FP32 term
@@ -768,6 +785,7 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
     // sin^2 = (1 - c)(1 + c) keeps a small angle's relative precision.
     T us[3];
     T tmin, tmax;
+    double cmin = 0.0, cmax = 0.0;  // their cosines
     {
         double u[3], pl[3], ph8[3];
         for (int k = 0; k < 3; ++k) {
@@ -776,7 +794,6 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
             pl[k] = u[k] * (sc.lo[k] - sc.qss[k]);
             ph8[k] = u[k] * (sc.hi[k] - sc.qss[k]);
         }
-        double cmin = 0.0, cmax = 0.0;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             const double dot = ((c & 1 ? ph8[0] : pl[0]) + (c & 2 ? ph8[1] : pl[1])) + (c & 4 ? ph8[2] : pl[2]);
@@ -796,9 +813,9 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
             tmax = angle_f(tsqrt(float((1.0 - cmin) * (1.0 + cmin))), float(cmin));
         }
     }
-    // the line voxel -> scatter point, extended 1000 mm, through the sub-cell.
-    // FP32 path: only its test against 0.001 is used, and a line that passes
-    // the sub-cell's centre farther than its bounding radius + 0.01 mm has
+    // the line voxel -> scatter point, extended 1000 mm, through the sub-cell:
+    // only the test of its chord against 0.001 is used.  FP32 path: a line that
+    // passes the sub-cell's centre farther than its bounding radius + 0.01 mm has
     // chord 0 in the reference too (its small-component branches move the
     // line by less than 0.001 mm), so the chord is formed only otherwise.
     T lthru = T(0);
@@ -813,29 +830,38 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
         lthru_needed = !(cx * cx + cy * cy + cz * cz > R * R * u2);
     }
     if (lthru_needed) {
-        double dis2 = 0.0;
-        double D[3];
-        for (int k = 0; k < 3; ++k) D[k] = sc.qss[k] - ps[k];
-        dis2 = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
-        double dis = 0.0;
+        double D[3], dis2 = 0.0;
+        for (int k = 0; k < 3; ++k) {
+            D[k] = sc.qss[k] - ps[k];
+            dis2 += D[k] * D[k];
+        }
         if constexpr (std::is_same<T, float>::value) {
-            const double idis = rsq_fast(dis2);
-            dis = dis2 * idis;
-            // De = D (1 + 1000 / |D|), so |De| - |D| = 1000 up to rounding,
-            // which the FP32 end parameter does not see
-            const double f = 1.0 + 1000.0 * idis;
-            const float De[3] = {float(D[0] * f), float(D[1] * f), float(D[2] * f)};
-            SegDir<float> se;
-            float tde = 4.0f * kUnit<float> * (tabs(De[0]) + tabs(De[1]) + tabs(De[2]));
-            segdir_init<float>(se, De[0], De[1], De[2], tde, near);
-            float of[3] = {float(sc.qss[0]), float(sc.qss[1]), float(sc.qss[2])};
-            float lo[3] = {float(sc.lo[0]), float(sc.lo[1]), float(sc.lo[2])};
-            float hi[3] = {float(sc.hi[0]), float(sc.hi[1]), float(sc.hi[2])};
-            const float af[3] = {float(ps[0]), float(ps[1]), float(ps[2])};
-            lthru = seg_box_local<true>(se, of, float(double(kSlabEps<float>) - dis), 1000.0f, lo, hi,
-                                        near, af);
+            // FP64 slab test of the extended line (length_box_ray; a line with one
+            // component below eps must start strictly between that axis' faces
+            // and runs over the other two, PESysMatGen.cu:69-73, and one with more
+            // goes to the FP64 path): an FP32 form with tolerances on every
+            // comparison takes three times the instructions.  The extension
+            // leaves len / D_k as it is.
+            const double idis = rsq_fast(dis2), dis = dis2 * idis, f = 1.0 + 1000.0 * idis;
+            const double eps = kSlabEps<double>;
+            double t0 = -1e300, t1 = 1e300;
+            int ns = 0;
+            bool in = true;
+            for (int k = 0; k < 3; ++k) {
+                const bool small = tabs(D[k] * f) < eps;
+                const double inv = dis * rcp_fast(small ? 1.0 : D[k]);
+                const double u = (sc.lo[k] - ps[k]) * inv, w = (sc.hi[k] - ps[k]) * inv;
+                t0 = small ? t0 : tmax2(t0, tmin2(u, w));
+                t1 = small ? t1 : tmin2(t1, tmax2(u, w));
+                in = in && (!small || (ps[k] > sc.lo[k] && ps[k] < sc.hi[k]));
+                ns += small;
+            }
+            near |= ns > 1;
+            const double end = dis + 1000.0;
+            const bool hit = in && t1 - t0 >= eps && t0 > eps && t1 < end;
+            lthru = hit && t1 - t0 > (double)0.001f ? 1.0f : 0.0f;
         } else {
-            dis = sqrt(dis2);
+            const double dis = sqrt(dis2);
             double De[3];
             for (int k = 0; k < 3; ++k) De[k] = (sc.qss[k] + 1000.0 * D[k] / dis) - ps[k];
             SegDir<double> se;
@@ -843,15 +869,21 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
             lthru = seg_box<double>(se, ps, sc.lo, sc.hi, near);
         }
     }
-    if (g_gt(lthru, T(0.001f), T(1e-5), near)) tmin = T(0);
+    if (lthru > T(0.001f)) tmin = T(0);
     T K;
     if constexpr (kTab) {
-        int n;  // as the node loops form it, with the FP32 loop's flag
+        int n;  // as the node loop forms it
         if constexpr (std::is_same<T, float>::value) {
-            const float x = (tmax - tmin) / float(kKnStep);
+            // a node count within the angles' rounding (below 1e-4 steps) of an
+            // integer is formed from FP64 angles; sending the whole term to
+            // FP64 for it (4 in 10,000 terms, so one in 40 of the 64 that a wave
+            // evaluates together) took the 1 mm collimator grid 272 ms instead
+            // of 263
+            const float x = (tmax - tmin) * float(1.0 / kKnStep);
             n = (int)x;
             const float fr = x - float(n);
-            near |= (fr < 2e-4f && n > 0) | (fr > 1.0f - 2e-4f);
+            if ((fr < 2e-4f && n > 0) || fr > 1.0f - 2e-4f)
+                n = (int)((acos(cmin) - (tmin == 0.0f ? 0.0 : acos(cmax))) / kKnStep);
         } else {
             n = (int)((tmax - tmin) / kKnStep);
         }
@@ -875,7 +907,7 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
             e1 = 1.0 + alpha * omc;
             e3 = e1 * e1 * e1;
         } else {
-            Lf = logf(float(1.0 + alpha * omc));  // ln(E0/E')
+            Lf = log_f(float(1.0 + alpha * omc));  // ln(E0/E')
             jf = mu_seg_f(*ph.tabf, Lf);
             e3 = mu_ratio_f(*ph.tabf, 0, jf, Lf);
             e1 = mu_ratio_f(*ph.tabf, 1, jf, Lf);

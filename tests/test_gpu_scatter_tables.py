@@ -1,0 +1,30 @@
+"""Scatter launches at the edges of the window tables: resolutions sharp enough
+that the FP32 term evaluates the window probability itself, the largest and
+smallest tables, windows relative to each bar's resolution, and detector
+sub-cells (one batch state over several of them)."""
+import numpy as np
+import pytest
+
+from conftest import TOL_FP32, TOL_FP64, assert_parity
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("res,same_window,sub", [(0.004, 1, (1, 1, 1)), (0.012, 1, (1, 1, 1)), (0.03, 0, (2, 1, 2)),
+                                                 (0.1, 0, (1, 1, 1)), (0.3, 1, (1, 2, 1)), (0.9, 1, (1, 1, 1))])
+def test_collimator_scatter_windows(smg_mod, oracle_mod, params_mod, res, same_window, sub):
+    p = params_mod.config(3)
+    params_mod.set_image(p, 9, 7, 3, 1.0, 1.0, 1.0)
+    n = p.n_det
+    p.det[10:10 + 12 * n:12] = np.float32(res) * np.linspace(0.97, 1.03, n).astype(np.float32)
+    params_mod.set_physics(p, same_window=same_window)
+    o = oracle_mod.Oracle(p)
+    d, v = [a.reshape(-1).astype(np.int32) for a in np.meshgrid(np.arange(0, n, 5), np.arange(p.n_vox), indexing="ij")]
+    ref = o.collimator_scatter_pairs(o.bitmap_collimator(), d, v, variant=0, sub=sub)
+    assert (ref > 0).any()
+    with smg_mod.open_context(p) as ctx:
+        ctx.set_scatter_subsamples(*sub)
+        for prec, tol in (("fp32", TOL_FP32), ("fp64", TOL_FP64)):
+            got, st = ctx.scatter_collimator(0, "combined", prec)
+            assert_parity(got[d, v].astype(np.float64), ref, tol,
+                          f"windows res={res} same={same_window} {prec} fallbacks={st['fp64_fallbacks']}")
