@@ -28,3 +28,26 @@ def test_collimator_scatter_windows(smg_mod, oracle_mod, params_mod, res, same_w
             got, st = ctx.scatter_collimator(0, "combined", prec)
             assert_parity(got[d, v].astype(np.float64), ref, tol,
                           f"windows res={res} same={same_window} {prec} fallbacks={st['fp64_fallbacks']}")
+
+
+@pytest.mark.parametrize("n,sub", [(2, (1, 1, 1)), (32, (1, 1, 1)), (34, (1, 1, 1)), (67, (2, 1, 1)), (131, (1, 1, 1))])
+def test_crystal_scatter_bitmap_words(smg_mod, oracle_mod, params_mod, n, sub):
+    """Records whose bits span 1 to 6 words (several share a wave's pass), with a
+    loaded bitmap that flags half of all bars, turned bars among them."""
+    p = params_mod.config(4)
+    params_mod.set_image(p, 5, 4, 2, 2.0, 2.0, 2.0)
+    p.det[0] = n
+    p.det[11:11 + 12 * n:12][1::3] = 0.3
+    o = oracle_mod.Oracle(p)
+    rng = np.random.default_rng(n)
+    pe = rng.uniform(0, 1e-9, (n, o.n_vox)).astype(np.float32)
+    bm = rng.integers(0, 1 << 32, o.bitmap_crystal().size, dtype=np.uint64).astype(np.uint32)
+    d, v = [a.reshape(-1).astype(np.int32) for a in np.meshgrid(np.arange(n), np.arange(0, o.n_vox, 7), indexing="ij")]
+    ref = o.crystal_scatter_pairs(pe, bm, d, v, sub=sub)
+    assert (ref > 0).any()
+    with smg_mod.open_context(p) as ctx:
+        ctx.set_scatter_subsamples(*sub)
+        ctx.load_bitmap_crystal(bm)
+        for prec, tol in (("fp32", TOL_FP32), ("fp64", TOL_FP64)):
+            got, _ = ctx.scatter_crystal(pe, 0, prec)
+            assert_parity(got[d, v].astype(np.float64), ref, tol, f"bitmap words n={n} {prec}")
