@@ -8,12 +8,13 @@
 // the ray from layer-0 hole h toward bar j; bit index h N^2 + j N + k.
 //
 // A row is the N bits of one pair (i, j) or one (hole h, bar j); along a row
-// only k changes.  The FP32 test keeps the row's terms (the unit vector from i
-// to j and R_j / L_ij) and forms per bit k - i in FP64 (rounded once to FP32,
-// so the direction does not inherit the rounding of ~100 mm coordinates), one
-// reciprocal square root and squared comparisons.  A decision within its
-// rounding bound is redone with the reference formula in FP64, so every bit
-// equals an FP64 evaluation of the reference test.
+// only k changes.  The unit vectors and the ratios R / L come from tables rounded
+// once from FP64 (bm_dir, bm_row), and a decision seen from one end is the sign of
+// bm_margin.  A decision within its rounding bound is redone with the reference
+// formula in FP64, so every bit equals an FP64 evaluation of the reference test.
+//
+// The second half of the file is the same predicate bit by bit (bm_bit), with a
+// row's FP32 terms formed as the walk reaches it: the host's check of the bits.
 #pragma once
 
 #include "smg_geometry.hpp"
@@ -53,6 +54,44 @@ SMG_FN bool bm_crystal_pred(const Sphere<T>& i, const Sphere<T>& j, const Sphere
     near |= n2;
     return a || b;
 }
+
+// From an origin (bar or hole) to a bar: unit vector and R / L.
+struct BmDir {
+    float x, y, z, r;
+};
+
+// What the bits of one row share: twice the unit vector from i to j, and both
+// bars' R / L_ij.
+struct BmRow {
+    float x2, y2, z2;
+    float c, cr;  // R_j / L_ij (seen from i), R_i / L_ij (seen from j)
+};
+
+SMG_FN BmDir bm_dir(const Sphere<double>& o, const Sphere<double>& t) {
+    const double l = bm_dist(o.x, o.y, o.z, t.x, t.y, t.z);
+    return BmDir{float((t.x - o.x) / l), float((t.y - o.y) / l), float((t.z - o.z) / l), float(t.r / l)};
+}
+
+SMG_FN BmRow bm_row(const Sphere<double>& o, const Sphere<double>& t) {
+    const BmDir d = bm_dir(o, t);
+    const double l = bm_dist(o.x, o.y, o.z, t.x, t.y, t.z);
+    return BmRow{2.0f * d.x, 2.0f * d.y, 2.0f * d.z, d.r, float(o.r / l)};
+}
+
+// lim^2 - |u - u'|^2 of the test seen from one end, u and lim's first part from
+// d, twice u' and its second part from the row: positive where the bit is set.
+// NaN where a length is 0, where the reference's comparison is false: so is
+// t > 0, and fmax of the two ends' margins keeps the other one's.
+SMG_FN float bm_margin(const BmDir& d, float x2, float y2, float z2, float c) {
+    const float lim = d.r + c;
+    return fmaf(lim, lim, fmaf(d.z, z2, fmaf(d.y, y2, fmaf(d.x, x2, -2.0f))));
+}
+
+// Rounding bound of bm_margin where its sign is in doubt, in units of 2^-24: the
+// unit vectors' roundings 2 * 2 sqrt(3) / 2, three sums of at most 4 in magnitude
+// 3 * 4, lim (at most 2 there, as |u - u'| is) 2 * 2 lim^2 = 16, the last sum 4:
+// below 36.  Where lim is above 2 the sign is positive by more than any of them.
+constexpr float kBmTol = 48.0f * kUnit<float>;
 
 // 1 / sqrt(x): the hardware reciprocal square root on the device (1 ulp),
 // the operators on the host.

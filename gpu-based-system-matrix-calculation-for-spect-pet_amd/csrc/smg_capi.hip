@@ -85,6 +85,7 @@ struct smg_ctx {
     DevBuf<float> out2, in2;  // second output and input of smg_scatter_sum
     DevBuf<unsigned long long> counters;
     DevBuf<uint32_t> bm_crystal, bm_coll;
+    DevBuf<unsigned char> bm_scratch;  // the bitmaps' direction tables
     bool have_bm_crystal = false, have_bm_coll = false;
     DevBuf<double> scratch;   // adjoint partials
     DevBuf<double> tan_v;     // tangent direction
@@ -283,6 +284,8 @@ smg_status ensure_bitmap(smg_ctx* c, bool collimator) {
     B.n_words = n_words;
     B.n_det = N;
     B.n_holes = hg.n_holes_l0;
+    SMG_HIP(c, c->bm_scratch.reserve(bitmap_scratch_bytes(collimator, N, hg.n_holes_l0)));
+    B.scratch = c->bm_scratch.ptr;
     SMG_HIP(c, launch_bitmap(B, collimator, c->stream));
     SMG_HIP(c, hipStreamSynchronize(c->stream));
     (collimator ? c->have_bm_coll : c->have_bm_crystal) = true;
@@ -625,6 +628,7 @@ smg_status smg_destroy(smg_ctx* c) {
     c->counters.release();
     c->bm_crystal.release();
     c->bm_coll.release();
+    c->bm_scratch.release();
     c->scratch.release();
     c->grad.release();
     c->sph_f.release();

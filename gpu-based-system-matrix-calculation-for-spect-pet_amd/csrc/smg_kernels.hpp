@@ -134,7 +134,10 @@ struct BitmapLaunch {
     uint32_t* words;
     int64_t n_words;
     int n_det, n_holes;
+    void* scratch;                    // bitmap_scratch_bytes
 };
+
+size_t bitmap_scratch_bytes(bool collimator, int n_det, int n_holes);
 
 hipError_t launch_bitmap(const BitmapLaunch& a, bool collimator, hipStream_t stream);
 
