@@ -51,3 +51,19 @@ def test_crystal_scatter_bitmap_words(smg_mod, oracle_mod, params_mod, n, sub):
         for prec, tol in (("fp32", TOL_FP32), ("fp64", TOL_FP64)):
             got, _ = ctx.scatter_crystal(pe, 0, prec)
             assert_parity(got[d, v].astype(np.float64), ref, tol, f"bitmap words n={n} {prec}")
+
+
+@pytest.mark.parametrize("n_rows", [1, 2, 7, 33, 64])
+def test_crystal_grid_row_counts(smg_mod, params_mod, n_rows):
+    """The grid points a few detector rows cannot use are left out, tested with a
+    lane per (point, row): as the full matrix's rows (whose points are all
+    formed), to the rounding of the different slices' sums, 2e-6 in FP32."""
+    p = params_mod.config(4)
+    params_mod.set_image(p, 9, 7, 1, 3.0, 3.0, 3.0)
+    p.det[0] = 90
+    rows = np.random.default_rng(n_rows).permutation(90)[:n_rows].astype(np.int32)
+    with smg_mod.open_context(p) as ctx:
+        full, _ = ctx.scatter_crystal_grid((2, 3, 2), None, 0, "fp32")
+        part, _ = ctx.scatter_crystal_grid((2, 3, 2), rows, 0, "fp32")
+    assert (full > 0).any()
+    np.testing.assert_allclose(part, full[rows], rtol=2e-6, atol=0.0)
