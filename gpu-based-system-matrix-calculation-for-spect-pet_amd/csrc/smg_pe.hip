@@ -40,7 +40,7 @@ constexpr int kRecWords = 244;
 // then holes), then the records of the narrowed pairs: bars upward from word n,
 // holes downward from the end.  The lists are short as a rule (about 27
 // candidates on the full-size geometry), so the records of a whole block fit.
-template <int CapB, int CapH>
+template <int CapB, int CapH, bool kShared = false>
 struct WaveListsT {
     static constexpr int cap_bars = CapB, cap_holes = CapH;
     static constexpr int arena_words = CapB + CapH + kRecWords;
@@ -49,8 +49,19 @@ struct WaveListsT {
     uint64_t sel[sel_cap];       // per sub-cell of the block: the candidates it keeps
     uint64_t redo[kBlockCells];  // per sub-cell of the block: the lanes to redo in FP64
     uint16_t idx[CapB + CapH];   // bar or hole number of each candidate
+    // kShared: the block has several waves, each with lists of its own.  A wave's
+    // LDS accesses are in order: only the compiler has to keep them so.
+    __device__ static void sync() {
+        if constexpr (kShared) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            __syncthreads();
+        }
+    }
 };
 using WaveLists = WaveListsT<kCapBars, kCapHoles>;
+using SharedLists = WaveListsT<kCapBars, kCapHoles, true>;
 
 // The adjoint's lists hold fewer bars: with its per-candidate FP64 sums and
 // kept chords, 13 KB of LDS per wave, so 12 waves (3 per SIMD) fit a CU.
@@ -67,6 +78,7 @@ struct SpillLists {
     uint64_t* redo;
     double* cand_acc;
     uint16_t* idx;
+    __device__ static void sync() { __syncthreads(); }
 };
 
 __device__ __forceinline__ SpillLists spill_lists(const PeSpill& S, int slot) {
@@ -490,9 +502,9 @@ __device__ __forceinline__ void trace_cells(const PeLaunch& A, const Bar<double>
             ns = min(block, c_end - c);
             c += ns;
         }
-        __syncthreads();  // the previous block's lists are no longer read
+        L.sync();  // the previous block's lists are no longer read
         select_cells(A, bd, d, my_cell, ns, W, lane, L, nb, n, words);
-        __syncthreads();
+        L.sync();
         uint64_t flagged = 0;
         if constexpr (kExact) {
             flagged = ns == 64 ? ~0ull : (1ull << ns) - 1ull;
@@ -521,7 +533,7 @@ __device__ __forceinline__ void trace_cells(const PeLaunch& A, const Bar<double>
                     ++s;
                     continue;
                 }
-                __syncthreads();
+                L.sync();
                 for (int i0 = 0; i0 < nbr; i0 += 64) {
                     const int i = i0 + lane;
                     const uint32_t tag = i < nbr ? bars[i].tag : 0u;
@@ -555,7 +567,7 @@ __device__ __forceinline__ void trace_cells(const PeLaunch& A, const Bar<double>
                         r.hole = (uint32_t)k;
                     }
                 }
-                __syncthreads();
+                L.sync();
                 int ib = 0, ih = 0;
                 for (; s < e; ++s) {
                     const int cell = __builtin_amdgcn_readlane(my_cell, s);
@@ -571,7 +583,7 @@ __device__ __forceinline__ void trace_cells(const PeLaunch& A, const Bar<double>
                         if (lane == 0) L.redo[s] = m;
                     }
                 }
-                __syncthreads();
+                L.sync();
             }
         }
         // FP64 rays: the candidates' positions in the place of the records
@@ -584,7 +596,7 @@ __device__ __forceinline__ void trace_cells(const PeLaunch& A, const Bar<double>
             tile_cell(A, bd, d, cell, W, lane, cc);
             ListCands<Lists> C{&L, cur, 0, 0};
             sel_count(L, s, words, nb, C.nb, C.nh);
-            __syncthreads();
+            L.sync();
             int ib = 0, ih = C.nb;
             for (int w = 0; w < words; ++w) {
                 uint64_t mb, mh;
@@ -594,7 +606,7 @@ __device__ __forceinline__ void trace_cells(const PeLaunch& A, const Bar<double>
                 ib += bit_count(mb);
                 ih += bit_count(mh);
             }
-            __syncthreads();
+            L.sync();
             f64(cell, cc, C, W.valid && (kExact || ((L.redo[s] >> lane) & 1ull)));
         }
     }
@@ -669,25 +681,48 @@ __device__ __forceinline__ int points_used(const PeLaunch& A, const Bar<double>&
     return n;
 }
 
+// This wave's number in a block of kWaves, in scalar registers.
+template <int kWaves>
+__device__ __forceinline__ int block_wave() {
+    return kWaves > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+}
+
+// Sum of the lane's accumulators over the block's waves, in wave order, with
+// their compensations, through the waves' candidate lists, which are done with
+// (L: this wave's; slot: 0 or 1).  Every wave comes here; the sum is the first
+// one's.
+template <int kWaves, class T, class Lists>
+__device__ __forceinline__ double block_sum(const KahanSum<T>& acc, int wave, int lane, Lists& L, int slot) {
+    double s = (double)acc.s + (double)acc.c;
+    L.arena[slot * 64 + lane] = (uint64_t)__double_as_longlong(s);
+    __syncthreads();
+    if (wave == 0)
+        for (int w = 1; w < kWaves; ++w) s += __longlong_as_double((long long)(&L)[w].arena[slot * 64 + lane]);
+    return s;
+}
+
 // Work item `item` of the launch (a block index: bar, tile and, for point
 // weights, slice of cells) with candidate lists L.  Returns false, having
 // written nothing, when the candidates overflow L.
-template <bool kExact, bool kPoints, bool kEll, class Lists>
+template <bool kExact, bool kPoints, bool kEll, int kWaves = 1, class Lists>
 __device__ __forceinline__ bool pe_forward_body(const PeLaunch& A, int item, Lists& L) {
     const PeGeom& G = A.geom;
     const GeomDesc& g = G.g;
-    const int lane = threadIdx.x;
+    // (masking the number in blocks of one wave too made the full-size step 0.8% slower)
+    const int lane = kWaves > 1 ? threadIdx.x & 63 : threadIdx.x;
     const int n_tiles = A.tiles[0] * A.tiles[1] * A.tiles[2];
-    // point weights: cells [c_begin, c_end) of the wave's slice; PE: all cells
+    // point weights: cells [c_begin, c_end) of the wave's slice; PE: all cells, or
+    // the wave's share of them
     const int slices = kPoints ? A.cell_slices : 1;
     const int wave = item / slices;
+    const int parts = kPoints ? slices : kWaves, part = kPoints ? item % slices : block_wave<kWaves>();
     const int d = A.bar0 + wave / n_tiles;
     const int tile = wave % n_tiles;
     float* out = A.dst + (int64_t)d * g.n_vox;
     const int n_cells = A.sub[0] * A.sub[1] * A.sub[2];
-    const int per = (n_cells + slices - 1) / slices;
-    const int c_begin = kPoints ? (item % slices) * per : 0;
-    const int c_end = kPoints ? min(n_cells, c_begin + per) : n_cells;
+    const int per = (n_cells + parts - 1) / parts;
+    const int c_begin = part * per;
+    const int c_end = min(n_cells, c_begin + per);
     float* pts = kPoints ? A.pts + (int64_t)(d - A.bar0) * n_cells * g.n_vox : nullptr;
     const Bar<double>& bd = G.bars_d[d];
     WaveSetup W;
@@ -697,13 +732,13 @@ __device__ __forceinline__ bool pe_forward_body(const PeLaunch& A, int item, Lis
             if (W.valid)
                 for (int c = c_begin; c < c_end; ++c) pts[(int64_t)c * g.n_vox + W.v] = 0.0f;
         } else {
-            if (W.valid) out[W.v] = 0.0f;
+            if (W.valid && part == 0) out[W.v] = 0.0f;
         }
         return true;
     }
     int nb, nh;
     if (!build_candidates<kExact>(A, d, lane, W, L, nb, nh)) return false;
-    __syncthreads();
+    L.sync();
 
     using T = typename std::conditional<kExact, double, float>::type;
     KahanSum<T> acc;
@@ -754,7 +789,12 @@ __device__ __forceinline__ bool pe_forward_body(const PeLaunch& A, int item, Lis
             }
         });
     if constexpr (!kPoints) {
-        if (W.valid) out[W.v] = float(acc.value());
+        if constexpr (kWaves > 1) {
+            const double sum = block_sum<kWaves>(acc, part, lane, L, 0);
+            if (W.valid && part == 0) out[W.v] = float(sum);
+        } else {
+            if (W.valid) out[W.v] = float(acc.value());
+        }
     }
     if constexpr (!kExact) {
         unsigned tot = fallbacks;
@@ -774,6 +814,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pe
     __shared__ WaveLists L;
     const int item = xcd_item((int)blockIdx.x, (int)gridDim.x);
     if (!pe_forward_body<kExact, false, kEll>(A, item, L)) spill_push(A, item, threadIdx.x);
+}
+
+// kWaves waves per work item, each with its share of the sub-cells and lists of
+// its own (wide_blocks).
+template <bool kExact, bool kEll, int kWaves>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4))) void pe_forward_wide_kernel(
+    PeLaunch A) {
+    __shared__ SharedLists L[kWaves];
+    const int item = xcd_item((int)blockIdx.x, (int)gridDim.x);
+    if (!pe_forward_body<kExact, false, kEll, kWaves>(A, item, L[block_wave<kWaves>()]))
+        spill_push(A, item, threadIdx.x);
 }
 
 // Point weights at 3 waves per SIMD (the register cap costs no spills here;
@@ -825,11 +876,11 @@ __device__ __forceinline__ double tangent_term(const PeGeom& G, int d, const dou
 // Work item `item` (bar, tile) of the tangent: as pe_forward_body, with the
 // derivative summed beside the element.  Returns false, having written
 // nothing, when the candidates overflow L.
-template <bool kExact, class Lists>
+template <bool kExact, int kWaves = 1, class Lists>
 __device__ __forceinline__ bool pe_tangent_body(const PeLaunch& A, const PeTangent& TG, int item, Lists& L) {
     const PeGeom& G = A.geom;
     const GeomDesc& g = G.g;
-    const int lane = threadIdx.x;
+    const int lane = kWaves > 1 ? threadIdx.x & 63 : threadIdx.x, part = block_wave<kWaves>();
     const int n_tiles = A.tiles[0] * A.tiles[1] * A.tiles[2];
     const int d = item / n_tiles;
     const int tile = item % n_tiles;
@@ -839,7 +890,7 @@ __device__ __forceinline__ bool pe_tangent_body(const PeLaunch& A, const PeTange
     wave_setup(A, d, tile, lane, W);
     const int64_t o = (int64_t)d * g.n_vox + W.v;
     if (!(bd.mut > (double)0.01f)) {  // PESysMatGen.cu:1116, :1194
-        if (W.valid) {
+        if (W.valid && part == 0) {
             TG.d_out[o] = 0.0f;
             if (TG.a_out) TG.a_out[o] = 0.0f;
         }
@@ -847,14 +898,15 @@ __device__ __forceinline__ bool pe_tangent_body(const PeLaunch& A, const PeTange
     }
     int nb, nh;
     if (!build_candidates<kExact>(A, d, lane, W, L, nb, nh)) return false;
-    __syncthreads();
+    L.sync();
     using T = typename std::conditional<kExact, double, float>::type;
     KahanSum<T> acc;
     KahanSum<double> dacc;
+    const int per = (n_cells + kWaves - 1) / kWaves, c_begin = part * per, c_end = min(n_cells, c_begin + per);
     unsigned fallbacks = 0;
     const double* vbar = TG.v + g.n_layers;
     trace_cells<kExact, false>(
-        A, bd, d, 0, n_cells, W, lane, L, nb, nh, [](int) { return true; },
+        A, bd, d, c_begin, c_end, W, lane, L, nb, nh, [](int) { return true; },
         [&](int, const CellCtx& cc, const RecCands<Lists>& C) {
             bool near = false;
             if (W.valid) {
@@ -879,7 +931,14 @@ __device__ __forceinline__ bool pe_tangent_body(const PeLaunch& A, const PeTange
                 ++fallbacks;
             }
         });
-    if (W.valid) {
+    if constexpr (kWaves > 1) {
+        const double ds = block_sum<kWaves>(dacc, part, lane, L, 0);
+        const double as = TG.a_out ? block_sum<kWaves>(acc, part, lane, L, 1) : 0.0;
+        if (W.valid && part == 0) {
+            TG.d_out[o] = float(ds);
+            if (TG.a_out) TG.a_out[o] = float(as);
+        }
+    } else if (W.valid) {
         TG.d_out[o] = float(dacc.value());
         if (TG.a_out) TG.a_out[o] = float(acc.value());
     }
@@ -895,6 +954,14 @@ template <bool kExact>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void pe_tangent_kernel(PeLaunch A, PeTangent TG) {
     __shared__ WaveLists L;
     if (!pe_tangent_body<kExact>(A, TG, (int)blockIdx.x, L)) spill_push(A, (int)blockIdx.x, threadIdx.x);
+}
+
+template <bool kExact, int kWaves>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(3))) void pe_tangent_wide_kernel(
+    PeLaunch A, PeTangent TG) {
+    __shared__ SharedLists L[kWaves];
+    if (!pe_tangent_body<kExact, kWaves>(A, TG, (int)blockIdx.x, L[block_wave<kWaves>()]))
+        spill_push(A, (int)blockIdx.x, threadIdx.x);
 }
 
 template <bool kExact>
@@ -1304,6 +1371,21 @@ hipError_t spill_begin(const PeLaunch& A, int64_t blocks, hipStream_t stream, un
 
 }  // namespace
 
+// Blocks whose waves share an item's sub-cells (4 waves, or the 3 that the
+// tangent's registers let a SIMD hold), where one wave per item is at most two per
+// SIMD: bound by latency then, 1,024 items of 64 sub-cells 197 -> 117 us a call
+// (tangent kernel 217 -> 147 us), 2,048 items 306 -> 249 us (tangent 317 -> 271).
+// From 4,096 items on the waves' own candidate lists cost more than they gain (467
+// -> 486 us), and below 16 sub-cells there is little to share (16: 159 -> 112 us).
+// The count is of the whole detector: a range of its rows is summed alike.
+constexpr int kWideWaves = 4, kTangentWaves = 3;
+static void launch_forward_wide(const PeLaunch& A, bool exact, int64_t blocks, hipStream_t stream);
+static void launch_tangent_wide(const PeLaunch& A, const PeTangent& TG, bool exact, int64_t blocks, hipStream_t stream);
+static bool wide_blocks(const PeLaunch& A) {
+    const int64_t items = (int64_t)A.geom.g.n_det * A.tiles[0] * A.tiles[1] * A.tiles[2];
+    return items <= 2048 && A.sub[0] * A.sub[1] * A.sub[2] >= 4 * kWideWaves;
+}
+
 hipError_t launch_pe_tangent(const PeLaunch& A, const PeTangent& TG, bool exact, hipStream_t stream) {
     const int n_tiles = A.tiles[0] * A.tiles[1] * A.tiles[2];
     const int64_t blocks = (int64_t)n_tiles * A.geom.g.n_det;
@@ -1311,11 +1393,18 @@ hipError_t launch_pe_tangent(const PeLaunch& A, const PeTangent& TG, bool exact,
     unsigned sg = 0;
     hipError_t e = spill_begin(A, blocks, stream, sg);
     if (e != hipSuccess) return e;
+    const bool wide = wide_blocks(A);
     if (exact) {
-        hipLaunchKernelGGL(pe_tangent_kernel<true>, dim3((unsigned)blocks), dim3(64), 0, stream, A, TG);
+        if (wide)
+            launch_tangent_wide(A, TG, exact, blocks, stream);
+        else
+            hipLaunchKernelGGL(pe_tangent_kernel<true>, dim3((unsigned)blocks), dim3(64), 0, stream, A, TG);
         if (sg) hipLaunchKernelGGL(pe_tangent_spill_kernel<true>, dim3(sg), dim3(64), 0, stream, A, TG);
     } else {
-        hipLaunchKernelGGL(pe_tangent_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, stream, A, TG);
+        if (wide)
+            launch_tangent_wide(A, TG, exact, blocks, stream);
+        else
+            hipLaunchKernelGGL(pe_tangent_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, stream, A, TG);
         if (sg) hipLaunchKernelGGL(pe_tangent_spill_kernel<false>, dim3(sg), dim3(64), 0, stream, A, TG);
     }
     return hipGetLastError();
@@ -1386,15 +1475,26 @@ hipError_t launch_pe_forward_rows(const PeLaunch& A, bool exact, int bar0, int n
     unsigned sg = 0;
     hipError_t e = spill_begin(B, blocks, stream, sg);
     if (e != hipSuccess) return e;
+    const bool wide = wide_blocks(A);
+    const dim3 grid((unsigned)blocks), threads(64);
     if (exact) {
-        hipLaunchKernelGGL(pe_forward_kernel<true>, dim3((unsigned)blocks), dim3(64), 0, stream, B);
+        if (wide)
+            launch_forward_wide(B, exact, blocks, stream);
+        else
+            hipLaunchKernelGGL(pe_forward_kernel<true>, grid, threads, 0, stream, B);
         if (sg) hipLaunchKernelGGL((pe_forward_spill_kernel<true, false>), dim3(sg), dim3(64), 0, stream, B);
     } else if (A.ell) {
-        hipLaunchKernelGGL((pe_forward_kernel<false, true>), dim3((unsigned)blocks), dim3(64), 0, stream, B);
+        if (wide)
+            launch_forward_wide(B, exact, blocks, stream);
+        else
+            hipLaunchKernelGGL((pe_forward_kernel<false, true>), grid, threads, 0, stream, B);
         if (sg)
             hipLaunchKernelGGL((pe_forward_spill_kernel<false, false, true>), dim3(sg), dim3(64), 0, stream, B);
     } else {
-        hipLaunchKernelGGL(pe_forward_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, stream, B);
+        if (wide)
+            launch_forward_wide(B, exact, blocks, stream);
+        else
+            hipLaunchKernelGGL(pe_forward_kernel<false>, grid, threads, 0, stream, B);
         if (sg) hipLaunchKernelGGL((pe_forward_spill_kernel<false, false>), dim3(sg), dim3(64), 0, stream, B);
     }
     return hipGetLastError();
@@ -1506,6 +1606,25 @@ hipError_t launch_pe_backproject(const PeLaunch& A, bool exact, const float* y, 
     hipLaunchKernelGGL(sum_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, partial,
                        n, n_grp, n, (int64_t)1, x);
     return hipGetLastError();
+}
+
+static void launch_forward_wide(const PeLaunch& A, bool exact, int64_t blocks, hipStream_t stream) {
+    const dim3 grid((unsigned)blocks), threads(64 * kWideWaves);
+    if (exact)
+        hipLaunchKernelGGL((pe_forward_wide_kernel<true, true, kWideWaves>), grid, threads, 0, stream, A);
+    else if (A.ell)
+        hipLaunchKernelGGL((pe_forward_wide_kernel<false, true, kWideWaves>), grid, threads, 0, stream, A);
+    else
+        hipLaunchKernelGGL((pe_forward_wide_kernel<false, false, kWideWaves>), grid, threads, 0, stream, A);
+}
+
+static void launch_tangent_wide(const PeLaunch& A, const PeTangent& TG, bool exact, int64_t blocks,
+                                hipStream_t stream) {
+    const dim3 grid((unsigned)blocks), threads(64 * kTangentWaves);
+    if (exact)
+        hipLaunchKernelGGL((pe_tangent_wide_kernel<true, kTangentWaves>), grid, threads, 0, stream, A, TG);
+    else
+        hipLaunchKernelGGL((pe_tangent_wide_kernel<false, kTangentWaves>), grid, threads, 0, stream, A, TG);
 }
 
 }  // namespace smg

@@ -40,3 +40,30 @@ def test_pe_block_edges(smg_mod, oracle_mod, params_mod, layers, voxel, turn, su
             want = A.astype(np.float64) @ x.astype(np.float64)
             # FP64 sums of the same FP32 elements, rounded once
             assert np.all(np.abs(y - want) <= 1.2e-7 * np.abs(want))
+
+
+@pytest.mark.parametrize("n_bars,sub", [(81, (5, 3, 1)), (81, (4, 4, 1)), (81, (17, 1, 1)), (2048, (2, 4, 2)),
+                                        (2049, (2, 4, 2))])
+def test_pe_shared_items(smg_mod, oracle_mod, params_mod, n_bars, sub):
+    """Items whose sub-cells several waves share (few items, 16 sub-cells and
+    more), one item and one sub-cell either side of the rule, and a bar without
+    attenuation.  The tangent along the matrix's mu_pe: every element is
+    proportional to its bar's mu_pe, so its derivative is the element over it."""
+    p = _geometry(params_mod, 1, 0.5, 0.0) if n_bars == 81 else params_mod.large_detector()
+    if n_bars != 81:
+        params_mod.set_image(p, 5, 3, 3, 0.5, 0.5, 0.5)
+        p.det[0] = n_bars
+    p.det[7 + 12 * 5] = 0.0
+    o = oracle_mod.Oracle(p)
+    rows = np.array([0, 5, n_bars // 2, n_bars - 1], np.int32)
+    ref = o.pe_rows(rows, sub=sub)
+    with smg_mod.open_context(p) as ctx:
+        ctx.set_pe_subsamples(*sub)
+        dmu = np.zeros(ctx._n_layers + 2 * n_bars)
+        dmu[ctx._n_layers + n_bars:] = p.det[8:8 + 12 * n_bars:12]
+        for prec, tol in (("fp32", TOL_FP32), ("fp64", TOL_FP64)):
+            A, _ = ctx.pe_forward(0, prec)
+            assert_parity(A[rows].reshape(-1), ref.reshape(-1), tol, f"shared items {n_bars} {sub} {prec}")
+            dA, A2, _ = ctx.pe_tangent(dmu, 0, prec, with_matrix=True)
+            assert_parity(dA[rows].reshape(-1), ref.reshape(-1), tol, f"tangent {n_bars} {sub} {prec}")
+            assert_parity(A2[rows].reshape(-1), ref.reshape(-1), tol, f"tangent's matrix {n_bars} {sub} {prec}")
