@@ -103,9 +103,6 @@ __device__ bool below_window_all(const ScatterLaunch& A, double c_lo, const doub
     return cos(th) < c_lo - 1.1e-4;
 }
 
-__device__ __forceinline__ float readlane_f(float x, int lane) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
-}
 __device__ __forceinline__ double readlane_d(double x, int lane) {
     const unsigned long long u = (unsigned long long)__double_as_longlong(x);
     const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)u, lane);

@@ -599,28 +599,6 @@ SMG_FN float angle_f(float s, float c) {
     return c < 0.0f ? 3.14159265358979324f - r : r;
 }
 
-// Angle between u and w (vectors src -> a and a -> det), used for the polar
-// range.  FP64 follows the reference, acos of the clamped cosine
-// (scatter.cu:996-1013); FP32 uses atan2(|u x w|, u.w), which keeps its
-// precision at small angles where acos of a rounded cosine does not.
-template <class T>
-SMG_FN T cone_angle(const T u[3], const T w[3]) {
-    T dot = u[0] * w[0] + u[1] * w[1] + u[2] * w[2];
-    if constexpr (std::is_same<T, double>::value) {
-        T nu = sqrt(u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
-        T nw = sqrt(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
-        T c = dot / (nu * nw);
-        if (c > T(1)) c = T(1);
-        if (c < T(-1)) c = T(-1);
-        return acos(c);
-    } else {
-        T cx = u[1] * w[2] - u[2] * w[1];
-        T cy = u[2] * w[0] - u[0] * w[2];
-        T cz = u[0] * w[1] - u[1] * w[0];
-        return atan2(sqrt(cx * cx + cy * cy + cz * cz), dot);
-    }
-}
-
 // Per (scatter point, sub-cell) quantities shared by the lanes.
 struct ScatterCell {
     double qs[3];        // scatter point, world
