@@ -698,7 +698,7 @@ SMG_FN void ray_aux(double aux[8], double eff, double om, double l1, double l2, 
 // direction, an unturned bar's own chords take the world direction data, and
 // holes are met in coordinates relative to the sub-cell point (with direction
 // data per frame, per-axis eps flags and absolute hole coordinates the full-size
-// PE step took 169.8 ms instead of 131.3, a slice at 8x16x8 sub-cells 30.1
+// PE step took 169.8 ms instead of 128.2, a slice at 8x16x8 sub-cells 30.1
 // instead of 22.7).
 template <bool kEll, class Cands>
 SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const double ps[3], const CellCtx& cc,
@@ -738,9 +738,11 @@ SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const do
 
     // solid angle: largest of the three projected cell faces over 4 pi |D|^3
     // (PESysMatGen.cu:1223-1231)
-    const float om = tmax2(tmax2(float(cc.area[0]) * tabs(Db[0]), float(cc.area[1]) * tabs(Db[1])),
-                           float(cc.area[2]) * tabs(Db[2])) *
-                     (float(inv_dd * inv_dd * inv_dd) * float(1.0 / (4.0 * 3.14159265358979323846)));
+    // in FP64: the areas and the constant are the same for all rays, so their
+    // rounding would not average out in sums over the matrix
+    const double fx = unturned ? D[0] : cc.qs[0] - ps[0], fz = unturned ? D[2] : cc.qs[2] - ps[2];
+    const float om = float(tmax2(tmax2(cc.area[0] * tabs(fx), cc.area[1] * tabs(D[1])), cc.area[2] * tabs(fz)) *
+                           (inv_dd * inv_dd * (inv_dd * (1.0 / (4.0 * 3.14159265358979323846)))));
 
     double att = 0.0;
     // plate gate: a ray that does not cross a plate is blocked (PESysMatGen.cu:1240-1254)
@@ -860,7 +862,7 @@ SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const do
     att += (double(d1) - double(d2)) * bd.mut;
     const float eff = exp_neg<float>(att);
     const float ea = exp_neg<float>(double(la) * bd.mut);
-    const float absf = (1.0f - ea) * float(bd.pe_frac);
+    const float absf = float(double(1.0f - ea) * bd.pe_frac);
     if (aux) ray_aux(aux, eff, om, d1, d2, la, ea, dsq);
     return eff * om * absf;
 }
