@@ -170,6 +170,51 @@ void launch_chunk(const BmChunk& C, bool whole, hipStream_t stream) {
         hipLaunchKernelGGL((bitmap_kernel<kColl, false>), grid, dim3(256), 0, stream, C);
 }
 
+// Small bitmaps, in one launch without tables: a wave owns 64 consecutive words; at
+// step s lane l evaluates bit 64 s + l, and a ballot gives words 2s and 2s + 1.  A
+// lane keeps its row's terms until its k wraps into the next row.
+constexpr int kWordsPerRun = 64;                // one word per lane
+constexpr int64_t kBitsPerRun = 32 * kWordsPerRun;
+
+template <bool kColl>
+__global__ __launch_bounds__(256) void bitmap_walk_kernel(BitmapLaunch A) {
+    const int lane = threadIdx.x & 63;
+    const int64_t n = A.n_det;
+    const int64_t total = bm_total_bits(kColl, n, A.n_holes);
+    const int64_t n_runs = (A.n_words + kWordsPerRun - 1) / kWordsPerRun;
+    const int64_t stride = ((int64_t)gridDim.x * blockDim.x) >> 6;
+    // the run index is the same for the 64 lanes of a wave, so every ballot
+    // below sees the whole wave
+    for (int64_t run = (((int64_t)blockIdx.x * blockDim.x) + threadIdx.x) >> 6; run < n_runs;
+         run += stride) {
+        int64_t b = run * kBitsPerRun + lane;
+        BitRow r{};
+        int k = 0;
+        if (b < total) {
+            bm_row_of_bit(kColl, b, n, r, k);
+            bm_row_setup(kColl, A.spheres_d, A.holes_d, r);
+        }
+        uint32_t word = 0;
+        for (int s = 0; s < 32; ++s) {
+            const bool bit = b < total && bm_bit(kColl, r, A.spheres_d, A.holes_d, k);
+            const uint64_t m = __ballot(bit);
+            if (lane == 2 * s) word = (uint32_t)m;
+            if (lane == 2 * s + 1) word = (uint32_t)(m >> 32);
+            b += 64;
+            k += 64;
+            if (b < total && k >= n) {
+                do {
+                    k -= (int)n;
+                    bm_next_row(kColl, n, r);
+                } while (k >= n);
+                bm_row_setup(kColl, A.spheres_d, A.holes_d, r);
+            }
+        }
+        const int64_t w = run * kWordsPerRun + lane;
+        if (w < A.n_words) A.words[w] = word;
+    }
+}
+
 // Chunk sizes: the tables stay within 2^23 entries each (128 MB of directions,
 // 168 MB of rows' terms), or one run of bars and one block of origins.
 struct BmPlan {
@@ -186,9 +231,17 @@ BmPlan bitmap_plan(bool coll, int64_t n, int64_t n_org) {
 
 }  // namespace
 
+// Without tables where their launches and scratch cost more than 67 instructions a
+// bit (calls of both kernels, us): crystal 300 bars (13.5M bits) 51 by the walk,
+// 53 by tables, 350 bars (21M) 68 and 61; collimator with 400 holes, 128 bars (6.6M)
+// 31 and 33, 192 bars (15M) 43 and 37.
+static bool bitmap_by_walk(bool collimator, int64_t n, int64_t n_org) {
+    return bm_total_bits(collimator, n, n_org) <= (int64_t)1 << (collimator ? 23 : 24);
+}
+
 size_t bitmap_scratch_bytes(bool collimator, int n_det, int n_holes) {
     const int n_org = collimator ? n_holes : n_det;
-    if (n_det <= 0 || n_org <= 0) return 0;
+    if (n_det <= 0 || n_org <= 0 || bitmap_by_walk(collimator, n_det, n_org)) return 0;
     const BmPlan p = bitmap_plan(collimator, n_det, n_org);
     return (size_t)p.n_dirs * sizeof(BmDir) + (size_t)p.n_rows * sizeof(BmRows);
 }
@@ -196,6 +249,15 @@ size_t bitmap_scratch_bytes(bool collimator, int n_det, int n_holes) {
 hipError_t launch_bitmap(const BitmapLaunch& A, bool collimator, hipStream_t stream) {
     if (A.n_words <= 0) return hipSuccess;
     const int n = A.n_det, n_org = collimator ? A.n_holes : n;
+    if (bitmap_by_walk(collimator, n, n_org)) {
+        const int64_t n_runs = (A.n_words + kWordsPerRun - 1) / kWordsPerRun;
+        const dim3 grid((unsigned)((n_runs + 3) / 4));
+        if (collimator)
+            hipLaunchKernelGGL(bitmap_walk_kernel<true>, grid, dim3(256), 0, stream, A);
+        else
+            hipLaunchKernelGGL(bitmap_walk_kernel<false>, grid, dim3(256), 0, stream, A);
+        return hipGetLastError();
+    }
     const BmPlan p = bitmap_plan(collimator, n, n_org);
     // rows of whole words are stored; others are OR-ed into cleared words (2,000
     // bars: 2.9 ms; 2,048: 2.2 ms)

@@ -284,7 +284,8 @@ smg_status ensure_bitmap(smg_ctx* c, bool collimator) {
     B.n_words = n_words;
     B.n_det = N;
     B.n_holes = hg.n_holes_l0;
-    SMG_HIP(c, c->bm_scratch.reserve(bitmap_scratch_bytes(collimator, N, hg.n_holes_l0)));
+    if (size_t scratch = bitmap_scratch_bytes(collimator, N, hg.n_holes_l0))
+        SMG_HIP(c, c->bm_scratch.reserve(scratch));
     B.scratch = c->bm_scratch.ptr;
     SMG_HIP(c, launch_bitmap(B, collimator, c->stream));
     SMG_HIP(c, hipStreamSynchronize(c->stream));
