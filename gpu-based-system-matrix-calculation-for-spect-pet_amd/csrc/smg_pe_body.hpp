@@ -700,7 +700,12 @@ SMG_FN void ray_aux(double aux[8], double eff, double om, double l1, double l2, 
 // data per frame, per-axis eps flags and absolute hole coordinates the full-size
 // PE step took 169.8 ms instead of 128.2, a slice at 8x16x8 sub-cells 30.1
 // instead of 22.7).
-template <bool kEll, class Cands>
+// kPinned: the rays of the tangent and the adjoint.  Their FP64 sums of FP32 terms
+// show a change of rounding at 1e-8 where the matrix hides it in its last FP32
+// digit, so these rays keep the form that rounds the solid angle, the frame of the
+// own bar and mu_pe / mu in FP32, and its eps flags (gradient over 2,048 bars 3.74
+// ms, 3.47 with the matrix's form).
+template <bool kEll, bool kPinned, class Cands>
 SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const double ps[3], const CellCtx& cc,
                              const Cands& C, bool& near, double* dl_layer, double* aux, float* keep,
                              int keep_stride, const double* tan_bar, double* tan_att) {
@@ -711,20 +716,30 @@ SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const do
     const double dsq = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
     const double inv_dd = rsq_fast(dsq), dd = dsq * inv_dd;
     SegDir<float> sw;
-    sw.ns = 0;
-    sw.len = float(dd);
+    bool thin = false;
+    double dy = D[1];
+    float tol_w = 0.0f;
+    if constexpr (kPinned) {
+        tol_w = 4.0f * kUnit<float> * (tabs(float(D[0])) + tabs(float(D[1])) + tabs(float(D[2])));
+        segdir_init<float>(sw, float(D[0]), float(D[1]), float(D[2]), tol_w, near);
+        if (!(tabs(dy) > 1e-300)) dy = 1e-300;
+    } else {
+        sw.ns = 0;
+        sw.len = float(dd);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        sw.D[k] = float(D[k]);
-        sw.inv[k] = sw.len * trcp(sw.D[k]);
-        sw.small[k] = 0;
+        for (int k = 0; k < 3; ++k) {
+            sw.D[k] = float(D[k]);
+            sw.inv[k] = sw.len * trcp(sw.D[k]);
+            sw.small[k] = 0;
+        }
+        sw.tol_d = 12.0f * kUnit<float> * sw.len;  // rounding of a component of D
+        tol_w = sw.tol_d;
+        const float dmin = tmin2(tmin2(tabs(sw.D[0]), tabs(sw.D[1])), tabs(sw.D[2]));
+        thin = dmin < kSlabEps<float> + sw.tol_d;
+        const bool flat = tabs(sw.D[1]) < kSlabEps<float> + sw.tol_d;
+        near |= flat;
+        dy = flat ? 1.0 : D[1];
     }
-    sw.tol_d = 12.0f * kUnit<float> * sw.len;  // rounding of a component of D
-    const float dmin = tmin2(tmin2(tabs(sw.D[0]), tabs(sw.D[1])), tabs(sw.D[2]));
-    const bool thin = dmin < kSlabEps<float> + sw.tol_d;
-    const bool flat = tabs(sw.D[1]) < kSlabEps<float> + sw.tol_d;
-    near |= flat;
-    const double dy = flat ? 1.0 : D[1];
 
     // direction in the frame of bar d
     float Db[3] = {sw.D[0], sw.D[1], sw.D[2]}, ib[3] = {tabs(sw.inv[0]), tabs(sw.inv[1]), tabs(sw.inv[2])};
@@ -741,7 +756,17 @@ SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const do
     // in FP64: the areas and the constant are the same for all rays, so their
     // rounding would not average out in sums over the matrix
     const double fx = unturned ? D[0] : cc.qs[0] - ps[0], fz = unturned ? D[2] : cc.qs[2] - ps[2];
-    const float om = float(tmax2(tmax2(cc.area[0] * tabs(fx), cc.area[1] * tabs(D[1])), cc.area[2] * tabs(fz)) *
+    float om;
+    if constexpr (kPinned) {
+        const float cb = float(bd.cb), sb = float(bd.sb);
+        const float Dx = float(D[0]), Dy = float(D[1]), Dz = float(D[2]), dsqf = float(dsq);
+        const float rc = trcp(float(4.0 * 3.14159265358979323846) * dsqf * tsqrt(dsqf));
+        const float omx = float(cc.area[0]) * tabs(Dx * cb - Dz * sb);
+        const float omz = float(cc.area[2]) * tabs(Dx * sb + Dz * cb);
+        const float omy = float(cc.area[1]) * tabs(Dy);
+        om = tmax2(tmax2(omx, omy), omz) * rc;
+    } else
+        om = float(tmax2(tmax2(cc.area[0] * tabs(fx), cc.area[1] * tabs(D[1])), cc.area[2] * tabs(fz)) *
                            (inv_dd * inv_dd * (inv_dd * (1.0 / (4.0 * 3.14159265358979323846)))));
 
     double att = 0.0;
@@ -811,11 +836,11 @@ SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const do
             if (keep && j < kKeepChords) keep[j * keep_stride] = 0.0f;
             continue;
         }
-        near |= thin;
+        if constexpr (!kPinned) near |= thin;
         float l;
         double mu_k;
         bool fast = false;
-        if constexpr (Cands::kFastFaces) fast = C.fast(j);
+        if constexpr (Cands::kFastFaces) fast = C.fast(j) && (!kPinned || sw.ns == 0);
         if (fast) {
             if constexpr (Cands::kFastFaces) {
                 mu_k = double(C.mu(j));
@@ -824,7 +849,7 @@ SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const do
         } else {
             const int k = C.bar(j);
             mu_k = G.bars_d[k].mut;
-            l = other_bar_chord<float>(G, k, p, D, dd, inv_dd, cc.q, sw, sw.tol_d, near);
+            l = other_bar_chord<float>(G, k, p, D, dd, inv_dd, cc.q, sw, tol_w, near);
         }
         if (keep && j < kKeepChords) keep[j * keep_stride] = l;
         att += double(l) * mu_k;
@@ -850,6 +875,28 @@ SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const do
     const Bar<float>& bf = G.bars_f[d];
     const float hb[3] = {0.5f * bf.w, 0.5f * bf.t, 0.5f * bf.h};
     float d1 = INFINITY, d2 = INFINITY;
+    if constexpr (kPinned) {
+        SegDir<float> ss;
+        const float Ds[3] = {float(cc.qs[0] - ps[0]), float(cc.qs[1] - ps[1]), float(cc.qs[2] - ps[2])};
+        const float tds = 4.0f * kUnit<float> * (tabs(Ds[0]) + tabs(Ds[1]) + tabs(Ds[2]));
+        segdir_init<float>(ss, Ds[0], Ds[1], Ds[2], tds, near);
+        near |= ss.ns == 3;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if (ss.small[k]) continue;
+            const float ia = tabs(ss.inv[k]), qk = float(cc.qs[k]);
+            const float face = ss.D[k] > 0.0f ? qk + hb[k] : hb[k] - qk;
+            d1 = tmin2(d1, face * ia);
+            d2 = tmin2(d2, cc.hc[k] * ia);
+        }
+        const bool level = g_lt(tabs(ss.D[1]), float(kInsideDy), ss.tol_d, near);
+        near |= (ss.len - d1 < 0.01f) | (d2 < 0.01f) | level;
+        const float la = 2.0f * d2;
+        att += (double(d1) - double(d2)) * bd.mut;
+        const float eff = exp_neg<float>(att), ea = exp_neg<float>(double(la) * bd.mut);
+        if (aux) ray_aux(aux, eff, om, d1, d2, la, ea, dsq);
+        return eff * om * ((1.0f - ea) * float(bd.pe_frac));
+    }
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const float qk = float(cc.qs[k]);
@@ -982,13 +1029,13 @@ SMG_FN double pe_cell_ray_f64(const PeGeom& G, int d, const double p[3], const d
 // tan_bar (optional): a direction over the bars' mu_total; *tan_att then
 // receives sum_k tan_bar[k] l_k over the other bars on the ray (the tangent of
 // their attenuation).
-template <class T, bool kEll, class Cands>
+template <class T, bool kEll, bool kPinned = false, class Cands>
 SMG_FN T pe_cell_ray(const PeGeom& G, int d, const double p[3], const double ps[3],
                      const CellCtx& cc, const Cands& C, bool& near, double* dl_layer = nullptr,
                      double* aux = nullptr, float* keep = nullptr, int keep_stride = 0,
                      const double* tan_bar = nullptr, double* tan_att = nullptr) {
     if constexpr (std::is_same<T, float>::value)
-        return pe_cell_ray_f32<kEll>(G, d, p, ps, cc, C, near, dl_layer, aux, keep, keep_stride, tan_bar, tan_att);
+        return pe_cell_ray_f32<kEll, kPinned>(G, d, p, ps, cc, C, near, dl_layer, aux, keep, keep_stride, tan_bar, tan_att);
     else
         return pe_cell_ray_f64<kEll>(G, d, p, ps, cc, C, dl_layer, aux, tan_bar, tan_att);
 }
