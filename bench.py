@@ -46,17 +46,17 @@ TRAFFIC_BYTES = 1.154e9
 # VALUBusy, lane utilisation and mean resident waves per SIMD (of the 4 the
 # kernel's registers and LDS allow)
 EXEC_SOURCE = "profiles/pe_forward_instruction_mix_fp32_fp64_64x64x32_2048bars.md"
-EXEC_FLOPS_PER_RAY = 250.9 + 182.1
-VALU_INSTS_PER_RAY = 819.6
-TRANS_INSTS_PER_RAY = 23.0 + 4.8
-VALU_BUSY = 0.841
+EXEC_FLOPS_PER_RAY = 149.4 + 141.8
+VALU_INSTS_PER_RAY = 553.9
+TRANS_INSTS_PER_RAY = 12.2 + 4.9
+VALU_BUSY = 0.822
 # the same instructions by issue cost (bin/valu_issue_probe on this GPU: 4 cycles
 # per wave instruction for FP32/FP64 arithmetic, integer and conversion, ~2 for
 # compares, selects, min/max and moves, ~8 for a transcendental)
-VALU_4CYCLE_INSTS_PER_RAY = 441.7
-VALU_2CYCLE_INSTS_PER_RAY = 377.9
+VALU_4CYCLE_INSTS_PER_RAY = 280.3
+VALU_2CYCLE_INSTS_PER_RAY = 273.6
 VALU_CYCLE_SOURCE = "profiles/valu_issue_rates_gfx950.md"
-LANE_UTILISATION = 0.738
+LANE_UTILISATION = 0.816
 WAVES_PER_SIMD = 3.73
 MAX_WAVES_PER_SIMD = 4
 # unpacked FP32 (= FP64) vector FMA peak, the transcendental peak (a quarter of
