@@ -754,8 +754,14 @@ SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const do
     // solid angle: largest of the three projected cell faces over 4 pi |D|^3
     // (PESysMatGen.cu:1223-1231)
     // in FP64: the areas and the constant are the same for all rays, so their
-    // rounding would not average out in sums over the matrix
-    const double fx = unturned ? D[0] : cc.qs[0] - ps[0], fz = unturned ? D[2] : cc.qs[2] - ps[2];
+    // rounding would not average out in sums over the matrix.  The reference
+    // projects a turned bar's x and z faces with the world direction turned by
+    // +beta, not by the -beta of the bar's frame.
+    double fx = D[0], fz = D[2];
+    if (!unturned) {
+        fx = D[0] * bd.cb - D[2] * bd.sb;
+        fz = D[0] * bd.sb + D[2] * bd.cb;
+    }
     float om;
     if constexpr (kPinned) {
         const float cb = float(bd.cb), sb = float(bd.sb);
