@@ -276,7 +276,8 @@ struct ScatterPhys {
     double mupe, muc;      // bar d
     const MuTables* tab = nullptr;  // mu(E) tables, or power laws
     const MuTablesF* tabf = nullptr;  // their FP32 form (FP32 term), or none
-    const double* knt = nullptr;    // KN prefix table (FP32 path), or the node loop
+    const double* knt = nullptr;    // KN prefix table (kn_sum_table), or the node loop: without
+                                    // kTab only, which no kernel uses
     double c_rej = -2.0;            // cos(theta) below this is outside the window for
                                     // sure (window_reject_cos with the path's margin)
     // the kernels' tables (scatter_term with kTab set)
@@ -374,7 +375,8 @@ SMG_FN T kn_sum(T lo, T hi, T alpha, bool& near) {
     }
 }
 
-// KN rectangle sums from a prefix table.  The reference's sum has nodes
+// KN rectangle sums from a prefix table, which the host tests use: the kernels
+// take the polynomials below.  The reference's sum has nodes
 // lo + i step, i = 0..n; with lo = phi + k0 step (0 <= phi < step) it is
 // P(phi, k0 + n) - P(phi, k0 - 1), P(phi, k) = sum_{i <= k} g(phi + i step),
 // g(t) = KN(cos t) sin t step.  The table holds P in FP64 for kKnPhase + 1
@@ -638,9 +640,10 @@ SMG_FN bool below_window(const ScatterPhys& ph, const double p[3], const Scatter
 
 // One (voxel, scatter point, sub-cell) term.  wgt is the weight of the
 // scatter point for this voxel.  Returns 0 for terms outside the 2-sigma
-// energy window (scatter.cu:1263-1269).  kTab: with the kernels' tables (the KN
-// prefix polynomials; in FP32 also the row's window probability).
-template <class T, bool kTab = false>
+// energy window (scatter.cu:1263-1269).  kTab: with the kernels' KN prefix
+// polynomials, the FP32 pre-test of the window made by the caller; kWin (FP32):
+// the row's window probability from its table, else evaluated here.
+template <class T, bool kTab = false, bool kWin = kTab && std::is_same<T, float>::value>
 SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[3],
                       const ScatterCell& sc, T wgt, bool& near) {
     // Cone angle at the scatter point (scatter.cu:1254), scattered energy
@@ -700,7 +703,7 @@ SMG_FN T scatter_term(const ScatterPhys& ph, const double p[3], const double ps[
     // window from g and one reciprocal, the FP64 path as the reference does
     double ep = 0.0, resp, z1 = 0.0, z2 = 0.0;
     T pe_win;
-    if constexpr (kTab && std::is_same<T, float>::value) {
+    if constexpr (kWin) {
         if (omc >= ph.omc_lo || omc <= ph.omc_hi) return T(0);  // scatter.cu:1263-1269
         pe_win = win_table_value(ph, omc);
     } else {
