@@ -365,9 +365,12 @@ hipError_t scatter_row_cuts(smg_ctx* c, ScatterLaunch& A, bool exact, const int*
         // with windows relative to the resolution, the widest) sets the intervals
         double lo = INFINITY, hi = 0.0;
         for (size_t r = 0; r < rows; ++r) {
-            const double res = c->hg.bars_d[rows_h ? rows_h[r] : (int)r].res;
-            lo = std::min(lo, res);
-            hi = std::max(hi, res);
+            // bars without attenuation have no terms (scatter.cu:1226-1228): their
+            // resolution does not matter
+            const Bar<double>& b = c->hg.bars_d[rows_h ? rows_h[r] : (int)r];
+            if (!(b.mut > (double)0.01f)) continue;
+            lo = std::min(lo, b.res);
+            hi = std::max(hi, b.res);
         }
         int n[2];
         for (int i = 0; i < 2; ++i) {
@@ -379,7 +382,7 @@ hipError_t scatter_row_cuts(smg_ctx* c, ScatterLaunch& A, bool exact, const int*
             ph.res = res;
             n[i] = win_intervals(ph, window_reject_cos(ph, 0.0));
         }
-        A.win_n = n[0] > 0 && n[1] > 0 ? std::max(n[0], n[1]) : 0;
+        A.win_n = lo <= hi && n[0] > 0 && n[1] > 0 ? std::max(n[0], n[1]) : 0;
     }
     if (A.win_n > 0) {
         e = c->sc_win_rows.reserve(rows);

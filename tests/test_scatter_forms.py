@@ -65,6 +65,31 @@ def test_lane_forms(forms_lib, oracle_mod, params_mod, kind, variant, sub, windo
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["crystal", "collimator", "grid", "crystal_grid"])
+def test_gpu_bar_without_attenuation(smg_mod, params_mod, kind):
+    """A bar without attenuation has no terms, so its resolution does not change how
+    the other rows are formed."""
+    out = []
+    for res in (0.1, 0.0):
+        p = params_mod.config(1)
+        params_mod.set_image(p, 16, 16, 2, 2.0, 2.0, 2.0)
+        p.det[12 * 5 + 7:12 * 5 + 11] = [0.0, 0.0, 0.0, res]
+        pe = np.random.default_rng(5).uniform(0, 1e-9, (p.n_det, p.n_vox)).astype(np.float32)
+        with smg_mod.open_context(p) as ctx:
+            if kind == "crystal":
+                got = ctx.scatter_crystal(pe, 0, "fp32")[0]
+            elif kind == "collimator":
+                got = ctx.scatter_collimator(0, "combined", "fp32")[0]
+            elif kind == "grid":
+                got = ctx.scatter_collimator_grid(4.0, 0, "fp32")[0]
+            else:
+                got = ctx.scatter_crystal_grid((2, 2, 2), np.array([3, 5, 9]), 0, "fp32")[0]
+        out.append(got)
+    assert (out[0] > 0).any()
+    assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("window,res", [(NARROW, 0.1), (SHARP, 0.005), (WIDE, 0.1)])
 @pytest.mark.parametrize("kind", ["crystal", "collimator", "grid"])
 def test_gpu_forms(smg_mod, params_mod, window, res, kind):
