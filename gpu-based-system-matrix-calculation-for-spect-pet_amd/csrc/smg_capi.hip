@@ -352,8 +352,8 @@ hipError_t kn_table(smg_ctx* c, ScatterLaunch& A) {
 
 // Energy-window cut of each output row of a scatter launch (A.row_cut) and, for
 // FP32 launches, the rows' window tables (A.win_rows, A.win_tab) with as many
-// intervals as the sharpest row needs, on the context's stream ahead of the pair
-// terms and scatter kernels.  rows_h: the launch's rows on the host, or all bars.
+// intervals as any of them needs, on the context's stream ahead of the pair terms
+// and scatter kernels.  rows_h: the launch's rows on the host, or all bars.
 hipError_t scatter_row_cuts(smg_ctx* c, ScatterLaunch& A, bool exact, const int* rows_h) {
     const size_t rows = (size_t)(A.rows ? A.n_rows : A.geom.g.n_det);
     hipError_t e = c->sc_row_cut.reserve(rows > 0 ? rows : 1);
@@ -361,28 +361,20 @@ hipError_t scatter_row_cuts(smg_ctx* c, ScatterLaunch& A, bool exact, const int*
     A.row_cut = c->sc_row_cut.ptr;
     A.win_n = 0;
     if (!exact && rows > 0) {
-        // a row's table depends on its resolution only; the sharpest row (and,
-        // with windows relative to the resolution, the widest) sets the intervals
+        // a row's table depends on its resolution only; bars without attenuation
+        // have no terms (scatter.cu:1226-1228), so theirs does not matter
         double lo = INFINITY, hi = 0.0;
         for (size_t r = 0; r < rows; ++r) {
-            // bars without attenuation have no terms (scatter.cu:1226-1228): their
-            // resolution does not matter
             const Bar<double>& b = c->hg.bars_d[rows_h ? rows_h[r] : (int)r];
             if (!(b.mut > (double)0.01f)) continue;
             lo = std::min(lo, b.res);
             hi = std::max(hi, b.res);
         }
-        int n[2];
-        for (int i = 0; i < 2; ++i) {
-            const double res = i ? hi : lo;
-            ScatterPhys ph;
-            ph.e0 = A.e0;
-            ph.lo = A.same_window ? A.win_lo : (1 - res / 2.0) * A.e0;
-            ph.hi = A.same_window ? A.win_hi : (1 + res / 2.0) * A.e0;
-            ph.res = res;
-            n[i] = win_intervals(ph, window_reject_cos(ph, 0.0));
-        }
-        A.win_n = lo <= hi && n[0] > 0 && n[1] > 0 ? std::max(n[0], n[1]) : 0;
+        ScatterPhys ph;
+        ph.e0 = A.e0;
+        ph.lo = A.win_lo;
+        ph.hi = A.win_hi;
+        if (lo <= hi) A.win_n = win_intervals_rows(ph, A.same_window, lo, hi);
     }
     if (A.win_n > 0) {
         e = c->sc_win_rows.reserve(rows);

@@ -556,10 +556,12 @@ SMG_FN float win_table_value(const ScatterPhys& ph, double omc) {
     const float* c = ph.win + 4 * i;
     return ((c[3] * t + c[2]) * t + c[1]) * t + c[0];
 }
-// Intervals a row needs for kWinStep (host: the launch takes the largest over its
-// rows), or 0 when kWinMax do not do (a resolution below ~1%) or the upper cut is
-// not monotonic (a resolution above 78%): the FP32 term then evaluates the
-// probability directly.
+// Intervals a row needs for kWinStep, or 0 when kWinMax do not do or the upper cut
+// is not monotonic (a resolution above 78%): the FP32 term then evaluates the
+// probability directly.  The bound takes the steepest slope of z over the whole
+// domain, so what does not do depends on the window's width too: a window of +-10%
+// has a table from 1% resolution up, 140.5 keV with 90-160 keV from 8%, 511 keV
+// with 350-650 keV from 5%, 511 keV with 250-650 keV at none.
 inline int win_intervals(const ScatterPhys& ph, double cut) {
     if (!(ph.res * (2.0 / kFwhm) < 0.66) || !(ph.res > 0.0) || !(ph.e0 > 0.0)) return 0;
     ScatterPhys q = ph;
@@ -579,6 +581,30 @@ inline int win_intervals(const ScatterPhys& ph, double cut) {
     for (int n = kWinMin; n <= kWinMax; n *= 2)
         if (need <= n) return n;
     return 0;
+}
+
+// Intervals of a launch with rows of resolutions res_lo to res_hi (ph: the window,
+// or with same = false each row's own, E0 (1 -+ res / 2)): the largest need, which
+// is not monotonic in the resolution (per-bar windows at 140.5 keV: 128 at 10% and
+// 77%, 256 at 30%), over steps of at most 1.25; 0 when one of them has no table.
+inline int win_intervals_rows(ScatterPhys ph, bool same, double res_lo, double res_hi) {
+    const auto need = [&](double res) {
+        ph.res = res;
+        if (!same) {
+            ph.lo = (1 - res / 2.0) * ph.e0;
+            ph.hi = (1 + res / 2.0) * ph.e0;
+        }
+        return win_intervals(ph, window_reject_cos(ph, 0.0));
+    };
+    int n = need(res_lo);
+    if (n == 0 || !(res_hi > res_lo)) return n;
+    const int steps = (int)std::ceil(std::log(res_hi / res_lo) / std::log(1.25));
+    for (int i = steps; i > 0; --i) {  // from the other end
+        const int k = need(i == steps ? res_hi : res_lo * std::pow(res_hi / res_lo, (double)i / steps));
+        if (k == 0) return 0;
+        n = k > n ? k : n;
+    }
+    return n;
 }
 
 // atan2(s, c) for s >= 0, in [0, pi]: the smaller over the larger of s and |c|

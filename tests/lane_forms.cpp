@@ -137,3 +137,25 @@ long form_scatter_pairs(const float* coll, const float* det, const float* img, c
 }
 
 }  // extern "C"
+
+extern "C" {
+
+// Intervals of the window tables: one row, and a launch with rows of resolutions
+// res_lo to res_hi (same = 0: each row's own window).
+int form_row_intervals(double e0, double lo, double hi, double res) {
+    ScatterPhys P;
+    P.e0 = e0;
+    P.lo = lo;
+    P.hi = hi;
+    P.res = res;
+    return win_intervals(P, window_reject_cos(P, 0.0));
+}
+int form_launch_intervals(double e0, double lo, double hi, int same, double res_lo, double res_hi) {
+    ScatterPhys P;
+    P.e0 = e0;
+    P.lo = lo;
+    P.hi = hi;
+    return win_intervals_rows(P, same != 0, res_lo, res_hi);
+}
+
+}  // extern "C"

@@ -38,6 +38,8 @@ def forms_lib():
     up = np.ctypeslib.ndpointer(np.uint32, flags="C")
     L.form_scatter_pairs.restype = C.c_long
     L.form_scatter_pairs.argtypes = [fp] * 5 + [up] + [C.c_int] * 7 + [ip, ip, C.c_int, dp]
+    L.form_row_intervals.argtypes = [C.c_double] * 4
+    L.form_launch_intervals.argtypes = [C.c_double] * 3 + [C.c_int] + [C.c_double] * 2
     return L
 
 
@@ -62,6 +64,23 @@ def test_lane_forms(forms_lib, oracle_mod, params_mod, kind, variant, sub, windo
            else o.collimator_scatter_pairs(bm, d, v, variant=variant, sub=sub))
     assert (ref > 0).any() and fb >= 0
     assert_parity(out, ref, TOL_FP32 if form else TOL_FP64, f"form {form} kind={kind} res={res} fallbacks={fb}")
+
+
+@pytest.mark.parametrize("e0,lo,hi,same", [(140.5, 0, 0, 0), (511.0, 0, 0, 0), (140.5, 126.45, 154.55, 1),
+                                           (364.0, 200.0, 300.0, 1), (511.0, 350.0, 650.0, 1)])
+@pytest.mark.parametrize("res_lo,res_hi", [(0.1, 0.77), (0.09, 0.11), (0.05, 0.05), (0.012, 0.5)])
+def test_launch_intervals(forms_lib, e0, lo, hi, same, res_lo, res_hi):
+    """A launch's window tables have the intervals that each of its rows needs
+    (kWinStep), and no tables where a row has none; the need between the steps of
+    1.25 in the resolution is within one doubling only next to a step."""
+    n = forms_lib.form_launch_intervals(e0, lo, hi, same, res_lo, res_hi)
+    ends = []
+    for r in np.geomspace(res_lo, res_hi, 40):
+        a, b = (lo, hi) if same else ((1 - r / 2) * e0, (1 + r / 2) * e0)
+        ends.append(forms_lib.form_row_intervals(e0, a, b, r))
+    assert (n == 0) == (min(ends) == 0)
+    if n:
+        assert n == max(ends)
 
 
 @pytest.mark.gpu
