@@ -355,7 +355,7 @@ hipError_t kn_table(smg_ctx* c, ScatterLaunch& A) {
 // intervals as any of them needs, on the context's stream ahead of the pair terms
 // and scatter kernels.  rows_h: the launch's rows on the host, or all bars.
 hipError_t scatter_row_cuts(smg_ctx* c, ScatterLaunch& A, bool exact, const int* rows_h) {
-    const size_t rows = (size_t)(A.rows ? A.n_rows : A.geom.g.n_det);
+    const size_t rows = (size_t)A.n_rows;
     hipError_t e = c->sc_row_cut.reserve(rows > 0 ? rows : 1);
     if (e != hipSuccess) return e;
     A.row_cut = c->sc_row_cut.ptr;
@@ -449,6 +449,11 @@ smg_status scatter_prep(smg_ctx* c) {
     return SMG_OK;
 }
 
+// Pair records of a bar-centre or hole-centre launch, at most (1.9 GB): a detector
+// of 2,048 bars takes 4 sub-cells in one launch; with more, rows go in chunks, so the
+// memory does not grow with bars x points x sub-cells.
+constexpr int64_t kPairRecords = (int64_t)1 << 24;
+
 // Enqueues one scatter matrix (crystal scatter driven by the device PE block
 // pe, or collimator scatter of `variant`) into the device block out, added to
 // it when accumulate; no synchronisation.  Adds its terms to *rays.
@@ -467,9 +472,11 @@ smg_status scatter_launch(smg_ctx* c, bool collimator, int rotation, int variant
     A.bitmap = collimator ? c->bm_coll.ptr : c->bm_crystal.ptr;
     A.pe = collimator ? nullptr : pe;
     const int ncell = c->sc_sub[0] * c->sc_sub[1] * c->sc_sub[2];
-    SMG_HIP(c, c->pair.reserve((size_t)g.n_det * (size_t)(A.n_pts > 0 ? A.n_pts : 1) * ncell));
+    // pair records of as many rows at a time as kPairRecords hold (at least one)
+    const int64_t row_recs = (int64_t)std::max(A.n_pts, 1) * ncell;
+    const int chunk = (int)std::min<int64_t>(g.n_det, std::max<int64_t>(1, kPairRecords / row_recs));
+    SMG_HIP(c, c->pair.reserve((size_t)chunk * (size_t)row_recs));
     A.pair = c->pair.ptr;
-    A.dst = out;
     A.counters = c->counters.ptr;
     double phi = (double)rotation * g.dphi;
     A.cphi = std::cos(phi);
@@ -490,13 +497,25 @@ smg_status scatter_launch(smg_ctx* c, bool collimator, int rotation, int variant
     A.w1 = nullptr;
     A.accumulate = accumulate ? 1 : 0;
     A.rows = nullptr;
-    A.n_rows = 0;
+    A.n_rows = g.n_det;
+    A.row0 = 0;
     A.pts_per_bar = 1;
     A.pt_bar0 = 0;
     SMG_HIP(c, scatter_row_cuts(c, A, prec == SMG_PREC_FP64, nullptr));
-    SMG_HIP(c, launch_pair_terms(A, c->stream));
-    SMG_HIP(c, scatter_partials(c, A));
-    SMG_HIP(c, launch_scatter(A, prec == SMG_PREC_FP64, c->stream));
+    const ScatterLaunch all = A;
+    for (int r0 = 0; r0 < g.n_det; r0 += chunk) {
+        A.row0 = r0;
+        A.n_rows = std::min(chunk, g.n_det - r0);
+        A.dst = out + (int64_t)r0 * g.n_vox;
+        A.row_cut = all.row_cut + r0;
+        if (A.win_n > 0) {
+            A.win_rows = all.win_rows + r0;
+            A.win_tab = all.win_tab + (int64_t)r0 * A.win_n * 4;
+        }
+        SMG_HIP(c, launch_pair_terms(A, c->stream));
+        SMG_HIP(c, scatter_partials(c, A));
+        SMG_HIP(c, launch_scatter(A, prec == SMG_PREC_FP64, c->stream));
+    }
     *rays += (uint64_t)g.n_det * (uint64_t)g.n_vox * (uint64_t)(A.n_pts > 0 ? A.n_pts : 0) * (uint64_t)ncell;
     return SMG_OK;
 }
@@ -1162,6 +1181,7 @@ smg_status smg_scatter_collimator_grid(smg_ctx* c, int rotation, double pitch_mm
     A.pe = nullptr;
     A.pair = c->pair.ptr;
     A.w1 = c->w1.ptr;
+    A.n_rows = g.n_det;
     float* out = dst;
     if (!dst_is_device) {
         SMG_HIP(c, c->out.reserve(n_el));

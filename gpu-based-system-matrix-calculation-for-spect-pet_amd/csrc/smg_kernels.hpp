@@ -156,8 +156,8 @@ struct ScatterLaunch {
     int variant;                     // collimator: 0 combined (r = 0.1), 1 standalone (r = 0.2)
     const float* pe;                 // crystal: PE block [N][V]
     const uint32_t* bitmap;          // crystal or collimator bitmap
-    PairRec* pair;                   // [N][n_pts][cells]
-    float* dst;                      // [N][V]
+    PairRec* pair;                   // [n_rows][n_pts][cells]
+    float* dst;                      // [n_rows][V]
     unsigned long long* counters;    // [0] FP64 fallback terms
     double cphi, sphi;
     int sub[3];                      // detection sub-cells
@@ -169,8 +169,8 @@ struct ScatterLaunch {
     const MuTablesF* tables_f;       // their FP32 form (when tables is set)
     const float* w1;                 // grid: first-leg weights [n_pts][V] of this chunk
     int accumulate;                  // add to dst instead of writing it
-    const int* rows;                 // detector rows to compute (dst row r = bar rows[r]),
-    int n_rows;                      // or nullptr for all bars
+    const int* rows;                 // detector rows to compute (dst row r = bar rows[r]), or
+    int n_rows, row0;                // nullptr for bars row0 .. row0 + n_rows - 1
     int pts_per_bar, pt_bar0;        // kind 3: point s lies in bar pt_bar0 + s / pts_per_bar
     double* partial;                 // [slices][rows][V] per-slice sums when the scatter points
                                      // are split over several waves per element

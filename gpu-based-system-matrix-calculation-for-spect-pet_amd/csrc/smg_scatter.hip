@@ -29,6 +29,9 @@ namespace smg {
 
 namespace {
 
+// The bar of output row r.
+__device__ __forceinline__ int row_bar(const ScatterLaunch& A, int r) { return A.rows ? A.rows[r] : A.row0 + r; }
+
 // The energy window of bar d's row.
 __device__ __forceinline__ void row_phys(const ScatterLaunch& A, const Bar<double>& bd, ScatterPhys& ph) {
     ph.e0 = A.e0;
@@ -47,10 +50,9 @@ __device__ __forceinline__ void row_phys(const ScatterLaunch& A, const Bar<doubl
 // per pair-term thread and per scatter wave (80-step FP64 bisections).
 __global__ __launch_bounds__(64) void row_cut_kernel(ScatterLaunch A, double* cut, WinRow* win) {
     const int r = (int)(blockIdx.x * 64 + threadIdx.x);
-    const int n_rows = A.rows ? A.n_rows : A.geom.g.n_det;
-    if (r >= n_rows) return;
+    if (r >= A.n_rows) return;
     ScatterPhys ph;
-    row_phys(A, A.geom.bars_d[A.rows ? A.rows[r] : r], ph);
+    row_phys(A, A.geom.bars_d[row_bar(A, r)], ph);
     cut[r] = window_reject_cos(ph, 0.0);
     if (A.win_n > 0) {
         win_domain(ph, cut[r], A.win_n);
@@ -61,11 +63,10 @@ __global__ __launch_bounds__(64) void row_cut_kernel(ScatterLaunch A, double* cu
 // One thread per interval of a row's window table.
 __global__ __launch_bounds__(256) void win_table_kernel(ScatterLaunch A, const WinRow* win, float* tab) {
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int n_rows = A.rows ? A.n_rows : A.geom.g.n_det;
-    if (tid >= (int64_t)n_rows * A.win_n) return;
+    if (tid >= (int64_t)A.n_rows * A.win_n) return;
     const int r = (int)(tid / A.win_n), i = (int)(tid % A.win_n);
     ScatterPhys ph;
-    row_phys(A, A.geom.bars_d[A.rows ? A.rows[r] : r], ph);
+    row_phys(A, A.geom.bars_d[row_bar(A, r)], ph);
     ph.win_x0 = win[r].x0;
     ph.win_scale = win[r].scale;
     float c[4];
@@ -121,7 +122,7 @@ __device__ __forceinline__ void pair_ids(const ScatterLaunch& A, int64_t tid, Pa
     const int cell = (int)(tid % ncell);
     P.s = (int)((tid / ncell) % A.n_pts);
     P.r = (int)(tid / ((int64_t)ncell * A.n_pts));
-    P.d = A.rows ? A.rows[P.r] : P.r;
+    P.d = row_bar(A, P.r);
     // the bar holding the scatter point (crystal scatter)
     P.sbar = A.kind == 3 ? A.pt_bar0 + P.s / A.pts_per_bar : P.s;
     const int a = cell % A.sub[0], b = (cell / A.sub[0]) % A.sub[1], c = cell / (A.sub[0] * A.sub[1]);
@@ -202,8 +203,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const PeGeom& G = A.geom;
     const int N = G.g.n_det;
-    const int n_rows = A.rows ? A.n_rows : N;
-    if (tid >= (int64_t)n_rows * A.n_pts * A.sub[0] * A.sub[1] * A.sub[2]) return;
+    if (tid >= (int64_t)A.n_rows * A.n_pts * A.sub[0] * A.sub[1] * A.sub[2]) return;
     PairIds P;
     pair_ids(A, tid, P);
     PairTerm out{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -273,8 +273,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pa
     const PeGeom& G = A.geom;
     const int N = G.g.n_det;
     const int lane = threadIdx.x;
-    const int n_rows = A.rows ? A.n_rows : N;
-    const int64_t total = (int64_t)n_rows * A.n_pts * A.sub[0] * A.sub[1] * A.sub[2];
+    const int64_t total = (int64_t)A.n_rows * A.n_pts * A.sub[0] * A.sub[1] * A.sub[2];
     const int64_t tid = (int64_t)blockIdx.x * 64 + lane;
     const bool valid = tid < total;
     PairIds P;
@@ -428,7 +427,7 @@ struct SliceShape {
 
 SliceShape slice_shape(const ScatterLaunch& A) {
     SliceShape s;
-    s.rows = A.rows ? A.n_rows : A.geom.g.n_det;
+    s.rows = A.n_rows;
     s.waves_per_det = (A.geom.g.n_vox + 63) / 64;
     const int64_t base = s.rows * s.waves_per_det;
     constexpr int64_t kFillWaves = 16384;     // 256 CUs x 4 SIMDs x 16
@@ -533,7 +532,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void sc
     const int64_t wrow = blockIdx.x % (sh.rows * waves_per_det);
     const int slice = (int)(blockIdx.x / (sh.rows * waves_per_det));
     const int r = (int)(wrow / waves_per_det);  // output row
-    const int d = A.rows ? A.rows[r] : r;
+    const int d = row_bar(A, r);
     const int64_t v = (wrow % waves_per_det) * 64 + lane;
     const bool valid = v < g.n_vox;
     const bool sliced = sh.slices > 1;
@@ -912,7 +911,7 @@ hipError_t launch_kn_table(double e0, double* tab, hipStream_t stream) {
 }
 
 hipError_t launch_row_cuts(const ScatterLaunch& A, double* cut, WinRow* win, float* tab, hipStream_t stream) {
-    const int64_t rows = A.rows ? A.n_rows : A.geom.g.n_det;
+    const int64_t rows = A.n_rows;
     if (rows <= 0) return hipSuccess;
     if (A.win_n > 0 && (!win || !tab)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(row_cut_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0, stream, A, cut, win);
@@ -923,7 +922,7 @@ hipError_t launch_row_cuts(const ScatterLaunch& A, double* cut, WinRow* win, flo
 }
 
 hipError_t launch_pair_terms(const ScatterLaunch& A, hipStream_t stream) {
-    const int64_t rows = A.rows ? A.n_rows : A.geom.g.n_det;
+    const int64_t rows = A.n_rows;
     const int64_t total = rows * A.n_pts * A.sub[0] * A.sub[1] * A.sub[2];
     if (total <= 0) return hipSuccess;
     if (A.kind == 2)
