@@ -263,8 +263,12 @@ __device__ __forceinline__ void append_candidates(Lists& L, int cap, int first, 
 // culling decision does not matter), each with the lanes whose reference
 // culling test keeps it: all of them where cull_keeps_all shows so for the
 // tile (99.97% of the candidates on the full-size geometry), else by a ballot
-// of the lanes' tests.  Returns false on overflow.
-template <bool kExact, class Lists>
+// of the lanes' tests.  kFew (the kernels for few sub-cells, where this scan is
+// most of the work): no cull_keeps_all in groups whose members all fail, of which a
+// panel turned by 0.25 rad scans several a tile (2.59 -> 2.45 ms at one sub-cell);
+// in the other kernels the branch costs 2% (full-size step 128.3 -> 130.5 ms).
+// Returns false on overflow.
+template <bool kExact, bool kFew, class Lists>
 __device__ bool build_candidates(const PeLaunch& A, int d, int lane, const WaveSetup& W,
                                  Lists& L, int& nb, int& nh) {
     const PeGeom& G = A.geom;
@@ -298,7 +302,7 @@ __device__ bool build_candidates(const PeLaunch& A, int d, int lane, const WaveS
                 pass = bar_tile_may_hit(bdf, W.tcf, rt, b.cx, b.cy, b.cz, b.cb, b.sb, 0.5f * b.w,
                                         0.5f * b.t, 0.5f * b.h);
                 const float c[3] = {b.cx, b.cy, b.cz};
-                all = cull_keeps_all(W.tcf, rho, c, 0.5f * b.rdiag, cd, 0.5f * bdf.rdiag);
+                all = (!kFew || pass) && cull_keeps_all(W.tcf, rho, c, 0.5f * b.rdiag, cd, 0.5f * bdf.rdiag);
             }
             append_candidates(L, L.cap_bars, 0, base, pass, all, valid, lane, nb, [&](int kk) {
                 return W.valid && cull_bar<kExact>(G, kk, W.p, W.pf, W.sc, W.udf, W.critf);
@@ -325,7 +329,7 @@ __device__ bool build_candidates(const PeLaunch& A, int d, int lane, const WaveS
                 pass = bar_tile_may_hit(bdf, W.tcf, W.te, o.xc, o.ymid, o.zc, 1.0f, 0.0f, o.r,
                                         0.5f * tabs(o.y2 - o.y1), o.r);
                 const float c[3] = {o.xc, o.ymid, o.zc};
-                all = cull_keeps_all(W.tcf, rho, c, o.crit, cd, 0.5f * bdf.rdiag);
+                all = (!kFew || pass) && cull_keeps_all(W.tcf, rho, c, o.crit, cd, 0.5f * bdf.rdiag);
             }
             append_candidates(L, L.cap_holes, nb, base, pass, all, valid, lane, nh, [&](int hh) {
                 return W.valid && cull_hole<kExact>(G, hh, W.p, W.pf, W.sc, W.udf, W.critf);
@@ -704,7 +708,7 @@ __device__ __forceinline__ double block_sum(const KahanSum<T>& acc, int wave, in
 // Work item `item` of the launch (a block index: bar, tile and, for point
 // weights, slice of cells) with candidate lists L.  Returns false, having
 // written nothing, when the candidates overflow L.
-template <bool kExact, bool kPoints, bool kEll, int kWaves = 1, class Lists>
+template <bool kExact, bool kPoints, bool kEll, int kWaves = 1, bool kFew = false, class Lists>
 __device__ __forceinline__ bool pe_forward_body(const PeLaunch& A, int item, Lists& L) {
     const PeGeom& G = A.geom;
     const GeomDesc& g = G.g;
@@ -737,7 +741,7 @@ __device__ __forceinline__ bool pe_forward_body(const PeLaunch& A, int item, Lis
         return true;
     }
     int nb, nh;
-    if (!build_candidates<kExact>(A, d, lane, W, L, nb, nh)) return false;
+    if (!build_candidates<kExact, kFew>(A, d, lane, W, L, nb, nh)) return false;
     L.sync();
 
     using T = typename std::conditional<kExact, double, float>::type;
@@ -809,11 +813,13 @@ __device__ __forceinline__ bool pe_forward_body(const PeLaunch& A, int item, Lis
 // within the LDS (10 KB of lists each).  The projections below likewise.
 // kEll: elliptical holes (the elliptic-cylinder chord compiled in; the
 // all-FP64 kernels always have it).
-template <bool kExact, bool kEll = kExact>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pe_forward_kernel(PeLaunch A) {
+// kFew (few_cells): 3 waves per SIMD, with few or no spills (36 B, else 176 B); so too
+// the projections.
+template <bool kExact, bool kEll = kExact, bool kFew = false>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kFew ? 3 : 4))) void pe_forward_kernel(PeLaunch A) {
     __shared__ WaveLists L;
     const int item = xcd_item((int)blockIdx.x, (int)gridDim.x);
-    if (!pe_forward_body<kExact, false, kEll>(A, item, L)) spill_push(A, item, threadIdx.x);
+    if (!pe_forward_body<kExact, false, kEll, 1, kFew>(A, item, L)) spill_push(A, item, threadIdx.x);
 }
 
 // kWaves waves per work item, each with its share of the sub-cells and lists of
@@ -897,7 +903,7 @@ __device__ __forceinline__ bool pe_tangent_body(const PeLaunch& A, const PeTange
         return true;
     }
     int nb, nh;
-    if (!build_candidates<kExact>(A, d, lane, W, L, nb, nh)) return false;
+    if (!build_candidates<kExact, false>(A, d, lane, W, L, nb, nh)) return false;
     L.sync();
     using T = typename std::conditional<kExact, double, float>::type;
     KahanSum<T> acc;
@@ -1091,7 +1097,7 @@ __device__ bool adjoint_cell(const PeGeom& G, int d, int lane, const WaveSetup& 
 // candidate lists L and per-candidate sums cand_acc.  Returns false when the
 // candidates overflow L (its scratch row is then incomplete; the spill kernel
 // rewrites all of it).
-template <bool kExact, class Lists>
+template <bool kExact, bool kFew = false, class Lists>
 __device__ __forceinline__ bool pe_backward_body(const PeLaunch& A, const PeGradScratch& S, int item,
                                                  Lists& L, double* cand_acc) {
     __shared__ double lay_acc[kMaxLayers];
@@ -1123,7 +1129,7 @@ __device__ __forceinline__ bool pe_backward_body(const PeLaunch& A, const PeGrad
             WaveSetup W;
             wave_setup(A, d, tile, lane, W);
             int nb, nh;
-            if (!build_candidates<kExact>(A, d, lane, W, L, nb, nh)) {
+            if (!build_candidates<kExact, kFew>(A, d, lane, W, L, nb, nh)) {
                 overflow = true;
                 break;
             }
@@ -1166,14 +1172,13 @@ __device__ __forceinline__ bool pe_backward_body(const PeLaunch& A, const PeGrad
     return true;
 }
 
-// 3 waves per SIMD (LDS and a 168-VGPR cap); uncapped the allocation lands
-// at 188 VGPRs, 2 waves.
-template <bool kExact>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void pe_backward_kernel(
+// 3 waves per SIMD (LDS and a 168-VGPR cap).  kFew (few_cells): 2, without spills.
+template <bool kExact, bool kFew = false>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kFew ? 2 : 3))) void pe_backward_kernel(
     PeLaunch A, PeGradScratch S) {
     __shared__ AdjointLists L;
     __shared__ double cand_acc[kCapBarsAdjoint];
-    if (!pe_backward_body<kExact>(A, S, (int)blockIdx.x, L, cand_acc)) spill_push(A, (int)blockIdx.x, threadIdx.x);
+    if (!pe_backward_body<kExact, kFew>(A, S, (int)blockIdx.x, L, cand_acc)) spill_push(A, (int)blockIdx.x, threadIdx.x);
 }
 
 // Queued work items of pe_backward_kernel redone with lists in global memory
@@ -1232,7 +1237,7 @@ __global__ __launch_bounds__(256) void pe_grad_reduce(PeGradScratch S, int n_det
 // A[d][v] of this lane for bar d and the wave's tile (W set up for them) into
 // a: 0 for a bar below the mu threshold.  Returns false (wave-uniform) when
 // the candidates overflow L; adds the lane's FP64 re-computations to fallbacks.
-template <bool kExact, bool kEll, class Lists>
+template <bool kExact, bool kEll, bool kFew, class Lists>
 __device__ bool pe_element(const PeLaunch& A, int d, int lane, const WaveSetup& W, Lists& L,
                            unsigned& fallbacks, double& a) {
     const PeGeom& G = A.geom;
@@ -1241,7 +1246,7 @@ __device__ bool pe_element(const PeLaunch& A, int d, int lane, const WaveSetup& 
     if (!(bd.mut > (double)0.01f)) return true;  // PESysMatGen.cu:1116, :1194
     int nb, nh;
     __syncthreads();  // the lists of the previous element are no longer read
-    if (!build_candidates<kExact>(A, d, lane, W, L, nb, nh)) return false;
+    if (!build_candidates<kExact, kFew>(A, d, lane, W, L, nb, nh)) return false;
     __syncthreads();
     using T = typename std::conditional<kExact, double, float>::type;
     KahanSum<T> acc;
@@ -1277,7 +1282,7 @@ __device__ __forceinline__ void add_fallbacks(const PeLaunch& A, int lane, unsig
 // Forward projection of work item `item` (bar d, voxel tile): the wave's share
 // of y[d] goes to partial[item].  Returns false, having written nothing, when
 // the candidates overflow L.
-template <bool kExact, bool kEll, class Lists>
+template <bool kExact, bool kEll, bool kFew = false, class Lists>
 __device__ __forceinline__ bool pe_project_body(const PeLaunch& A, const float* x, double* partial, int item,
                                                 Lists& L) {
     const int lane = threadIdx.x;
@@ -1288,24 +1293,24 @@ __device__ __forceinline__ bool pe_project_body(const PeLaunch& A, const float* 
     wave_setup(A, d, tile, lane, W);
     unsigned fallbacks = 0;
     double a;
-    if (!pe_element<kExact, kEll>(A, d, lane, W, L, fallbacks, a)) return false;
+    if (!pe_element<kExact, kEll, kFew>(A, d, lane, W, L, fallbacks, a)) return false;
     const double s = wave_sum(W.valid ? a * (double)x[W.v] : 0.0);
     if (lane == 0) partial[item] = s;
     if constexpr (!kExact) add_fallbacks(A, lane, fallbacks);
     return true;
 }
 
-template <bool kExact, bool kEll = kExact>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pe_project_kernel(PeLaunch A, const float* x, double* partial) {
+template <bool kExact, bool kEll = kExact, bool kFew = false>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kFew ? 3 : 4))) void pe_project_kernel(PeLaunch A, const float* x, double* partial) {
     __shared__ WaveLists L;
-    if (!pe_project_body<kExact, kEll>(A, x, partial, (int)blockIdx.x, L)) spill_push(A, (int)blockIdx.x, threadIdx.x);
+    if (!pe_project_body<kExact, kEll, kFew>(A, x, partial, (int)blockIdx.x, L)) spill_push(A, (int)blockIdx.x, threadIdx.x);
 }
 
 // Back-projection of work item `item` (group of `group` consecutive bars,
 // voxel tile), looping over the group's bars (those with y[d] = 0 skipped);
 // each lane's share of x[v] goes to partial[group][v].  Returns false, having
 // written nothing, when the candidates of one of the bars overflow L.
-template <bool kExact, bool kEll, class Lists>
+template <bool kExact, bool kEll, bool kFew = false, class Lists>
 __device__ __forceinline__ bool pe_backproject_body(const PeLaunch& A, const float* y, int group,
                                                     double* partial, int item, Lists& L) {
     const GeomDesc& g = A.geom.g;
@@ -1322,7 +1327,7 @@ __device__ __forceinline__ bool pe_backproject_body(const PeLaunch& A, const flo
         WaveSetup W;
         wave_setup(A, d, tile, lane, W);
         double a;
-        if (!pe_element<kExact, kEll>(A, d, lane, W, L, fallbacks, a)) return false;
+        if (!pe_element<kExact, kEll, kFew>(A, d, lane, W, L, fallbacks, a)) return false;
         acc += a * (double)yd;
     }
     // the lane's voxel (it does not depend on the bar)
@@ -1337,11 +1342,11 @@ __device__ __forceinline__ bool pe_backproject_body(const PeLaunch& A, const flo
     return true;
 }
 
-template <bool kExact, bool kEll = kExact>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pe_backproject_kernel(
+template <bool kExact, bool kEll = kExact, bool kFew = false>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kFew ? 3 : 4))) void pe_backproject_kernel(
     PeLaunch A, const float* y, int group, double* partial) {
     __shared__ WaveLists L;
-    if (!pe_backproject_body<kExact, kEll>(A, y, group, partial, (int)blockIdx.x, L)) spill_push(A, (int)blockIdx.x, threadIdx.x);
+    if (!pe_backproject_body<kExact, kEll, kFew>(A, y, group, partial, (int)blockIdx.x, L)) spill_push(A, (int)blockIdx.x, threadIdx.x);
 }
 
 // Queued work items of the projection kernels redone with lists in global
@@ -1407,6 +1412,21 @@ static bool wide_blocks(const PeLaunch& A) {
     return items <= 2048 && A.sub[0] * A.sub[1] * A.sub[2] >= 4 * kWideWaves;
 }
 
+// FP32 launches of few sub-cells over small tiles: setting a wave up (its lists, the
+// first block of sub-cells) is then most of its work, and registers spilled there
+// cost more than a wave more per SIMD gives.  2,048 bars, 8,192 voxels of 0.6 mm, one
+// sub-cell: matrix 2.11 -> 1.76 ms (1.97 with one sub-cell narrowed at a time), panel
+// turned by 0.25 rad 3.00 -> 2.45 (2.47; 4 sub-cells 4.57 -> 4.13), adjoint kernel of
+// 1,024 voxels 0.65 -> 0.51 (0.58).  At 8 sub-cells both are alike
+// (0.5 mm voxels, 1.78 and 1.77 ms), and with voxels of 2 mm (half diagonal of a tile
+// 5.2 mm), whose candidate lists are long, the rays count (4 sub-cells: 6.0 ms, 6.4
+// with few_cells's kernels).
+static bool few_cells(const PeLaunch& A) {
+    const GeomDesc& g = A.geom.g;
+    const double x = (A.tile[0] - 1) * g.wx, y = (A.tile[1] - 1) * g.wy, z = (A.tile[2] - 1) * g.wz;
+    return A.sub[0] * A.sub[1] * A.sub[2] <= 4 && x * x + y * y + z * z <= 100.0;
+}
+
 hipError_t launch_pe_tangent(const PeLaunch& A, const PeTangent& TG, bool exact, hipStream_t stream) {
     const int n_tiles = A.tiles[0] * A.tiles[1] * A.tiles[2];
     const int64_t blocks = (int64_t)n_tiles * A.geom.g.n_det;
@@ -1442,7 +1462,10 @@ hipError_t launch_pe_backward(const PeLaunch& A, const PeGradScratch& S, bool ex
         hipLaunchKernelGGL(pe_backward_kernel<true>, dim3((unsigned)blocks), dim3(64), 0, stream, A, S);
         if (sg) hipLaunchKernelGGL(pe_backward_spill_kernel<true>, dim3(sg), dim3(64), 0, stream, A, S);
     } else {
-        hipLaunchKernelGGL(pe_backward_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, stream, A, S);
+        if (few_cells(A))
+            hipLaunchKernelGGL((pe_backward_kernel<false, true>), dim3((unsigned)blocks), dim3(64), 0, stream, A, S);
+        else
+            hipLaunchKernelGGL(pe_backward_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, stream, A, S);
         if (sg) hipLaunchKernelGGL(pe_backward_spill_kernel<false>, dim3(sg), dim3(64), 0, stream, A, S);
     }
     e = hipGetLastError();
@@ -1496,7 +1519,7 @@ hipError_t launch_pe_forward_rows(const PeLaunch& A, bool exact, int bar0, int n
     unsigned sg = 0;
     hipError_t e = spill_begin(B, blocks, stream, sg);
     if (e != hipSuccess) return e;
-    const bool wide = wide_blocks(A);
+    const bool wide = wide_blocks(A), few = few_cells(A);
     const dim3 grid((unsigned)blocks), threads(64);
     if (exact) {
         if (wide)
@@ -1508,14 +1531,16 @@ hipError_t launch_pe_forward_rows(const PeLaunch& A, bool exact, int bar0, int n
         if (wide)
             launch_forward_wide(B, exact, blocks, stream);
         else
-            hipLaunchKernelGGL((pe_forward_kernel<false, true>), grid, threads, 0, stream, B);
+            hipLaunchKernelGGL((few ? pe_forward_kernel<false, true, true> : pe_forward_kernel<false, true>), grid,
+                               threads, 0, stream, B);
         if (sg)
             hipLaunchKernelGGL((pe_forward_spill_kernel<false, false, true>), dim3(sg), dim3(64), 0, stream, B);
     } else {
         if (wide)
             launch_forward_wide(B, exact, blocks, stream);
         else
-            hipLaunchKernelGGL(pe_forward_kernel<false>, grid, threads, 0, stream, B);
+            hipLaunchKernelGGL((few ? pe_forward_kernel<false, false, true> : pe_forward_kernel<false>), grid, threads, 0,
+                               stream, B);
         if (sg) hipLaunchKernelGGL((pe_forward_spill_kernel<false, false>), dim3(sg), dim3(64), 0, stream, B);
     }
     return hipGetLastError();
@@ -1570,18 +1595,20 @@ hipError_t launch_pe_project(const PeLaunch& A, bool exact, const float* x, doub
     unsigned sg = 0;
     hipError_t e = spill_begin(A, blocks, stream, sg);
     if (e != hipSuccess) return e;
+    const bool few = few_cells(A);
     if (exact) {
         hipLaunchKernelGGL(pe_project_kernel<true>, dim3((unsigned)blocks), dim3(64), 0, stream, A, x, partial);
         if (sg) hipLaunchKernelGGL((pe_project_spill_kernel<true, false>), dim3(sg), dim3(64), 0, stream, A, x, 0,
                            partial);
     } else if (A.ell) {
-        hipLaunchKernelGGL((pe_project_kernel<false, true>), dim3((unsigned)blocks), dim3(64), 0, stream, A, x,
-                           partial);
+        hipLaunchKernelGGL((few ? pe_project_kernel<false, true, true> : pe_project_kernel<false, true>),
+                           dim3((unsigned)blocks), dim3(64), 0, stream, A, x, partial);
         if (sg)
             hipLaunchKernelGGL((pe_project_spill_kernel<false, false, true>), dim3(sg), dim3(64), 0, stream, A, x,
                                0, partial);
     } else {
-        hipLaunchKernelGGL(pe_project_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, stream, A, x, partial);
+        hipLaunchKernelGGL((few ? pe_project_kernel<false, false, true> : pe_project_kernel<false>),
+                           dim3((unsigned)blocks), dim3(64), 0, stream, A, x, partial);
         if (sg) hipLaunchKernelGGL((pe_project_spill_kernel<false, false>), dim3(sg), dim3(64), 0, stream, A, x, 0,
                            partial);
     }
@@ -1604,20 +1631,21 @@ hipError_t launch_pe_backproject(const PeLaunch& A, bool exact, const float* y, 
     unsigned sg = 0;
     hipError_t e = spill_begin(A, blocks, stream, sg);
     if (e != hipSuccess) return e;
+    const bool few = few_cells(A);
     if (exact) {
         hipLaunchKernelGGL(pe_backproject_kernel<true>, dim3((unsigned)blocks), dim3(64), 0, stream, A, y, grp,
                            partial);
         if (sg) hipLaunchKernelGGL((pe_project_spill_kernel<true, true>), dim3(sg), dim3(64), 0, stream, A, y, grp,
                            partial);
     } else if (A.ell) {
-        hipLaunchKernelGGL((pe_backproject_kernel<false, true>), dim3((unsigned)blocks), dim3(64), 0, stream, A, y,
-                           grp, partial);
+        hipLaunchKernelGGL((few ? pe_backproject_kernel<false, true, true> : pe_backproject_kernel<false, true>),
+                           dim3((unsigned)blocks), dim3(64), 0, stream, A, y, grp, partial);
         if (sg)
             hipLaunchKernelGGL((pe_project_spill_kernel<false, true, true>), dim3(sg), dim3(64), 0, stream, A, y,
                                grp, partial);
     } else {
-        hipLaunchKernelGGL(pe_backproject_kernel<false>, dim3((unsigned)blocks), dim3(64), 0, stream, A, y, grp,
-                           partial);
+        hipLaunchKernelGGL((few ? pe_backproject_kernel<false, false, true> : pe_backproject_kernel<false>),
+                           dim3((unsigned)blocks), dim3(64), 0, stream, A, y, grp, partial);
         if (sg) hipLaunchKernelGGL((pe_project_spill_kernel<false, true>), dim3(sg), dim3(64), 0, stream, A, y, grp,
                            partial);
     }
