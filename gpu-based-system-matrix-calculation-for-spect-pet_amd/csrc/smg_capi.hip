@@ -353,14 +353,18 @@ hipError_t kn_table(smg_ctx* c, ScatterLaunch& A) {
 // Energy-window cut of each output row of a scatter launch (A.row_cut) and, for
 // FP32 launches, the rows' window tables (A.win_rows, A.win_tab) with as many
 // intervals as any of them needs, on the context's stream ahead of the pair terms
-// and scatter kernels.  rows_h: the launch's rows on the host, or all bars.
-hipError_t scatter_row_cuts(smg_ctx* c, ScatterLaunch& A, bool exact, const int* rows_h) {
+// and scatter kernels.  rows_h: the launch's rows on the host, or all bars.  n_pts:
+// the call's scatter points.  Calls of less than 2^16 terms have no tables, whose
+// launch and host work are 8-15 us (16 bars, 64 voxels: 102 us with them, 94 without;
+// what a million terms gain by them is about 1 us).
+hipError_t scatter_row_cuts(smg_ctx* c, ScatterLaunch& A, bool exact, const int* rows_h, int64_t n_pts) {
     const size_t rows = (size_t)A.n_rows;
     hipError_t e = c->sc_row_cut.reserve(rows > 0 ? rows : 1);
     if (e != hipSuccess) return e;
     A.row_cut = c->sc_row_cut.ptr;
     A.win_n = 0;
-    if (!exact && rows > 0) {
+    const double terms = (double)rows * (double)A.geom.g.n_vox * (double)n_pts * A.sub[0] * A.sub[1] * A.sub[2];
+    if (!exact && terms >= 65536.0) {
         // a row's table depends on its resolution only; bars without attenuation
         // have no terms (scatter.cu:1226-1228), so theirs does not matter
         double lo = INFINITY, hi = 0.0;
@@ -501,7 +505,7 @@ smg_status scatter_launch(smg_ctx* c, bool collimator, int rotation, int variant
     A.row0 = 0;
     A.pts_per_bar = 1;
     A.pt_bar0 = 0;
-    SMG_HIP(c, scatter_row_cuts(c, A, prec == SMG_PREC_FP64, nullptr));
+    SMG_HIP(c, scatter_row_cuts(c, A, prec == SMG_PREC_FP64, nullptr, A.n_pts));
     const ScatterLaunch all = A;
     for (int r0 = 0; r0 < g.n_det; r0 += chunk) {
         A.row0 = r0;
@@ -1214,7 +1218,7 @@ smg_status smg_scatter_collimator_grid(smg_ctx* c, int rotation, double pitch_mm
     if (pts.empty()) {
         SMG_HIP(c, hipMemsetAsync(out, 0, n_el * sizeof(float), c->stream));
     }
-    SMG_HIP(c, scatter_row_cuts(c, A, prec == SMG_PREC_FP64, nullptr));
+    SMG_HIP(c, scatter_row_cuts(c, A, prec == SMG_PREC_FP64, nullptr, (int64_t)pts.size()));
     for (int64_t s0 = 0; s0 < (int64_t)pts.size(); s0 += chunk) {
         A.pts_d = c->pts_grid.ptr + s0;
         A.n_pts = (int)std::min<int64_t>(chunk, (int64_t)pts.size() - s0);
@@ -1358,7 +1362,7 @@ smg_status smg_scatter_crystal_grid(smg_ctx* c, int rotation, int gx, int gy, in
             P.n_use_rows = nr;
         }
     }
-    SMG_HIP(c, scatter_row_cuts(c, A, prec == SMG_PREC_FP64, rows));
+    SMG_HIP(c, scatter_row_cuts(c, A, prec == SMG_PREC_FP64, rows, (int64_t)g.n_det * npb));
     std::vector<ScatterPt<double>> pts((size_t)nbc * npb);
     const int sub[3] = {gx, gy, gz};
     for (int b0 = 0; b0 < g.n_det; b0 += (int)nbc) {

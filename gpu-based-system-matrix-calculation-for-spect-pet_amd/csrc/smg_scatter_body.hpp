@@ -311,6 +311,7 @@ SMG_FN double window_reject_cos(const ScatterPhys& ph, double margin) {
     double g0 = 0.0, g1 = 1.0;  // e0 g (1 + r sqrt g) <= lo at g0, > lo at g1
     for (int it = 0; it < 80; ++it) {
         const double gm = 0.5 * (g0 + g1);
+        if (gm == g0 || gm == g1) break;  // neighbours: no step changes them any more
         if (ph.e0 * gm * (1.0 + r * sqrt(gm)) <= ph.lo) g0 = gm;
         else g1 = gm;
     }
@@ -498,6 +499,7 @@ SMG_FN double window_reject_omc_hi(const ScatterPhys& ph) {
     double g0 = 0.0, g1 = 1.0;  // below hi at g0, at or above it at g1
     for (int it = 0; it < 80; ++it) {
         const double gm = 0.5 * (g0 + g1);
+        if (gm == g0 || gm == g1) break;
         if (ph.e0 * gm * (1.0 - r * sqrt(gm)) >= ph.hi) g1 = gm;
         else g0 = gm;
     }
@@ -586,7 +588,7 @@ inline int win_intervals(const ScatterPhys& ph, double cut) {
 // Intervals of a launch with rows of resolutions res_lo to res_hi (ph: the window,
 // or with same = false each row's own, E0 (1 -+ res / 2)): the largest need, which
 // is not monotonic in the resolution (per-bar windows at 140.5 keV: 128 at 10% and
-// 77%, 256 at 30%), over steps of at most 1.25; 0 when one of them has no table.
+// 77%, 256 at 30%), over steps of at most 2; 0 when one of them has no table.
 inline int win_intervals_rows(ScatterPhys ph, bool same, double res_lo, double res_hi) {
     const auto need = [&](double res) {
         ph.res = res;
@@ -598,7 +600,7 @@ inline int win_intervals_rows(ScatterPhys ph, bool same, double res_lo, double r
     };
     int n = need(res_lo);
     if (n == 0 || !(res_hi > res_lo)) return n;
-    const int steps = (int)std::ceil(std::log(res_hi / res_lo) / std::log(1.25));
+    const int steps = (int)std::ceil(std::log(res_hi / res_lo) / std::log(2.0));
     for (int i = steps; i > 0; --i) {  // from the other end
         const int k = need(i == steps ? res_hi : res_lo * std::pow(res_hi / res_lo, (double)i / steps));
         if (k == 0) return 0;
