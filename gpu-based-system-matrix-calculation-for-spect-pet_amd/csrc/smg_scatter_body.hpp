@@ -311,7 +311,6 @@ SMG_FN double window_reject_cos(const ScatterPhys& ph, double margin) {
     double g0 = 0.0, g1 = 1.0;  // e0 g (1 + r sqrt g) <= lo at g0, > lo at g1
     for (int it = 0; it < 80; ++it) {
         const double gm = 0.5 * (g0 + g1);
-        if (gm == g0 || gm == g1) break;  // neighbours: no step changes them any more
         if (ph.e0 * gm * (1.0 + r * sqrt(gm)) <= ph.lo) g0 = gm;
         else g1 = gm;
     }
@@ -499,7 +498,6 @@ SMG_FN double window_reject_omc_hi(const ScatterPhys& ph) {
     double g0 = 0.0, g1 = 1.0;  // below hi at g0, at or above it at g1
     for (int it = 0; it < 80; ++it) {
         const double gm = 0.5 * (g0 + g1);
-        if (gm == g0 || gm == g1) break;
         if (ph.e0 * gm * (1.0 - r * sqrt(gm)) >= ph.hi) g1 = gm;
         else g0 = gm;
     }
