@@ -251,8 +251,8 @@ SMG_FN bool leg_may_hit(const float c[3], float diag, const float qs[3], const f
 
 // Bar-centre, hole-centre and crystal grid points: the bars flagged in the
 // bitmap between the scatter point and bar d count (scatter.cu:1343-1401).  A
-// wave takes 64 consecutive records, one per lane for the window test and the
-// own-bar part.  The bits of the records that any voxel can use are walked by the
+// wave takes `per` consecutive records (64, or fewer where they are too few to fill
+// the chip), one per lane for the window test and the own-bar part.  The bits of the records that any voxel can use are walked by the
 // whole wave: a record's words on the smallest power of two of lanes that covers
 // them (64 bars: 4 lanes, 16 records a pass; 2,048 bars: 64 lanes, 64 words a
 // pass).  The words become a list of bars, those the segment's line passes clear
@@ -268,14 +268,14 @@ struct PairWalk {
     uint32_t pair[128];  // (record << 26) | bar
     uint16_t bar[2048];  // bit within the 64 words
 };
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pair_terms_kernel(ScatterLaunch A) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void pair_terms_kernel(ScatterLaunch A, int per) {
     __shared__ PairWalk W;
     const PeGeom& G = A.geom;
     const int N = G.g.n_det;
     const int lane = threadIdx.x;
     const int64_t total = (int64_t)A.n_rows * A.n_pts * A.sub[0] * A.sub[1] * A.sub[2];
-    const int64_t tid = (int64_t)blockIdx.x * 64 + lane;
-    const bool valid = tid < total;
+    const int64_t tid = (int64_t)blockIdx.x * per + lane;
+    const bool valid = lane < per && tid < total;
     PairIds P;
     pair_ids(A, valid ? tid : total - 1, P);
     PairTerm out{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -925,10 +925,17 @@ hipError_t launch_pair_terms(const ScatterLaunch& A, hipStream_t stream) {
     const int64_t rows = A.n_rows;
     const int64_t total = rows * A.n_pts * A.sub[0] * A.sub[1] * A.sub[2];
     if (total <= 0) return hipSuccess;
-    if (A.kind == 2)
+    if (A.kind == 2) {
         hipLaunchKernelGGL(pair_terms_all_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, A);
-    else
-        hipLaunchKernelGGL(pair_terms_kernel, dim3((unsigned)((total + 63) / 64)), dim3(64), 0, stream, A);
+        return hipGetLastError();
+    }
+    // 2,048 waves (2 per SIMD) where the records allow it, of 8 records at least: a
+    // wave's passes over its records are one chain of latencies (160 bars, one hole, 3
+    // sub-cells, 480 records: 170 us at 64 a wave, call 300 us; 160 us at 8; 256 bars
+    // crystal, 65,536 records: 50 us at 64, 40 at 32)
+    int per = 64;
+    while (per > 8 && total <= (int64_t)(per / 2) * 2048) per /= 2;
+    hipLaunchKernelGGL(pair_terms_kernel, dim3((unsigned)((total + per - 1) / per)), dim3(64), 0, stream, A, per);
     return hipGetLastError();
 }
 
