@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "smg_kernels.hpp"
 #include "smg_pe_body.hpp"
@@ -1417,14 +1418,18 @@ static bool wide_blocks(const PeLaunch& A) {
 // cost more than a wave more per SIMD gives.  2,048 bars, 8,192 voxels of 0.6 mm, one
 // sub-cell: matrix 2.11 -> 1.76 ms (1.97 with one sub-cell narrowed at a time), panel
 // turned by 0.25 rad 3.00 -> 2.45 (2.47; 4 sub-cells 4.57 -> 4.13), adjoint kernel of
-// 1,024 voxels 0.65 -> 0.51 (0.58).  At 8 sub-cells both are alike
-// (0.5 mm voxels, 1.78 and 1.77 ms), and with voxels of 2 mm (half diagonal of a tile
-// 5.2 mm), whose candidate lists are long, the rays count (4 sub-cells: 6.0 ms, 6.4
-// with few_cells's kernels).
+// 1,024 voxels 0.65 -> 0.51 (0.58); 64 turned bars, 10,752 voxels of 0.3 mm, 6
+// sub-cells 156 -> 130 us (141).  With more sub-cells or wider tiles, whose candidate
+// lists are longer, the rays count: 2,048 bars, 8 sub-cells, half diagonal of a tile
+// 1.6 mm 2.35 and 2.33 ms, 2.6 mm 2.65 and 2.70; 4 sub-cells, 5.2 mm 6.0 and 6.4; one,
+// 10.4 mm 14.9 and 16.9.  The kernels with the elliptic chord spill more and gain up to
+// twice that (512 bars, 8 sub-cells, 2.6 mm 899 -> 821 us, 6.5 mm 1.50 ms both).
 static bool few_cells(const PeLaunch& A) {
     const GeomDesc& g = A.geom.g;
     const double x = (A.tile[0] - 1) * g.wx, y = (A.tile[1] - 1) * g.wy, z = (A.tile[2] - 1) * g.wz;
-    return A.sub[0] * A.sub[1] * A.sub[2] <= 4 && x * x + y * y + z * z <= 100.0;
+    const double rho = 0.5 * std::sqrt(x * x + y * y + z * z);
+    const int cells = A.sub[0] * A.sub[1] * A.sub[2];
+    return cells <= 8 && rho <= 5.0 && cells * rho <= (A.ell ? 40.0 : 20.0);
 }
 
 hipError_t launch_pe_tangent(const PeLaunch& A, const PeTangent& TG, bool exact, hipStream_t stream) {

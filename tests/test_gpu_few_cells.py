@@ -1,5 +1,5 @@
-"""The PE kernels for few sub-cells (at most 4, tiles of a half diagonal of at most 5
-mm) and their neighbours across that line, against the oracle: matrix, projections and
+"""The PE kernels for few sub-cells (at most 8, by the tiles' half diagonal) and their
+neighbours across that line, against the oracle: matrix, projections and
 gradient, turned bars and elliptical holes among them."""
 import numpy as np
 import pytest
@@ -9,9 +9,9 @@ from conftest import TOL_FP32, assert_parity, elliptic_hole_shapes, small_geomet
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("sub", [(1, 1, 1), (2, 1, 1), (1, 3, 1), (2, 1, 2), (5, 1, 1)])
+@pytest.mark.parametrize("sub", [(1, 1, 1), (2, 1, 1), (1, 3, 1), (2, 1, 2), (5, 1, 1), (2, 2, 2), (3, 1, 3)])
 @pytest.mark.parametrize("beta,ell", [(0.0, False), (0.3, False), (0.0, True)])
-@pytest.mark.parametrize("scale", [1.0, 2.0])  # tiles of 8 x 4 x 2 voxels: half diagonal 3.2 and 6.3 mm
+@pytest.mark.parametrize("scale", [0.5, 1.0, 2.0])  # tiles of 8 x 4 x 2 voxels: half diagonal 1.6, 3.2, 6.3 mm
 def test_few_cells(smg_mod, oracle_mod, params_mod, sub, beta, ell, scale):
     p = small_geometry(params_mod, beta=beta, n_rot=3, dphi=0.4)
     p.img[3:6] = [0.8 * scale, 0.9 * scale, 1.1 * scale]
