@@ -42,7 +42,7 @@ struct BmChunk {
     BmDir* dirs;                    // [origin][nk_pad]: every bar, or the chunk's holes
     BmRows* rows;                   // [block of origins][bar j]
     uint32_t* words;
-    int n, n_org, i0, ni, k0, nk, nk_pad, slice;
+    int n, i0, ni, k0, nk, nk_pad, slice;
 };
 
 template <bool kColl>
@@ -273,7 +273,6 @@ hipError_t launch_bitmap(const BitmapLaunch& A, bool collimator, hipStream_t str
     C.rows = (BmRows*)((unsigned char*)A.scratch + (size_t)p.n_dirs * sizeof(BmDir));
     C.words = A.words;
     C.n = n;
-    C.n_org = n_org;
     for (int k0 = 0; k0 < n; k0 += p.ck) {
         C.k0 = k0;
         C.nk = std::min(p.ck, n - k0);

@@ -14,7 +14,8 @@
 // formula in FP64, so every bit equals an FP64 evaluation of the reference test.
 //
 // The second half of the file is the same predicate bit by bit (bm_bit), with a
-// row's FP32 terms formed as the walk reaches it: the host's check of the bits.
+// row's FP32 terms formed as the walk reaches it: the kernel of small bitmaps, and the
+// host's check of the bits.
 #pragma once
 
 #include "smg_geometry.hpp"

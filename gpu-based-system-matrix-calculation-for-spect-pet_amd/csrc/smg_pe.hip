@@ -138,7 +138,6 @@ struct RecCands {
     __device__ int nbars() const { return nb; }
     __device__ bool fast(int j) const { return b[j].tag & kFastBar; }
     __device__ const float* faces(int j) const { return b[j].face; }
-    __device__ bool has_mu(int) const { return true; }
     __device__ double mu(int j) const { return b[j].mu; }
     __device__ int pos(int j) const { return b[j].tag & 0xffff; }
     // the index is wave-uniform: readfirstlane lets the record loads go
@@ -1268,8 +1267,10 @@ __device__ bool pe_element(const PeLaunch& A, int d, int lane, const WaveSetup& 
                 ++fallbacks;
             }
         });
-    // the element as the matrix kernel stores it (FP32), so that projecting
-    // equals multiplying by the stored matrix
+    // the element as the matrix kernel stores it (FP32), so that projecting equals
+    // multiplying by the stored matrix; wide blocks (wide_blocks) add their waves'
+    // compensated sums in FP64, which rounds to the same float unless the sum lies
+    // within its last bits of a tie (none of 1e7 sums tried)
     a = (double)float(acc.value());
     return true;
 }

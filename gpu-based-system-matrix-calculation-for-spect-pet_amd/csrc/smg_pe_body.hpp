@@ -757,11 +757,8 @@ SMG_FN float pe_cell_ray_f32(const PeGeom& G, int d, const double p[3], const do
     // rounding would not average out in sums over the matrix.  The reference
     // projects a turned bar's x and z faces with the world direction turned by
     // +beta, not by the -beta of the bar's frame.
-    double fx = D[0], fz = D[2];
-    if (!unturned) {
-        fx = D[0] * bd.cb - D[2] * bd.sb;
-        fz = D[0] * bd.sb + D[2] * bd.cb;
-    }
+    const double fx = unturned ? D[0] : D[0] * bd.cb - D[2] * bd.sb;
+    const double fz = unturned ? D[2] : D[0] * bd.sb + D[2] * bd.cb;
     float om;
     if constexpr (kPinned) {
         const float cb = float(bd.cb), sb = float(bd.sb);

@@ -67,7 +67,8 @@ typedef struct smg_stats {
     double total_ms;           /* host wall time of the call */
     uint64_t elements;         /* matrix elements produced */
     uint64_t rays;             /* element x sub-cell (x scatterer) terms */
-    uint64_t fp64_fallbacks;   /* FP32 terms recomputed in FP64 */
+    uint64_t fp64_fallbacks;   /* FP32 terms formed in FP64: decisions near a threshold, and PE
+                                  rays of sub-cells whose candidates do not fit LDS at once */
     uint64_t overflow_waves;   /* work items whose candidate lists overflowed LDS and were
                                   redone with lists in global memory (same result) */
 } smg_stats;
@@ -143,7 +144,8 @@ smg_status smg_pe_forward(smg_ctx* ctx, int rotation, smg_precision prec, float*
  * over the parameters of smg_pe_backward's gradient (dmu[0 .. Lc-1] layers,
  * dmu[Lc .. Lc+N-1] mu_total and dmu[Lc+N .. Lc+2N-1] mu_pe of each bar, host
  * memory): dA[d][v] = sum_k dmu[k] dA[d][v]/dmu_k, N x V floats, and the
- * matrix itself into A (optional, NULL to skip).  With smg_pe_backward it
+ * matrix itself into A (optional, NULL to skip; to FP32 rounding, since the
+ * tangent's FP32 rays round the solid angle on their own).  With smg_pe_backward it
  * gives Gauss-Newton products J^T (J v) at two passes per product, whatever
  * the number of parameters.  No counterpart in the reference. */
 smg_status smg_pe_tangent(smg_ctx* ctx, int rotation, smg_precision prec, const double* dmu, float* dA,
