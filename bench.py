@@ -38,8 +38,9 @@ METRIC = "matrix elements/s (PE, scatter) at ≤1e-5 rel err vs FP64; fwd+grad w
 PEAK_FP32_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
 # measured HBM traffic of one FP32 launch of the full-size PE step (rocprofv3 PMC
-# FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, factors from a plain 1 GiB copy)
-TRAFFIC_BYTES = 1.154e9
+# FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, factors from a plain 1 GiB copy); 1.07e9 of it is
+# the matrix, the rest scratch: registers spilled at a wave's set-up
+TRAFFIC_BYTES = 6.60e10
 # executed work of the same launch (rocprofv3 PMC, FP32 path): FLOPs per sub-cell ray
 # the lanes execute (64 x SQ_INSTS_VALU_FLOPS_FP32 + _FP64 per ray), VALU wave
 # instructions per ray x 64, transcendental instructions per ray x 64 (FP32 + FP64),
@@ -47,17 +48,17 @@ TRAFFIC_BYTES = 1.154e9
 # kernel's registers and LDS allow)
 EXEC_SOURCE = "profiles/pe_forward_instruction_mix_fp32_fp64_64x64x32_2048bars.md"
 EXEC_FLOPS_PER_RAY = 149.4 + 141.8
-VALU_INSTS_PER_RAY = 553.9
+VALU_INSTS_PER_RAY = 547.0
 TRANS_INSTS_PER_RAY = 12.2 + 4.9
-VALU_BUSY = 0.822
+VALU_BUSY = 0.818
 # the same instructions by issue cost (bin/valu_issue_probe on this GPU: 4 cycles
 # per wave instruction for FP32/FP64 arithmetic, integer and conversion, ~2 for
 # compares, selects, min/max and moves, ~8 for a transcendental)
-VALU_4CYCLE_INSTS_PER_RAY = 280.3
-VALU_2CYCLE_INSTS_PER_RAY = 273.6
+VALU_4CYCLE_INSTS_PER_RAY = 280.2
+VALU_2CYCLE_INSTS_PER_RAY = 266.9
 VALU_CYCLE_SOURCE = "profiles/valu_issue_rates_gfx950.md"
-LANE_UTILISATION = 0.816
-WAVES_PER_SIMD = 3.73
+LANE_UTILISATION = 0.814
+WAVES_PER_SIMD = 3.72
 MAX_WAVES_PER_SIMD = 4
 # unpacked FP32 (= FP64) vector FMA peak, the transcendental peak (a quarter of
 # the unpacked FMA rate in operations), and the VALU issue reference rate (256 CUs x
@@ -133,15 +134,15 @@ def ops_per_ray(p, sub):
     return o.pe_ops_per_ray(d, v, sub=sub)
 
 
-# executed work of scatter_kernel<false> per (row, voxel, scatter point, cell) term
+# executed work of scatter_kernel<false, true> per (row, voxel, scatter point, cell) term
 # (rocprofv3 PMC, FP32): FLOPs the lanes execute, VALU instructions x 64, lane
 # utilisation and VALUBusy
 SCATTER_EXEC_SOURCE = "profiles/scatter_kernels_4_workloads.md"
 SCATTER_EXEC = {
-    "crystal_scatter": {"flops_per_term": 89.3, "valu_insts_per_term": 110.9, "lane_utilisation": 0.754,
-                        "valu_busy": 0.68},
-    "collimator_grid": {"flops_per_term": 275.8, "valu_insts_per_term": 359.7, "lane_utilisation": 0.703,
-                        "valu_busy": 0.56},
+    "crystal_scatter": {"flops_per_term": 26.6, "valu_insts_per_term": 43.5, "lane_utilisation": 0.788,
+                        "valu_busy": 0.485},
+    "collimator_grid": {"flops_per_term": 111.0, "valu_insts_per_term": 178.9, "lane_utilisation": 0.801,
+                        "valu_busy": 0.401},
 }
 
 
