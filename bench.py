@@ -40,7 +40,7 @@ PEAK_HBM_GBS = 8000.0
 # measured HBM traffic of one FP32 launch of the full-size PE step (rocprofv3 PMC
 # FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0, factors from a plain 1 GiB copy); 1.07e9 of it is
 # the matrix, the rest scratch: registers spilled at a wave's set-up
-TRAFFIC_BYTES = 6.60e10
+TRAFFIC_BYTES = 6.69e10
 # executed work of the same launch (rocprofv3 PMC, FP32 path): FLOPs per sub-cell ray
 # the lanes execute (64 x SQ_INSTS_VALU_FLOPS_FP32 + _FP64 per ray), VALU wave
 # instructions per ray x 64, transcendental instructions per ray x 64 (FP32 + FP64),
@@ -48,17 +48,17 @@ TRAFFIC_BYTES = 6.60e10
 # kernel's registers and LDS allow)
 EXEC_SOURCE = "profiles/pe_forward_instruction_mix_fp32_fp64_64x64x32_2048bars.md"
 EXEC_FLOPS_PER_RAY = 149.4 + 141.8
-VALU_INSTS_PER_RAY = 547.0
+VALU_INSTS_PER_RAY = 533.6
 TRANS_INSTS_PER_RAY = 12.2 + 4.9
-VALU_BUSY = 0.818
+VALU_BUSY = 0.806
 # the same instructions by issue cost (bin/valu_issue_probe on this GPU: 4 cycles
 # per wave instruction for FP32/FP64 arithmetic, integer and conversion, ~2 for
 # compares, selects, min/max and moves, ~8 for a transcendental)
-VALU_4CYCLE_INSTS_PER_RAY = 280.2
-VALU_2CYCLE_INSTS_PER_RAY = 266.9
+VALU_4CYCLE_INSTS_PER_RAY = 285.9
+VALU_2CYCLE_INSTS_PER_RAY = 247.7
 VALU_CYCLE_SOURCE = "profiles/valu_issue_rates_gfx950.md"
-LANE_UTILISATION = 0.814
-WAVES_PER_SIMD = 3.72
+LANE_UTILISATION = 0.802
+WAVES_PER_SIMD = 3.73
 MAX_WAVES_PER_SIMD = 4
 # unpacked FP32 (= FP64) vector FMA peak, the transcendental peak (a quarter of
 # the unpacked FMA rate in operations), and the VALU issue reference rate (256 CUs x

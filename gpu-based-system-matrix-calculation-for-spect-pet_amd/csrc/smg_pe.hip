@@ -804,12 +804,12 @@ __device__ __forceinline__ bool pe_forward_body(const PeLaunch& A, int item, Lis
 }
 
 // 4 waves per SIMD: 128 VGPRs (the sub-cell context and the tile ball in
-// scalar registers) with 176 B of scratch a lane (spills of the set-up: 6.5e10 B of
+// scalar registers) with 180 B of scratch a lane (spills of the set-up: 6.6e10 B of
 // HBM traffic on the full-size step, 6% of its rate), and 16 one-wave blocks per CU
 // within the LDS (10 KB of lists each).  The projections below likewise.
 // kEll: elliptical holes (the elliptic-cylinder chord compiled in; the
 // all-FP64 kernels always have it).
-// kFew (few_cells): 3 waves per SIMD, with few or no spills (36 B, else 176 B); so too
+// kFew (few_cells): 3 waves per SIMD, with few or no spills (32 B, else 180 B); so too
 // the projections.
 template <bool kExact, bool kEll = kExact, bool kFew = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kFew ? 3 : 4))) void pe_forward_kernel(PeLaunch A) {
@@ -1421,6 +1421,8 @@ static bool wide_blocks(const PeLaunch& A) {
 // 1.6 mm 2.35 and 2.33 ms, 2.6 mm 2.65 and 2.70; 4 sub-cells, 5.2 mm 6.0 and 6.4; one,
 // 10.4 mm 14.9 and 16.9.  The kernels with the elliptic chord spill more and gain up to
 // twice that (512 bars, 8 sub-cells, 2.6 mm 899 -> 821 us, 6.5 mm 1.50 ms both).
+// (Both sides have since gained from frustum_cut and append_candidates alike: matrix
+// and turned panel 1.60 and 2.27 ms.)
 static bool few_cells(const PeLaunch& A) {
     const GeomDesc& g = A.geom.g;
     const double x = (A.tile[0] - 1) * g.wx, y = (A.tile[1] - 1) * g.wy, z = (A.tile[2] - 1) * g.wz;
